@@ -663,6 +663,190 @@ int build_segments(Accel &a, hipStream_t st, const std::vector<uint32_t> &off,
 
 }  // namespace
 
+// ------------------------------------------------------------ cell grid
+namespace {
+
+constexpr float kGridMaxCell = 4194304.0f;  // 2^22: cell centres and planes are exact floats
+
+// Cell of a voxel centre; false when the centre is not a cell's.
+__device__ __forceinline__ bool centre_cell(float c, int32_t &cell) {
+  const float x = c * 32.0f, f = floorf(x);  // exact: a power of two
+  cell = (int32_t)f;
+  return fabsf(x) < kGridMaxCell && f + 0.5f == x;
+}
+
+__global__ void k_grid_clear(uint4 *bricks, uint32_t n, uint32_t *work) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) bricks[i] = make_uint4(0u, 0u, 0u, 0u);
+  if (i < 2u) work[i] = 0u;
+}
+
+// Sets each voxel's bit.  work[0] collects why the scene cannot have a grid:
+// 1 a centre off the lattice or out of range, 2 two voxels in one cell.
+__global__ void __launch_bounds__(kBlock) k_grid_mark(SegView sv, const ct_aabb *aabbs, DGrid g, uint32_t *bricks,
+                                                      uint32_t *cells, uint32_t *work) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= sv.n) return;
+  const uint32_t s = find_seg(sv.off, sv.nseg, k), slot = sv.base[s] + (k - sv.off[s]);
+  const ct_aabb &b = aabbs[slot];
+  int32_t c[3];
+  bool ok = true;
+  uint32_t r[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    ok = centre_cell((b.minimum[a] + b.maximum[a]) * 0.5f, c[a]) && ok;
+    r[a] = (uint32_t)(c[a] - g.org[a]);
+    ok = ok && r[a] < 16u * g.nblk[a];
+  }
+  if (!ok) {
+    cells[slot] = kInvalid;
+    atomicOr(work, 1u);
+    return;
+  }
+  const uint32_t blk = ((r[2] >> 4) * g.nblk[1] + (r[1] >> 4)) * g.nblk[0] + (r[0] >> 4);
+  const uint32_t rec = (blk << 6) | ((r[0] >> 2) & 3u) | (r[1] & 12u) | ((r[2] & 12u) << 2);
+  const uint32_t bit = (r[0] & 3u) | ((r[1] & 3u) << 2) | ((r[2] & 3u) << 4);
+  cells[slot] = (rec << 6) | bit;
+  const uint32_t old = atomicOr(bricks + 4 * (size_t)rec + (bit >> 5), 1u << (bit & 31u));
+  if ((old >> (bit & 31u)) & 1u) atomicOr(work, 2u);
+}
+
+// One wave per block of 64 bricks: each brick's place in `ids` (the order of
+// bricks there is free, so a wave takes its range with one atomic) and its
+// empty cubes.  The occupancy of the bricks within kGridSkip - 1 of the
+// block is staged in LDS as rows of bits along x.
+constexpr int kSkipHalo = (int)kGridSkip - 1, kSkipRow = 4 + 2 * kSkipHalo;
+__global__ void __launch_bounds__(64) k_grid_link(DGrid g, uint4 *bricks, uint32_t *work) {
+  __shared__ uint32_t rows[kSkipRow * kSkipRow];
+  const uint32_t blk = blockIdx.x, l = threadIdx.x;
+  const uint32_t rec = (blk << 6) | l;
+  const uint4 e = bricks[rec];
+  const uint32_t n = (uint32_t)(__popc(e.x) + __popc(e.y));
+  uint32_t at = n;  // inclusive prefix over the wave
+  for (uint32_t o = 1; o < 64u; o <<= 1) {
+    const uint32_t v = __shfl_up(at, o);
+    if (l >= o) at += v;
+  }
+  uint32_t first = 0;
+  if (l == 63u && at) first = atomicAdd(work + 1, at);
+  first = __shfl(first, 63);
+  const int32_t x0 = (int32_t)(4u * (blk % g.nblk[0])), y0 = (int32_t)(4u * ((blk / g.nblk[0]) % g.nblk[1])),
+                z0 = (int32_t)(4u * (blk / (g.nblk[0] * g.nblk[1])));
+  for (uint32_t r = l; r < (uint32_t)(kSkipRow * kSkipRow); r += 64u) {
+    const uint32_t y = (uint32_t)(y0 - kSkipHalo + (int32_t)(r % kSkipRow)), z = (uint32_t)(z0 - kSkipHalo + (int32_t)(r / kSkipRow));
+    uint32_t row = 0;
+    if (y < 4u * g.nblk[1] && z < 4u * g.nblk[2])
+      for (int32_t i = 0; i < kSkipRow; ++i) {
+        const uint32_t x = (uint32_t)(x0 - kSkipHalo + i);
+        if (x >= 4u * g.nblk[0]) continue;
+        const uint32_t b = ((z >> 2) * g.nblk[1] + (y >> 2)) * g.nblk[0] + (x >> 2);
+        const uint2 m = *reinterpret_cast<const uint2 *>(bricks + ((b << 6) | (x & 3u) | ((y & 3u) << 2) | ((z & 3u) << 4)));
+        if (m.x | m.y) row |= 1u << i;
+      }
+    rows[r] = row;
+  }
+  __syncthreads();
+  uint32_t skip = 0;
+  if (n == 0u) {
+    const int32_t x = (int32_t)(l & 3u) + kSkipHalo, y = (int32_t)((l >> 2) & 3u) + kSkipHalo, z = (int32_t)(l >> 4) + kSkipHalo;
+    for (uint32_t o = 0; o < 8u; ++o) {
+      const int32_t dy = (o & 2u) ? -1 : 1, dz = (o & 4u) ? -1 : 1;
+      uint32_t side = 1, seen = 0;  // `seen`: the occupied columns of the rows within side x side
+      for (uint32_t s = 2; s <= kGridSkip; ++s) {
+        // the rows that a side of s adds to one of s - 1
+        for (uint32_t k = 0; k < s; ++k)
+          seen |= rows[(z + dz * (int32_t)(s - 1)) * kSkipRow + (y + dy * (int32_t)k)] |
+                  rows[(z + dz * (int32_t)k) * kSkipRow + (y + dy * (int32_t)(s - 1))];
+        if (s == 2u) seen |= rows[z * kSkipRow + y];
+        const uint32_t cols = ((1u << s) - 1u) << ((o & 1u) ? x - (int32_t)(s - 1) : x);
+        if (seen & cols) break;
+        side = s;
+      }
+      skip |= side << (4u * o);
+    }
+  }
+  reinterpret_cast<uint2 *>(bricks + rec)[1] = make_uint2(first + at - n, skip);
+}
+
+__global__ void __launch_bounds__(kBlock) k_grid_ids(SegView sv, const uint32_t *inst, const uint4 *bricks,
+                                                     const uint32_t *cells, uint2 *ids) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= sv.n) return;
+  const uint32_t s = find_seg(sv.off, sv.nseg, k), p = k - sv.off[s], c = cells[sv.base[s] + p];
+  if (c == kInvalid) return;
+  const uint4 e = bricks[c >> 6];
+  const unsigned long long m = ((unsigned long long)e.y << 32) | e.x;
+  const uint32_t i = e.z + (uint32_t)__popcll(m & ((1ull << (c & 63u)) - 1ull));
+  if (i < sv.n) ids[i] = make_uint2(inst[s], p);
+}
+
+// Builds the scene's cell grid (DGrid) when it can have one: every instance
+// has the same transform, every voxel is a cell of the 2^-5 lattice, no cell
+// holds two voxels, and the bricks of the bounding box are few against the
+// voxels (16 B a brick against about 130 B a voxel for the BVH).  Enqueued
+// on `st`, which reads `seg` and writes `flags`: once it has drained, the
+// caller drops the grid if `flags` is not zero.
+int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::vector<uint32_t> &seg, uint32_t &flags) {
+  BvhSet &S = a.set;
+  S.grid = DGrid{};
+  flags = 0;
+  if (ids.empty()) return CT_OK;
+  const float *w = &a.w2o[16 * ids[0]];
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  seg.assign(3 * ids.size() + 1, 0u);  // offsets, first slots, instance ids
+  const size_t nseg = ids.size();
+  for (size_t q = 0; q < nseg; ++q) {
+    const uint32_t id = ids[q];
+    if (std::memcmp(w, &a.w2o[16 * id], 16 * sizeof(float)) != 0) return CT_OK;
+    for (int c = 0; c < 3; ++c) {
+      lo[c] = std::fmin(lo[c], a.blas_root_box[6 * id + c]);
+      hi[c] = std::fmax(hi[c], a.blas_root_box[6 * id + 3 + c]);
+    }
+    seg[q + 1] = seg[q] + a.instances[id].primitive_count;
+    seg[nseg + 1 + q] = a.instances[id].first_primitive_index;
+    seg[2 * nseg + 1 + q] = id;
+  }
+  const uint32_t n = seg[nseg];
+  DGrid g{};
+  uint64_t nblk = 1;
+  for (int c = 0; c < 3; ++c) {
+    if (!(std::fabs(lo[c]) < kGridMaxCell / 64.0f) || !(std::fabs(hi[c]) < kGridMaxCell / 64.0f)) return CT_OK;
+    // an empty brick at least around the boxes
+    const int32_t l = (int32_t)std::floor(lo[c] * 32.0f) - 5, h = (int32_t)std::floor(hi[c] * 32.0f) + 5;
+    g.org[c] = l & ~15;
+    g.nblk[c] = (uint32_t)((h | 15) + 1 - g.org[c]) / 16u;
+    nblk *= g.nblk[c];
+    if (g.nblk[c] > 1024u || nblk > (1u << 19)) return CT_OK;
+  }
+  const uint32_t nrec = (uint32_t)(64 * nblk);
+  if ((uint64_t)nrec > 4ull * n + (1u << 20)) return CT_OK;
+  for (int c = 0; c < 4; ++c)
+    for (int r = 0; r < 3; ++r) g.w2o[c * 3 + r] = w[c * 4 + r];
+  int rc;
+  if ((rc = S.grid_bricks.reserve(16 * (size_t)nrec)) || (rc = S.grid_ids.reserve(8 * (size_t)n)) ||
+      (rc = S.grid_cells.reserve(4 * (size_t)S.prim_capacity)) || (rc = S.grid_work.reserve(8 + 4 * seg.size())))
+    return rc;
+  uint32_t *work = S.grid_work.as<uint32_t>(), *d_seg = work + 2;
+  CT_HIP(hipMemcpyAsync(d_seg, seg.data(), 4 * seg.size(), hipMemcpyHostToDevice, st));
+  const SegView sv{d_seg, d_seg + nseg + 1, nullptr, (uint32_t)nseg, n};
+  uint4 *bricks = S.grid_bricks.as<uint4>();
+  hipLaunchKernelGGL(k_grid_clear, dim3(blocks(nrec)), dim3(kBlock), 0, st, bricks, nrec, work);
+  hipLaunchKernelGGL(k_grid_mark, dim3(blocks(n)), dim3(kBlock), 0, st, sv, S.aabbs.as<ct_aabb>(), g,
+                     S.grid_bricks.as<uint32_t>(), S.grid_cells.as<uint32_t>(), work);
+  hipLaunchKernelGGL(k_grid_link, dim3((uint32_t)nblk), dim3(64), 0, st, g, bricks, work);
+  hipLaunchKernelGGL(k_grid_ids, dim3(blocks(n)), dim3(kBlock), 0, st, sv, d_seg + 2 * nseg + 1, bricks,
+                     S.grid_cells.as<uint32_t>(), S.grid_ids.as<uint2>());
+  CT_HIP(hipGetLastError());
+  CT_HIP(hipMemcpyAsync(&flags, work, 4, hipMemcpyDeviceToHost, st));
+  g.bricks = bricks;
+  g.ids = S.grid_ids.as<uint2>();
+  g.cells = S.grid_cells.as<uint32_t>();
+  S.grid = g;
+  return CT_OK;
+}
+
+}  // namespace
+
 DScene scene_view(const Accel &a) {
   DScene s;
   s.blas_nodes = a.set.nodes.as<DNode>();
@@ -672,6 +856,7 @@ DScene scene_view(const Accel &a) {
   s.tlas_inst = a.set.tlas_inst.as<uint32_t>();
   s.tlas_root = a.set.tlas_root;
   s.n_inst = (uint32_t)a.instances.size();
+  s.grid = a.set.grid;
   return s;
 }
 
@@ -685,6 +870,7 @@ DScene previous_scene_view(const Accel &a) {
   s.tlas_inst = a.prev.tlas_inst.as<uint32_t>();
   s.tlas_root = a.prev.tlas_root;
   s.n_inst = a.prev.n_inst;
+  s.grid = DGrid{};  // the previous set is walked as a BVH
   return s;
 }
 
@@ -932,6 +1118,7 @@ int commit(Accel &a, const Dirty &d) {
   a.blas_depth.resize(a.instances.size(), 0);
   const uint32_t cap = std::max<uint32_t>(a.prim_high_water, 1);
   const bool full = d.full || S.prim_capacity != cap || !S.nodes.p;
+  S.grid = DGrid{};  // until this commit's own is built
   if (full) {
     S.prim_capacity = cap;
     if ((rc = S.aabbs.reserve(sizeof(ct_aabb) * (size_t)cap)) || (rc = S.prims.reserve(sizeof(ct_primitive) * (size_t)cap)) ||
@@ -1011,7 +1198,14 @@ int commit(Accel &a, const Dirty &d) {
     if ((rc = refit_blas_set(a, st, d.refit))) return rc;
   }
   if ((rc = upload_tables(a, st))) return rc;
-  return build_tlas(a, st);
+  uint32_t grid_flags = 0;
+  std::vector<uint32_t> grid_seg;
+  rc = build_grid(a, st, used_ids(a), grid_seg, grid_flags);
+  if (!rc) rc = build_tlas(a, st);
+  const hipError_t e = hipStreamSynchronize(st);  // grid_seg was read, grid_flags has arrived
+  if (rc || e != hipSuccess || grid_flags) S.grid = DGrid{};
+  if (!rc && e != hipSuccess) return fail(CT_E_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
+  return rc;
 }
 
 int device_count_gfx950() {

@@ -67,13 +67,14 @@ CT_D void view_ray(const AView &V, uint32_t x, uint32_t y, uint32_t &seed, F3 &o
 
 // Closest voxel of the segment from `origin` along `dir` (intersect()):
 // returns the slot and the world hit position and normal.
+template <int kWalk>
 CT_D bool segment(const AArgs &A, F3 origin, F3 dir, uint32_t *stk, uint32_t &g, F3 &pos, F3 &nrm) {
   const F3 ro = compute_ray_origin(origin, dir);
   float bt = kFar;
   uint32_t bi = kInvalid, bp = kInvalid;
   bool ovf = false;
   TraceCnt cnt;
-  traverse_mode<kTraceBounce, false>(A.S, ro, dir, kFar, kInvalid, kInvalid, bt, bi, bp, stk, kBlockA, cnt, ovf);
+  traverse_mode<kTraceBounce, kWalk>(A.S, ro, dir, kFar, kInvalid, kInvalid, bt, bi, bp, stk, kBlockA, cnt, ovf);
   if (bi == kInvalid) return false;
   const DInst &I = A.S.inst[bi];
   float w[12];
@@ -102,6 +103,7 @@ CT_D F3 albedo_of(const AArgs &A, uint32_t g) {
 
 // Traces one sample; fills the vertices (when `path` is given) and returns
 // the sample's radiance.
+template <int kWalk>
 CT_D F3 trace_sample(const AArgs &A, const AView &V, uint32_t x, uint32_t y, uint32_t seed, uint32_t *stk,
                      Vertex *path, uint32_t &nv) {
   F3 o, d;
@@ -111,7 +113,7 @@ CT_D F3 trace_sample(const AArgs &A, const AView &V, uint32_t x, uint32_t y, uin
   for (uint32_t k = 0; k <= A.max_depth; ++k) {
     uint32_t g;
     F3 pos, nrm;
-    if (!segment(A, o, d, stk, g, pos, nrm)) break;
+    if (!segment<kWalk>(A, o, d, stk, g, pos, nrm)) break;
     if (path) {
       path[k].g = g;
       path[k].beta = beta;
@@ -130,8 +132,9 @@ CT_D F3 trace_sample(const AArgs &A, const AView &V, uint32_t x, uint32_t y, uin
 
 CT_D uint32_t sample_seed(uint32_t gpix, uint32_t seed, uint32_t s) { return tea(tea(gpix, seed), s); }
 
+template <int kWalk>
 __global__ void __launch_bounds__(kBlockA) k_adj_forward(AArgs A, float *image) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlockA];
+  __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
   const uint2 b = A.blocks[blockIdx.x];
   const AView &V = A.views[b.x];
   const uint32_t p = b.y + threadIdx.x;
@@ -140,16 +143,17 @@ __global__ void __launch_bounds__(kBlockA) k_adj_forward(AArgs A, float *image) 
   F3 sum = f3(0, 0, 0);
   uint32_t nv;
   for (uint32_t s = 0; s < A.spp; ++s)
-    sum = add(sum, trace_sample(A, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x, nullptr, nv));
+    sum = add(sum, trace_sample<kWalk>(A, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x, nullptr, nv));
   const F3 I = divs(sum, (float)A.spp);
   image[3 * (size_t)gpix] = I.x;
   image[3 * (size_t)gpix + 1] = I.y;
   image[3 * (size_t)gpix + 2] = I.z;
 }
 
+template <int kWalk>
 __global__ void __launch_bounds__(kBlockA) k_adj_backward(AArgs A, const float *grad_image, float *grad_albedo,
                                                           float *grad_emission) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlockA];
+  __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
   const uint2 b = A.blocks[blockIdx.x];
   const AView &V = A.views[b.x];
   const uint32_t p = b.y + threadIdx.x;
@@ -161,7 +165,7 @@ __global__ void __launch_bounds__(kBlockA) k_adj_backward(AArgs A, const float *
   Vertex path[CT_ADJOINT_MAX_DEPTH + 1];
   for (uint32_t s = 0; s < A.spp; ++s) {
     uint32_t nv;
-    trace_sample(A, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x, path, nv);
+    trace_sample<kWalk>(A, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x, path, nv);
     F3 S = f3(0, 0, 0);  // radiance from the vertices after k, relative to vertex k+1
     for (int k = (int)nv - 1; k >= 0; --k) {
       const uint32_t g = path[k].g;
@@ -281,6 +285,7 @@ CT_D bool scatter_material(const PMat &m, F3 dir, F3 nrm, uint32_t &seed, F3 &sd
   return true;
 }
 
+template <int kWalk>
 CT_D F3 path_sample(const PArgs &P, const AView &V, uint32_t x, uint32_t y, uint32_t seed, uint32_t *stk) {
   const AArgs &A = P.A;
   F3 o, d;
@@ -289,7 +294,7 @@ CT_D F3 path_sample(const PArgs &P, const AView &V, uint32_t x, uint32_t y, uint
   for (uint32_t k = 0; k <= A.max_depth; ++k) {
     uint32_t g;
     F3 pos, nrm;
-    if (!segment(A, o, d, stk, g, pos, nrm)) break;
+    if (!segment<kWalk>(A, o, d, stk, g, pos, nrm)) break;
     const uint32_t mi = P.prims[g].material_index;
     if (mi >= P.n_mats) break;  // no material: absorbs
     const PMat m = P.mats[mi];
@@ -306,8 +311,9 @@ CT_D F3 path_sample(const PArgs &P, const AView &V, uint32_t x, uint32_t y, uint
   return L;
 }
 
+template <int kWalk>
 __global__ void __launch_bounds__(kBlockA) k_path_trace(PArgs P, float *image) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlockA];
+  __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
   const AArgs &A = P.A;
   const uint2 b = A.blocks[blockIdx.x];
   const AView &V = A.views[b.x];
@@ -315,7 +321,7 @@ __global__ void __launch_bounds__(kBlockA) k_path_trace(PArgs P, float *image) {
   if (p >= V.width * V.height) return;
   const uint32_t x = p % V.width, y = p / V.width, gpix = V.base + p;
   F3 sum = f3(0, 0, 0);
-  for (uint32_t s = 0; s < A.spp; ++s) sum = add(sum, path_sample(P, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x));
+  for (uint32_t s = 0; s < A.spp; ++s) sum = add(sum, path_sample<kWalk>(P, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x));
   const F3 I = divs(sum, (float)A.spp);
   image[3 * (size_t)gpix] = I.x;
   image[3 * (size_t)gpix + 1] = I.y;
@@ -377,7 +383,10 @@ int ct_adjoint_render(ct_accel *a, const ct_adjoint_desc *d, const ct_adjoint_vi
   if ((rc = plan(*a, d, views, st, P, A))) return rc;
   A.albedo = albedo;
   A.emission = emission;
-  hipLaunchKernelGGL(k_adj_forward, dim3(P.nblocks), dim3(kBlockA), 0, st, A, image);
+  if (A.S.grid.bricks)
+    hipLaunchKernelGGL(k_adj_forward<kWalkGrid>, dim3(P.nblocks), dim3(kBlockA), 0, st, A, image);
+  else
+    hipLaunchKernelGGL(k_adj_forward<kWalkBvh>, dim3(P.nblocks), dim3(kBlockA), 0, st, A, image);
   CT_HIP(hipGetLastError());
   CT_HIP(hipStreamSynchronize(st));  // the plan's buffers are released on return
   return CT_OK;
@@ -415,7 +424,10 @@ int ct_path_trace(ct_accel *a, const ct_adjoint_desc *d, const ct_adjoint_view *
   PA.n_mats = a->pt_mat_count;
   PA.A.albedo = nullptr;
   PA.A.emission = nullptr;
-  hipLaunchKernelGGL(k_path_trace, dim3(P.nblocks), dim3(kBlockA), 0, st, PA, image);
+  if (PA.A.S.grid.bricks)
+    hipLaunchKernelGGL(k_path_trace<kWalkGrid>, dim3(P.nblocks), dim3(kBlockA), 0, st, PA, image);
+  else
+    hipLaunchKernelGGL(k_path_trace<kWalkBvh>, dim3(P.nblocks), dim3(kBlockA), 0, st, PA, image);
   CT_HIP(hipGetLastError());
   CT_HIP(hipStreamSynchronize(st));  // the plan's buffers are released on return
   return CT_OK;
@@ -434,8 +446,12 @@ int ct_adjoint_backward(ct_accel *a, const ct_adjoint_desc *d, const ct_adjoint_
   if ((rc = plan(*a, d, views, st, P, A))) return rc;
   A.albedo = albedo;
   A.emission = emission;
-  hipLaunchKernelGGL(k_adj_backward, dim3(P.nblocks), dim3(kBlockA), 0, st, A, grad_image, grad_albedo,
-                     grad_emission);
+  if (A.S.grid.bricks)
+    hipLaunchKernelGGL(k_adj_backward<kWalkGrid>, dim3(P.nblocks), dim3(kBlockA), 0, st, A, grad_image, grad_albedo,
+                       grad_emission);
+  else
+    hipLaunchKernelGGL(k_adj_backward<kWalkBvh>, dim3(P.nblocks), dim3(kBlockA), 0, st, A, grad_image, grad_albedo,
+                       grad_emission);
   CT_HIP(hipGetLastError());
   CT_HIP(hipStreamSynchronize(st));
   return CT_OK;

@@ -293,12 +293,17 @@ struct Stack {
 // global load instead of a flat one, which would also count against the
 // LDS wait counter that the traversal stack uses.
 typedef float gf4 __attribute__((ext_vector_type(4)));
+typedef uint32_t gu2 __attribute__((ext_vector_type(2)));
 typedef uint32_t gu4 __attribute__((ext_vector_type(4)));
 CT_D float gld(const float *p) { return *(const __attribute__((address_space(1))) float *)p; }
 CT_D uint32_t gld(const uint32_t *p) { return *(const __attribute__((address_space(1))) uint32_t *)p; }
 CT_D float4 gld(const float4 *p) {
   const gf4 v = *(const __attribute__((address_space(1))) gf4 *)p;
   return make_float4(v.x, v.y, v.z, v.w);
+}
+CT_D uint2 gld(const uint2 *p) {
+  const gu2 v = *(const __attribute__((address_space(1))) gu2 *)p;
+  return make_uint2(v.x, v.y);
 }
 CT_D uint4 gld(const uint4 *p) {
   const gu4 v = *(const __attribute__((address_space(1))) gu4 *)p;
@@ -481,32 +486,336 @@ struct Walker {
   }
 };
 
+// ------------------------------------------------------------ cell grid
+// The walk of one ray through the scene's cell grid (DGrid) instead of its
+// BVH: the same voxel tests on the same operands, so the same hits to the
+// bit, in far fewer instructions and bytes.  A BVH walk of the noise scenes
+// visits about 30 nodes of 64 B per ray; here a ray takes about 10 steps,
+// each over an empty box (a cube of up to kGridSkip bricks, 2x2x2 cells of a
+// brick, or a cell), and reads 16 B per brick it stops in.
+//
+// Which voxels can a test accept?  intersect_box() accepts a voxel when the
+// ray's computed crossing of the plane of one of its faces lies within the
+// face, so up to rounding the ray enters the voxel's cell there (or starts
+// in it).  The walk enters every cell the ray enters, except in boxes that
+// hold no voxel, and tests it.  Where a crossing lies within p of a cell's
+// edge, the cells across that edge are tested too.  p bounds the rounding of
+// both sides, in cells, with u = 2^-24, T the ray parameter scaled to 1/2..1
+// cells on the fastest axis and iv the crossing times of a cell:
+//   walk:  (plane - q) * iv, then q + v T:         3 u T + u |q + v T|
+//   test:  ro - c, +-r, * inv, o + dr t:     6 u T + u max(iv) / 2 + 2 u
+// hence p = 10 u T + u (1.5 max|position| + max(iv) + 4).  Past 1/64 cell it
+// is cut off: there the BVH's own boxes (padded by 2^-12, 1/128 cell) do not
+// bound the test's rounding either.
+//
+// An empty box may be stepped over when neither its entry nor its exit lies
+// within p iv_a of a lattice plane of an axis other than the crossed one, a.
+// Take a voxel outside the box whose plane b the ray crosses inside it,
+// within p of a face c of the box: positions along the ray only grow, so at
+// the exit (or entry) the ray is within p of face c; if c is the crossed
+// axis, at most p iv_c of the ray lies between, and there the ray is within
+// p iv_c of plane b.  Otherwise the ray takes the cell alone, which has no
+// inner planes, with its neighbours.
+//
+// Coordinates are lattice cells (32 per unit), exact in float, negated on
+// the axes the ray runs down (cell i becomes ~i), so every axis runs up.
+constexpr float kCellsPerUnit = 32.0f;
+constexpr float kU = 5.9604644775390625e-8f;  // 2^-24
+constexpr float kNearMax = 0.015625f;
+constexpr float kDeadAxis = 9.094947017729282e-13f;  // 2^-40: an axis that is never crossed
+
+CT_D float med3f(float a, float b, float c) { return gmax(gmin(a, b), gmin(gmax(a, b), c)); }
+CT_D int32_t imin(int32_t a, int32_t b) { return a < b ? a : b; }
+CT_D int32_t imax(int32_t a, int32_t b) { return a > b ? a : b; }
+CT_D int32_t clampi(int32_t x, int32_t lo, int32_t hi) { return imax(imin(x, lo), imin(imax(x, lo), hi)); }
+
+template <int kMode>
+struct GridWalk {
+  static constexpr bool kAny = kMode == kTraceAny;
+  const DGrid &G;
+  F3 oo, dr, sg, sinv;           // object-space ray as the voxel test takes it
+  int32_t sx, sy, sz;            // -1 on negated axes
+  uint32_t target;               // any hit: the target voxel's cell (DGrid::cells)
+  float limit, best_t;
+  uint32_t best;                 // index in ids of the closest voxel
+  bool occluded;
+
+  // The brick record of a (negated) cell and its index (times 64); false
+  // outside the grid.
+  CT_D bool brick(int32_t ix, int32_t iy, int32_t iz, uint4 &e, uint32_t &base) const {
+    const uint32_t x = (uint32_t)((ix ^ sx) - G.org[0]), y = (uint32_t)((iy ^ sy) - G.org[1]),
+                   z = (uint32_t)((iz ^ sz) - G.org[2]);
+    const uint32_t bx = x >> 4, by = y >> 4, bz = z >> 4;
+    if (bx >= G.nblk[0] || by >= G.nblk[1] || bz >= G.nblk[2]) return false;
+    const uint32_t b = (bz * G.nblk[1] + by) * G.nblk[0] + bx;
+    const uint32_t r = (b << 6) | ((x >> 2) & 3u) | (y & 12u) | ((z & 12u) << 2);
+    e = gld(G.bricks + r);
+    base = r << 6;
+    return true;
+  }
+  // The bit of a (negated) cell in its brick (the grid starts at a multiple
+  // of 16 cells).
+  CT_D uint32_t bit_of(int32_t ix, int32_t iy, int32_t iz) const {
+    return ((uint32_t)(ix ^ sx) & 3u) | (((uint32_t)(iy ^ sy) & 3u) << 2) | (((uint32_t)(iz ^ sz) & 3u) << 4);
+  }
+
+  // The voxel test on an occupied cell.
+  CT_D void test(int32_t ix, int32_t iy, int32_t iz, const uint4 &e, uint32_t base, uint32_t bit) {
+    const int32_t cx = ix ^ sx, cy = iy ^ sy, cz = iz ^ sz;
+    const F3 c = f3(((float)cx + 0.5f) * 0.03125f, ((float)cy + 0.5f) * 0.03125f, ((float)cz + 0.5f) * 0.03125f);
+    float t;
+    if (kAny) {
+      const bool hit = intersect_box<false, false>(c, oo, dr, sg, sinv, t);
+      if (hit && (t >= 0.0f) && (t <= limit) && (base | bit) != target) occluded = true;
+    } else {
+      const bool hit = kMode == kTraceClosest ? intersect_box<true, true>(c, oo, dr, sg, sinv, t)
+                                              : intersect_box<true, false>(c, oo, dr, sg, sinv, t);
+      if (hit && (kMode == kTraceClosest ? t > 0.0f : t >= 0.0f) && t <= best_t) {
+        const uint64_t mask = ((uint64_t)e.y << 32) | e.x;
+        const uint32_t idx = e.z + (uint32_t)__popcll(mask & ((1ull << bit) - 1ull));
+        bool better = t < best_t || best == kInvalid;
+        if (!better) {  // equal t: the smaller (instance, primitive)
+          const uint2 a = gld(G.ids + idx), b = gld(G.ids + best);
+          better = a.x < b.x || (a.x == b.x && a.y < b.y);
+        }
+        if (better) {
+          best_t = t;
+          best = idx;
+        }
+      }
+    }
+  }
+
+  // The state of a walk between its steps; `done` once it has ended.
+  int32_t ix, iy, iz;            // the cell
+  float px, py, pz, p;           // the position the ray entered it at, and p there
+  bool near, done;
+  float vx, vy, vz, qx, qy, qz, ivx, ivy, ivz, t_unit, t_end, k1;
+  uint32_t octant;               // shift of the ray's nibble
+
+  // Whether a position is within `m` of a lattice plane on an axis other
+  // than the crossed one (always near its own plane); `any`: on any axis.
+  CT_D static bool near_plane(float x, float y, float z, float m, bool any) {
+    const float fx = fabsf((x - floorf(x)) - 0.5f), fy = fabsf((y - floorf(y)) - 0.5f), fz = fabsf((z - floorf(z)) - 0.5f);
+    return (any ? gmax(gmax(fx, fy), fz) : med3f(fx, fy, fz)) > 0.5f - m;
+  }
+
+  // Tests the cells across the edges within p of the position the ray
+  // entered the cell at.
+  CT_D void test_near() {
+    const float fx = px - (float)ix, fy = py - (float)iy, fz = pz - (float)iz;
+    const int32_t ax = fx < p ? -1 : (fx > 1.0f - p ? 1 : 0), ay = fy < p ? -1 : (fy > 1.0f - p ? 1 : 0),
+                  az = fz < p ? -1 : (fz > 1.0f - p ? 1 : 0);
+    // bit k: the cell offset on the axes of k's bits
+    uint32_t ks = 0xFEu & (ax ? 0xFFu : 0x55u) & (ay ? 0xFFu : 0x33u) & (az ? 0xFFu : 0x0Fu);
+    while (ks) {
+      const uint32_t k = (uint32_t)__ffs((int)ks) - 1u;
+      ks &= ks - 1u;
+      const int32_t x = (k & 1u) ? ix + ax : ix, y = (k & 2u) ? iy + ay : iy, z = (k & 4u) ? iz + az : iz;
+      uint4 e;
+      uint32_t base;
+      if (!brick(x, y, z, e, base)) continue;
+      const uint32_t bit = bit_of(x, y, z);
+      if (((((bit & 32u) ? e.y : e.x) >> (bit & 31u)) & 1u) != 0u) test(x, y, z, e, base, bit);
+    }
+  }
+
+  // Where the ray leaves the box of cells from its cell to (ex, ey, ez).
+  CT_D float leave(int32_t ex, int32_t ey, int32_t ez, float &tx, float &ty, float &tz, float &x, float &y, float &z,
+                   float &pn) const {
+    tx = ((float)(ex + 1) - qx) * ivx;
+    ty = ((float)(ey + 1) - qy) * ivy;
+    tz = ((float)(ez + 1) - qz) * ivz;
+    const float t = gmin(gmin(tx, ty), tz);
+    x = __builtin_fmaf(vx, t, qx);
+    y = __builtin_fmaf(vy, t, qy);
+    z = __builtin_fmaf(vz, t, qz);
+    pn = gmin(__builtin_fmaf(10.0f * kU, t, k1), kNearMax);
+    return t;
+  }
+
+  // Sets the walk up; `done` at once when the ray misses the grid.
+  CT_D void start(const DScene &S, F3 o, F3 d, uint32_t ti, uint32_t tp) {
+    done = true;
+    float m[12];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) m[k] = G.w2o[k];
+    oo = xform3(m, o, 1.0f);
+    const F3 od = xform3(m, d, 0.0f);
+    target = kInvalid;
+    if (kAny && ti < S.n_inst) {
+      const DInst *I = S.inst + ti;
+      if (tp < gld(&I->count)) target = gld(G.cells + gld(&I->first) + tp);
+    }
+    const F3 inv = f3(safe_inverse(od.x), safe_inverse(od.y), safe_inverse(od.z));
+    sinv = inv;
+    dr = kMode == kTraceClosest ? mul_rot(od) : od;
+    sg = f3(-gsign(dr.x), -gsign(dr.y), -gsign(dr.z));
+    const float qmax = gmax(gmax(fabsf(oo.x), fabsf(oo.y)), fabsf(oo.z)) * kCellsPerUnit;
+    const float dmax = gmax(gmax(fabsf(od.x), fabsf(od.y)), fabsf(od.z));
+    // A direction of zero length or with a term that is not finite, or an
+    // origin whose cells are not distinct floats, hits nothing.
+    if (!(dmax > 0.0f) || !((fabsf(od.x) + fabsf(od.y)) + fabsf(od.z) < INFINITY) ||
+        !((fabsf(oo.x) + fabsf(oo.y)) + fabsf(oo.z) < 1e9f))
+      return;
+    int ex;
+    (void)frexpf(dmax, &ex);
+    sx = od.x < 0.0f ? -1 : 0;
+    sy = od.y < 0.0f ? -1 : 0;
+    sz = od.z < 0.0f ? -1 : 0;
+    octant = ((uint32_t)sx & 4u) | ((uint32_t)sy & 8u) | ((uint32_t)sz & 16u);
+    vx = ldexpf(fabsf(od.x), -ex);
+    vy = ldexpf(fabsf(od.y), -ex);
+    vz = ldexpf(fabsf(od.z), -ex);
+    qx = (sx ? -oo.x : oo.x) * kCellsPerUnit;
+    qy = (sy ? -oo.y : oo.y) * kCellsPerUnit;
+    qz = (sz ? -oo.z : oo.z) * kCellsPerUnit;
+    const bool lx = vx > kDeadAxis, ly = vy > kDeadAxis, lz = vz > kDeadAxis;
+    ivx = lx ? ldexpf(fabsf(inv.x), ex) : 1e30f;
+    ivy = ly ? ldexpf(fabsf(inv.y), ex) : 1e30f;
+    ivz = lz ? ldexpf(fabsf(inv.z), ex) : 1e30f;
+    // the grid's first and last cells in negated coordinates
+    const int32_t dx = (int32_t)(16u * G.nblk[0]), dy = (int32_t)(16u * G.nblk[1]), dz = (int32_t)(16u * G.nblk[2]);
+    const int32_t l0x = sx ? -(G.org[0] + dx) : G.org[0], l0y = sy ? -(G.org[1] + dy) : G.org[1],
+                  l0z = sz ? -(G.org[2] + dz) : G.org[2];
+    const int32_t hx = l0x + dx - 1, hy = l0y + dy - 1, hz = l0z + dz - 1;
+    const float tn = gmax(gmax(((float)l0x - qx) * ivx, ((float)l0y - qy) * ivy), ((float)l0z - qz) * ivz);
+    const float tf = gmin(gmin(((float)(hx + 1) - qx) * ivx, ((float)(hy + 1) - qy) * ivy), ((float)(hz + 1) - qz) * ivz);
+    t_unit = ldexpf(1.0f, ex + 5);  // T of one unit of t
+    t_end = (kAny ? limit : best_t) * t_unit;
+    const float t = gmax(tn, 0.0f);
+    if (!(t <= tf) || t > t_end + kNearMax) return;
+    done = false;
+    const float gm = gmax(gmax(gmax(fabsf((float)l0x), fabsf((float)hx)), gmax(fabsf((float)l0y), fabsf((float)hy))),
+                          gmax(fabsf((float)l0z), fabsf((float)hz)));
+    k1 = kU * (1.5f * gmax(qmax, gm) + gmax(gmax(lx ? ivx : 0.0f, ly ? ivy : 0.0f), lz ? ivz : 0.0f) + 4.0f);
+    px = __builtin_fmaf(vx, t, qx);
+    py = __builtin_fmaf(vy, t, qy);
+    pz = __builtin_fmaf(vz, t, qz);
+    ix = clampi((int32_t)floorf(px), l0x, hx);
+    iy = clampi((int32_t)floorf(py), l0y, hy);
+    iz = clampi((int32_t)floorf(pz), l0z, hz);
+    p = gmin(__builtin_fmaf(10.0f * kU, t, k1), kNearMax);
+    near = near_plane(px, py, pz, p, true);  // an origin in the grid has crossed no axis
+  }
+
+  // Lanes step until each has come to a voxel or ended (a cell's neighbours,
+  // rare, are tested on the spot); the voxel tests then run together, and
+  // nearly all accept.
+  CT_D void run(const DScene &S, F3 o, F3 d, uint32_t ti, uint32_t tp) {
+    constexpr uint32_t kStepping = 0, kAtVoxel = 1, kEnded = 2;
+    start(S, o, d, ti, tp);
+    if (done) return;
+    uint4 e = make_uint4(0u, 0u, 0u, 0u);
+    uint32_t base = 0, bit = 0, tested = kInvalid;  // the cell tested last
+    int32_t moved = ~0;  // bits of the cell that the last step changed
+    for (;;) {
+      uint32_t state = kStepping;
+      while (state == kStepping) {
+        if ((moved & ~3) != 0 && !brick(ix, iy, iz, e, base)) {
+          state = kEnded;
+          break;
+        }
+        if (near) {
+          test_near();
+          if (!kAny) t_end = best_t * t_unit;
+          if (kAny && occluded) {
+            state = kEnded;
+            break;
+          }
+        }
+        // the cell, the 2x2x2 cells around it when all are empty, or the
+        // empty cube of bricks
+        int32_t m = 3, ext = (int32_t)((e.w >> octant) & 15u) * 4 - 4;
+        if ((e.x | e.y) != 0u) {
+          bit = bit_of(ix, iy, iz);
+          const uint32_t w = (uint32_t)((((uint64_t)e.y << 32) | e.x) >> (bit & 0x2Au));
+          if (((w >> (bit & 0x15u)) & 1u) != 0u && (base | bit) != tested) {
+            state = kAtVoxel;
+            break;
+          }
+          m = (w & 0x00330033u) == 0u ? 1 : 0;
+          ext = 0;
+        }
+        if (near) m = ext = 0;
+        int32_t fx = (ix | m) + ext, fy = (iy | m) + ext, fz = (iz | m) + ext;
+        float tx, ty, tz, x, y, z, pn;
+        float t = leave(fx, fy, fz, tx, ty, tz, x, y, z, pn);
+        bool nr = near_plane(x, y, z, pn * (tx <= t ? ivx : (ty <= t ? ivy : ivz)), false);
+        if (nr && m != 0) {
+          fx = ix;
+          fy = iy;
+          fz = iz;
+          t = leave(fx, fy, fz, tx, ty, tz, x, y, z, pn);
+          nr = near_plane(x, y, z, pn * (tx <= t ? ivx : (ty <= t ? ivy : ivz)), false);
+        }
+        if (t > t_end + pn) {
+          state = kEnded;
+          break;
+        }
+        const int32_t nx = tx <= t ? fx + 1 : clampi((int32_t)floorf(x), ix, fx),
+                      ny = ty <= t ? fy + 1 : clampi((int32_t)floorf(y), iy, fy),
+                      nz = tz <= t ? fz + 1 : clampi((int32_t)floorf(z), iz, fz);
+        moved = (ix ^ nx) | (iy ^ ny) | (iz ^ nz);
+        ix = nx;
+        iy = ny;
+        iz = nz;
+        px = x;
+        py = y;
+        pz = z;
+        p = pn;
+        near = nr;
+      }
+      if (state == kEnded) return;
+      test(ix, iy, iz, e, base, bit);
+      if (kAny && occluded) return;
+      if (!kAny) t_end = best_t * t_unit;
+      tested = base | bit;
+      near = false;  // its neighbours are done too
+      moved = 0;
+    }
+  }
+};
+
+// How a kernel is built to walk: the BVH, the BVH with counters, or the cell
+// grid (scenes that have one; the counters are the BVH's, so counted
+// launches walk it).
+constexpr int kWalkBvh = 0, kWalkCount = 1, kWalkGrid = 2;
+
 // The whole walk of one ray.  Returns true when an any-hit query is
 // occluded; a closest query leaves its hit in best_t/best_i/best_p (which
 // enter as the current limit and an invalid hit).
-template <int kMode, bool kCount>
+template <int kMode, int kWalk>
 CT_D bool traverse_mode(const DScene &S, F3 o, F3 d, float limit, uint32_t ti, uint32_t tp,
                         float &best_t, uint32_t &best_i, uint32_t &best_p, uint32_t *stk,
                         uint32_t stride, TraceCnt &cnt, bool &overflow) {
-  Walker<kMode, kCount> w;
-  w.start(S, o, d, limit, ti, tp, stk, stride);
-  w.best_t = best_t;
-  w.best_i = best_i;
-  w.best_p = best_p;
-  while (!w.done) w.step(S, cnt);
-  best_t = w.best_t;
-  best_i = w.best_i;
-  best_p = w.best_p;
-  overflow = overflow || w.overflow;
-  return w.occluded && !w.overflow;
-}
-
-template <bool kAny, bool kCount>
-CT_D bool traverse(const DScene &S, F3 o, F3 d, float limit, uint32_t ti, uint32_t tp,
-                   float &best_t, uint32_t &best_i, uint32_t &best_p, uint32_t *stk,
-                   uint32_t stride, TraceCnt &cnt, bool &overflow) {
-  return traverse_mode<kAny ? kTraceAny : kTraceClosest, kCount>(S, o, d, limit, ti, tp, best_t, best_i, best_p, stk,
-                                                                  stride, cnt, overflow);
+  if constexpr (kWalk == kWalkGrid) {
+    GridWalk<kMode> w{S.grid};
+    w.limit = limit;
+    w.best_t = best_t;
+    w.best = kInvalid;
+    w.occluded = false;
+    w.run(S, o, d, ti, tp);
+    if (kMode != kTraceAny && w.best != kInvalid) {
+      const uint2 id = gld(S.grid.ids + w.best);
+      best_t = w.best_t;
+      best_i = id.x;
+      best_p = id.y;
+    }
+    return w.occluded;
+  } else {
+    Walker<kMode, kWalk == kWalkCount> w;
+    w.start(S, o, d, limit, ti, tp, stk, stride);
+    w.best_t = best_t;
+    w.best_i = best_i;
+    w.best_p = best_p;
+    while (!w.done) w.step(S, cnt);
+    best_t = w.best_t;
+    best_i = w.best_i;
+    best_p = w.best_p;
+    overflow = overflow || w.overflow;
+    return w.occluded && !w.overflow;
+  }
 }
 
 }  // namespace dev

@@ -67,6 +67,25 @@ struct alignas(16) DInst {
   uint32_t pad;
 };
 
+// Cell grid of a scene whose voxels all sit on the 2^-5 lattice of one object
+// space (host side: build_grid).  Cells are grouped in bricks of 4x4x4 and
+// blocks of 4x4x4 bricks; the bricks of a block are contiguous, 64 records
+// of 16 B: the 64-bit occupancy mask (bit x + 4y + 16z), the index in `ids`
+// of the brick's first voxel (voxels in bit order), and 8 nibbles, one for
+// each octant of directions (nibble o: down the x, y, z axis where bit 0, 1,
+// 2 of o is set): the side, in bricks, of the largest empty cube that starts
+// at the brick and extends into the octant (up to kGridSkip; 0: the brick
+// itself is not empty).  Everything outside the grid is empty.
+constexpr uint32_t kGridSkip = 4;
+struct DGrid {
+  const uint4 *bricks;   // null: the scene has no grid and is walked as a BVH
+  const uint2 *ids;      // (instance, primitive)
+  const uint32_t *cells; // by primitive slot: brick record << 6 | bit
+  int32_t org[3];        // lattice cell of the grid's first cell, a multiple of 16
+  uint32_t nblk[3];      // blocks per axis
+  float w2o[12];         // world-to-object, shared by every instance (DInst::w2o)
+};
+
 struct DScene {
   const DNode *blas_nodes;
   const float4 *blas_leaves;  // (centre.xyz, prim id bits), Morton order
@@ -75,6 +94,7 @@ struct DScene {
   const uint32_t *tlas_inst;  // instance id per TLAS leaf
   uint32_t tlas_root;
   uint32_t n_inst;            // entries of `inst` (instance slots)
+  DGrid grid;
 };
 
 // Raw device buffer with RAII.
@@ -159,6 +179,8 @@ struct BvhSet {
   uint32_t prim_capacity = 0;
   uint32_t cube_light_count = 0;
   uint32_t cube_light_hw = 0;   // entries held: deleted lights leave stale records past the count
+  DevBuf grid_bricks, grid_ids, grid_cells, grid_work;
+  DGrid grid{};                 // bricks null: no grid
 };
 
 // The scene as the frames before an update saw it: the traversable state

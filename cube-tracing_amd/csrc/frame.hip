@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <type_traits>
 
 #include "ct_device.h"
 #include "ct_internal.h"
@@ -934,10 +935,14 @@ CT_D void queue_flush(const DFrame &F, uint32_t px, uint32_t emitted, uint32_t f
 }
 
 // ---------------------------------------------------------------- kernels
+// LDS words of a block's traversal stacks: the grid walk has none.
+template <int kWalk>
+constexpr uint32_t kStackWords = kWalk == kWalkGrid ? 1u : (uint32_t)((kStackLds > 0 ? kStackLds : 1) * kBlock);
+
 // Primary rays: raygen rgen.glsl:18-42 + closest hit; one 8x8 tile per wave.
-template <bool kCount>
+template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_primary(FrameSet FS, unsigned long long *stats) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint2 blk_ = FS.blk[blockIdx.x];
   const DFrame &F = FS.fb[blk_.x];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
@@ -952,10 +957,11 @@ __global__ void __launch_bounds__(kBlock) k_primary(FrameSet FS, unsigned long l
     float bt = kMaxDistance;
     uint32_t bi = kInvalid, bp = kInvalid;
     bool ovf = false;
-    traverse<false, kCount>(F.S, o, d, kMaxDistance, kInvalid, kInvalid, bt, bi, bp, stk + tid, kBlock, cnt, ovf);
+    traverse_mode<kTraceClosest, kWalk>(F.S, o, d, kMaxDistance, kInvalid, kInvalid, bt, bi, bp, stk + tid, kBlock,
+                                        cnt, ovf);
     F.hit[y * F.W + x] = make_float4(bi != kInvalid ? bt : -1.0f, __uint_as_float(bi), __uint_as_float(bp), 0.0f);
   }
-  if (kCount) {
+  if (kWalk == kWalkCount) {
     unsigned long long a = cnt.nodes, b = cnt.leaves, c = cnt.insts;
     for (int off = 32; off > 0; off >>= 1) {
       a += __shfl_down(a, off);
@@ -1009,6 +1015,7 @@ CT_D bool pass_pixel(const DFrame &F, uint2 blk, uint32_t &px) {
 // (PRIMITIVE.light_index); any other candidate has weight 0 and light -1.
 // All are CUBE candidates.  Returns whether the merge into `r` selected the
 // strategy's reservoir: then the reservoir skips the visibility pass.
+template <int kWalk>
 CT_D bool ris_brdf(const DFrame &F, Res &r, F3 ray_o, Hit &hit, const Mat &mat, const RisCounts &rc, uint32_t &seed,
                    uint32_t *stk, uint32_t &rays) {
   Res br = res_init();
@@ -1028,7 +1035,7 @@ CT_D bool ris_brdf(const DFrame &F, Res &r, F3 ray_o, Hit &hit, const Mat &mat, 
     uint32_t bi = kInvalid, bp = kInvalid;
     bool ovf = false;
     TraceCnt cnt;
-    traverse_mode<kTraceBounce, false>(F.S, ro, wi, kMaxDistance, kInvalid, kInvalid, bt, bi, bp, stk, kBlock, cnt,
+    traverse_mode<kTraceBounce, kWalk>(F.S, ro, wi, kMaxDistance, kInvalid, kInvalid, bt, bi, bp, stk, kBlock, cnt,
                                        ovf);
     ++rays;
     if (bi != kInvalid) {
@@ -1064,9 +1071,9 @@ constexpr uint32_t kNoVisibilityPass = 0x80000000u;
 // (rmiss.glsl:19-29), motion vector, temporal gather, confidence and RIS.
 // EMIT for the RIS visibility ray.  kBrdf: some frame of the set has the
 // RIS BRDF strategy on (its rays need an LDS stack).
-template <bool kBrdf>
+template <bool kBrdf, int kWalk>
 CT_D void ris_pass(const FrameSet &FS) {
-  __shared__ uint32_t stk[kBrdf ? (kStackLds > 0 ? kStackLds : 1) * kBlock : 1];
+  __shared__ uint32_t stk[kBrdf ? kStackWords<kWalk> : 1];
   const uint2 blk_ = FS.blk[blockIdx.x];
   const DFrame &F = FS.fb[blk_.x];
   uint32_t px;
@@ -1143,7 +1150,7 @@ CT_D void ris_pass(const FrameSet &FS) {
       Res r = ris(F, confidence, rd, hit, mat, di.seed, rc);
       bool needs_visibility = true;
       if (kBrdf && (F.active & CT_RIS_BRDF_BIT) &&
-          ris_brdf(F, r, ro, hit, mat, rc, di.seed, stk + threadIdx.x, brdf_rays))
+          ris_brdf<kWalk>(F, r, ro, hit, mat, rc, di.seed, stk + threadIdx.x, brdf_rays))
         needs_visibility = false;
       Vis v{true, px, 0u, 0u, 0u, 0u};
       Res rv = r;
@@ -1180,11 +1187,12 @@ CT_D void ris_pass(const FrameSet &FS) {
 #define CT_RIS_BRDF_WAVES 4
 #endif
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(5))) k_ris(FrameSet FS) {
-  ris_pass<false>(FS);
+  ris_pass<false, kWalkBvh>(FS);
 }
+template <int kWalk>
 __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(CT_RIS_BRDF_WAVES)))
 k_ris_brdf(FrameSet FS) {
-  ris_pass<true>(FS);
+  ris_pass<true, kWalk>(FS);
 }
 
 // RIS visibility (slot 0) and temporal reuse (slots 1, 2) with the results
@@ -1361,9 +1369,9 @@ struct RayBatches {
 
 // Closest voxel of each queued path segment (intersect() semantics), one
 // 64-ray fetch per wave.  kMulti: segments of several frames (scenes).
-template <bool kCount, bool kMulti>
+template <int kWalk, bool kMulti>
 __global__ void __launch_bounds__(kBlock) k_trace_segments(FrameSet FS, uint32_t d, unsigned long long *stats) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const DFrame &F0 = FS.fb[0];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t n = F0.counters[kCntPtQueue + (d & 1u)];
@@ -1376,12 +1384,12 @@ __global__ void __launch_bounds__(kBlock) k_trace_segments(FrameSet FS, uint32_t
       float bt = kMaxDistance;
       uint32_t bi = kInvalid, bp = kInvalid;
       bool ovf = false;
-      traverse_mode<kTraceBounce, kCount>(FS.fb[view].S, xyz(o), xyz(dd), kMaxDistance, kInvalid, kInvalid, bt, bi,
-                                          bp, stk + tid, kBlock, cnt, ovf);
+      traverse_mode<kTraceBounce, kWalk>(FS.fb[view].S, xyz(o), xyz(dd), kMaxDistance, kInvalid, kInvalid, bt, bi,
+                                         bp, stk + tid, kBlock, cnt, ovf);
       F0.seg_hit[q] = make_float4(bt, __uint_as_float(bi), __uint_as_float(bp), 0.0f);
     }
   }
-  if (kCount) wave_add_cnt(cnt, stats);
+  if (kWalk == kWalkCount) wave_add_cnt(cnt, stats);
 }
 
 // One path-loop iteration for every path of queue `d & 1`.
@@ -1495,9 +1503,9 @@ __global__ void __launch_bounds__(kBlock) k_pt_end(FrameSet FS) {
 // queue k holds the pixels whose slot-k shift replays a source path (slot
 // 0 from the pixel's own primary hit, slot 1 from the previous pixel's);
 // each result replaces the request in the pixel's retrace record.
-template <bool kMulti>
+template <int kWalk, bool kMulti>
 __global__ void __launch_bounds__(kBlock) k_pt_retrace(FrameSet FS) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const DFrame &F0 = FS.fb[0];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t n0 = F0.counters[kCntPtQueue], n = n0 + F0.counters[kCntPtQueue + 1];
@@ -1520,7 +1528,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_retrace(FrameSet FS) {
       src.flags = __float_as_uint(req.z);
       const Isect dst = slot == 0u ? isect_from_di(F, ld_di(F.dpos_c, F.dnrm_c, F.dorg_c, F.dhit_c, di_index))
                                    : isect_from_di_raw(F, ld_di(F.dpos_p, F.dnrm_p, F.dorg_p, F.dhit_p, di_index));
-      st_rc(F, px, slot, hybrid_retrace(F, dst, src, tr));
+      st_rc(F, px, slot, hybrid_retrace<kWalk>(F, dst, src, tr));
     }
   }
 }
@@ -1528,9 +1536,9 @@ __global__ void __launch_bounds__(kBlock) k_pt_retrace(FrameSet FS) {
 // Spatial path reuse (indirect_illumination_spatial_reuse, rgen.glsl:427-452)
 // and the rest of the shading pass: indirect term, emission, NaN scrub,
 // image store (rgen.glsl:449-489).
-template <bool kCount, bool kHybrid>
+template <int kWalk, bool kHybrid>
 __global__ void __launch_bounds__(kBlock) k_pt_spatial(FrameSet FS, unsigned long long *stats) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint2 blk_ = FS.blk[blockIdx.x];
   const DFrame &F = FS.fb[blk_.x];
   uint32_t px;
@@ -1548,7 +1556,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_spatial(FrameSet FS, unsigned lon
     if (F.rp.pt_spatial) {
       const Isect ci = isect_from_di(F, di);
       const F3 cam = f3(F.inv_view[12], F.inv_view[13], F.inv_view[14]);
-      const PRes fin = pt_spatial<kCount, kHybrid>(F, x, y, ci, cam, seed, tr);
+      const PRes fin = pt_spatial<kWalk, kHybrid>(F, x, y, ci, cam, seed, tr);
       st_pres(F.pres_t, px, fin);
       ind = muls(fin.F, fin.weight);
     } else {
@@ -1570,15 +1578,15 @@ __global__ void __launch_bounds__(kBlock) k_pt_spatial(FrameSet FS, unsigned lon
     F.dorg_p[px].w = __uint_as_float(seed);
   }
   wave_add(tr.shadow_rays, &F.counters[kCntPtShadow]);
-  if (kCount) wave_add_cnt(tr.cnt, stats + 9);
+  if (kWalk == kWalkCount) wave_add_cnt(tr.cnt, stats + 9);
 }
 
 // Path segments on caller rays (ct_trace_bounce).
-template <bool kCount>
+template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_trace_bounce(DFrame F, const float4 *ro, const float4 *rd, uint32_t n,
                                                         float4 *pos_dist, float4 *nrm_ids, float4 *wo_prim,
                                                         unsigned long long *stats) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   PtTrace tr;
   tr.stk = stk + threadIdx.x;
@@ -1586,13 +1594,13 @@ __global__ void __launch_bounds__(kBlock) k_trace_bounce(DFrame F, const float4 
   tr.shadow_rays = 0u;
   tr.overflow = false;
   if (i < n) {
-    const Isect h = bounce_intersect<kCount>(F, xyz(ro[i]), xyz(rd[i]), tr);
+    const Isect h = bounce_intersect<kWalk>(F, xyz(ro[i]), xyz(rd[i]), tr);
     const uint32_t inst = h.is_hit ? h.inst : kInvalid, prim = h.is_hit ? h.prim : kInvalid;
     pos_dist[i] = make_float4(h.P.x, h.P.y, h.P.z, h.distance);
     nrm_ids[i] = make_float4(h.n.x, h.n.y, h.n.z, __uint_as_float(inst));
     wo_prim[i] = make_float4(h.wo.x, h.wo.y, h.wo.z, __uint_as_float(prim));
   }
-  if (kCount) wave_add_cnt(tr.cnt, stats);
+  if (kWalk == kWalkCount) wave_add_cnt(tr.cnt, stats);
 }
 
 // taa.glsl:16-108 over the dispatch region.
@@ -1671,9 +1679,9 @@ __global__ void k_store_frame(DFrame F, DFrame *dst) {
 }
 
 // Any-hit traversal over a ray queue; each wave fetches 64 rays at a time.
-template <bool kCount>
+template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_trace_any(DScene S, TraceAnyArgs A) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   uint32_t count = *A.count;
   if (count > A.max_rays) count = A.max_rays;
@@ -1687,13 +1695,13 @@ __global__ void __launch_bounds__(kBlock) k_trace_any(DScene S, TraceAnyArgs A) 
       float bt = 0.0f;
       uint32_t bi = 0, bp = 0;
       bool ovf = false;
-      bool occ = traverse<true, kCount>(S, f3(o.x, o.y, o.z), f3(d.x, d.y, d.z), o.w, __float_as_uint(d.w), tp, bt, bi,
-                                        bp, stk + tid, kBlock, cnt, ovf);
+      bool occ = traverse_mode<kTraceAny, kWalk>(S, f3(o.x, o.y, o.z), f3(d.x, d.y, d.z), o.w, __float_as_uint(d.w), tp,
+                                                 bt, bi, bp, stk + tid, kBlock, cnt, ovf);
       if (occ && A.mask) atomicOr(&A.mask[idx / kRaySlots], 1u << (idx % kRaySlots));
       if (A.occ) A.occ[idx] = occ ? 1 : 0;
     }
   }
-  if (kCount) {
+  if (kWalk == kWalkCount) {
     unsigned long long a = cnt.nodes, b = cnt.leaves, c = cnt.insts;
     for (int off = 32; off > 0; off >>= 1) {
       a += __shfl_down(a, off);
@@ -1715,10 +1723,10 @@ __global__ void __launch_bounds__(kBlock) k_trace_any(DScene S, TraceAnyArgs A) 
 // its slot-1 rays (temporal reuse's target at the previous pixel) and kSel
 // 2 traces only those, in the previous set.
 constexpr int kSelAll = 0, kSelCurrent = 1, kSelPrevious = 2;
-template <bool kCount, bool kMulti, int kSel = kSelAll>
+template <int kWalk, bool kMulti, int kSel = kSelAll>
 __global__ void __launch_bounds__(kBlock) k_trace_any_frames(FrameSet FS, uint32_t max_rays,
                                                              unsigned long long *stats) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const DFrame &F0 = FS.fb[0];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t nfar = F0.counters[kCntQueue];
@@ -1739,18 +1747,19 @@ __global__ void __launch_bounds__(kBlock) k_trace_any_frames(FrameSet FS, uint32
         float bt = 0.0f;
         uint32_t bi = 0, bp = 0;
         bool ovf = false;
-        const bool occ = traverse<true, kCount>(kSel == kSelPrevious ? F.Sp : F.S, xyz(o), xyz(d), o.w,
-                                                __float_as_uint(d.w), tp, bt, bi, bp, stk + tid, kBlock, cnt, ovf);
+        const bool occ = traverse_mode<kTraceAny, kWalk>(kSel == kSelPrevious ? F.Sp : F.S, xyz(o), xyz(d), o.w,
+                                                         __float_as_uint(d.w), tp, bt, bi, bp, stk + tid, kBlock, cnt,
+                                                         ovf);
         if (occ) atomicOr(&F.mask[idx / kRaySlots], 1u << (idx % kRaySlots));
       }
     }
   }
-  if (kCount) wave_add_cnt(cnt, stats);
+  if (kWalk == kWalkCount) wave_add_cnt(cnt, stats);
 }
 
-template <bool kCount>
+template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_trace_closest(DScene S, TraceClosestArgs A) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t i = blockIdx.x * blockDim.x + tid;
   TraceCnt cnt;
@@ -1759,11 +1768,11 @@ __global__ void __launch_bounds__(kBlock) k_trace_closest(DScene S, TraceClosest
     float bt = A.tmax;
     uint32_t bi = kInvalid, bp = kInvalid;
     bool ovf = false;
-    traverse<false, kCount>(S, f3(o.x, o.y, o.z), f3(d.x, d.y, d.z), A.tmax, kInvalid, kInvalid, bt, bi, bp, stk + tid,
-                            kBlock, cnt, ovf);
+    traverse_mode<kTraceClosest, kWalk>(S, f3(o.x, o.y, o.z), f3(d.x, d.y, d.z), A.tmax, kInvalid, kInvalid, bt, bi, bp,
+                                        stk + tid, kBlock, cnt, ovf);
     A.hit[i] = make_float4(bi != kInvalid ? bt : -1.0f, __uint_as_float(bi), __uint_as_float(bp), 0.0f);
   }
-  if (kCount) {
+  if (kWalk == kWalkCount) {
     unsigned long long a = cnt.nodes, b = cnt.leaves, c = cnt.insts;
     for (int off = 32; off > 0; off >>= 1) {
       a += __shfl_down(a, off);
@@ -1803,47 +1812,59 @@ uint32_t resident_grid(K kernel) {
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kBlock, 0) != hipSuccess || per_cu < 1) per_cu = 1;
   return (uint32_t)(per_cu * cus);
 }
-template <bool kCount, bool kMulti, int kSel = kSelAll>
+template <int kWalk, bool kMulti, int kSel = kSelAll>
 uint32_t any_resident() {
-  static const uint32_t n = resident_grid(k_trace_any_frames<kCount, kMulti, kSel>);
+  static const uint32_t n = resident_grid(k_trace_any_frames<kWalk, kMulti, kSel>);
   return n;
 }
-template <bool kCount>
+template <int kWalk>
 uint32_t any_single_resident() {
-  static const uint32_t n = resident_grid(k_trace_any<kCount>);
+  static const uint32_t n = resident_grid(k_trace_any<kWalk>);
   return n;
 }
-template <bool kCount, bool kMulti>
+template <int kWalk, bool kMulti>
 uint32_t segments_resident() {
-  static const uint32_t n = resident_grid(k_trace_segments<kCount, kMulti>);
+  static const uint32_t n = resident_grid(k_trace_segments<kWalk, kMulti>);
   return n;
 }
-template <bool kMulti>
+template <int kWalk, bool kMulti>
 uint32_t retrace_resident() {
-  static const uint32_t n = resident_grid(k_pt_retrace<kMulti>);
+  static const uint32_t n = resident_grid(k_pt_retrace<kWalk, kMulti>);
   return n;
+}
+
+// How a launch over a scene walks it: with counters (the BVH's) when they
+// are asked for, through the cell grid when the scene has one.
+int scene_walk(const DScene &s, bool counted) { return counted ? kWalkCount : (s.grid.bricks ? kWalkGrid : kWalkBvh); }
+// Calls f with the walk as a compile-time constant.
+template <class F>
+void with_walk(int walk, F f) {
+  if (walk == kWalkGrid)
+    f(std::integral_constant<int, kWalkGrid>{});
+  else if (walk == kWalkCount)
+    f(std::integral_constant<int, kWalkCount>{});
+  else
+    f(std::integral_constant<int, kWalkBvh>{});
 }
 
 }  // namespace
 
 int launch_trace_any(const DScene &s, const TraceAnyArgs &a, hipStream_t st) {
   hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, a.head, 0, 1);
-  const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(a.max_rays), 1),
-                                           a.stats ? any_single_resident<true>() : any_single_resident<false>());
-  if (a.stats)
-    hipLaunchKernelGGL(k_trace_any<true>, dim3(grid), dim3(kBlock), 0, st, s, a);
-  else
-    hipLaunchKernelGGL(k_trace_any<false>, dim3(grid), dim3(kBlock), 0, st, s, a);
+  with_walk(scene_walk(s, a.stats != nullptr), [&](auto w) {
+    constexpr int kWalk = decltype(w)::value;
+    const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(a.max_rays), 1), any_single_resident<kWalk>());
+    hipLaunchKernelGGL(k_trace_any<kWalk>, dim3(grid), dim3(kBlock), 0, st, s, a);
+  });
   CT_HIP(hipGetLastError());
   return CT_OK;
 }
 
 int launch_trace_closest(const DScene &s, const TraceClosestArgs &a, hipStream_t st) {
   if (a.n == 0) return CT_OK;
-  if (a.stats)
-    hipLaunchKernelGGL(k_trace_closest<true>, dim3(nblocks(a.n)), dim3(kBlock), 0, st, s, a);
-  else
-    hipLaunchKernelGGL(k_trace_closest<false>, dim3(nblocks(a.n)), dim3(kBlock), 0, st, s, a);
+  with_walk(scene_walk(s, a.stats != nullptr), [&](auto w) {
+    hipLaunchKernelGGL(k_trace_closest<decltype(w)::value>, dim3(nblocks(a.n)), dim3(kBlock), 0, st, s, a);
+  });
   CT_HIP(hipGetLastError());
   return CT_OK;
 }
@@ -2142,27 +2163,36 @@ struct Launch {
   bool prev_trace = false;     // some frame traces the previous set (DFrame::prev_set)
   bool hybrid = false;         // some frame's path reuse uses the hybrid shift
   bool ris_brdf = false;       // some frame's RIS has the BRDF strategy on
+  int walk = kWalkBvh;         // kWalkCount with stats, kWalkGrid when every scene of the set has a grid
   uint32_t *counters = nullptr;
   unsigned long long *stats = nullptr;
 };
 
-template <bool kCount, bool kMulti, int kSel>
-void launch_any_frames(const Launch &L, FrameSet fs, uint32_t max_rays, hipStream_t st) {
-  const uint32_t grid = std::min<uint32_t>(std::min<uint32_t>(std::max<uint32_t>(nblocks(max_rays), 1), L.trace_blocks),
-                                           any_resident<kCount, kMulti, kSel>());
-  hipLaunchKernelGGL((k_trace_any_frames<kCount, kMulti, kSel>), dim3(grid), dim3(kBlock), 0, st, fs, max_rays,
-                     L.stats);
+// Blocks of a persistent traversal launch: those that can be resident, for
+// the BVH walks also at most the set's own bound.
+template <int kWalk>
+uint32_t trace_blocks(const Launch &L, uint32_t resident) {
+  return kWalk == kWalkGrid ? resident : std::min<uint32_t>(L.trace_blocks, resident);
 }
+
 // The queue length and the fetch head (kCntHead) are zeroed by the caller
-// before the pass that fills the queue.
+// before the pass that fills the queue.  The previous set has no grid.
 template <int kSel = kSelAll>
 void launch_any(const Launch &L, FrameSet fs, uint32_t max_rays, hipStream_t st) {
-  if (L.stats)
-    L.multi ? launch_any_frames<true, true, kSel>(L, fs, max_rays, st)
-            : launch_any_frames<true, false, kSel>(L, fs, max_rays, st);
-  else
-    L.multi ? launch_any_frames<false, true, kSel>(L, fs, max_rays, st)
-            : launch_any_frames<false, false, kSel>(L, fs, max_rays, st);
+  with_walk(kSel == kSelPrevious && L.walk == kWalkGrid ? kWalkBvh : L.walk, [&](auto w) {
+    constexpr int kWalk = decltype(w)::value;
+    auto go = [&](auto m) {
+      constexpr bool kMulti = decltype(m)::value;
+      const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(max_rays), 1),
+                                               trace_blocks<kWalk>(L, any_resident<kWalk, kMulti, kSel>()));
+      hipLaunchKernelGGL((k_trace_any_frames<kWalk, kMulti, kSel>), dim3(grid), dim3(kBlock), 0, st, fs, max_rays,
+                         L.stats);
+    };
+    if (L.multi)
+      go(std::true_type{});
+    else
+      go(std::false_type{});
+  });
 }
 
 // The command list of App::draw (main.cpp:1436-1703) for every frame of the
@@ -2187,13 +2217,16 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
   hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, L.counters, 0, 8);
   if (L.stats) hipLaunchKernelGGL(k_reset_u64, dim3(1), dim3(64), 0, st, L.stats, 12);
   if ((rc = mark())) return rc;  // kMarkStart
-  if (L.stats)
-    hipLaunchKernelGGL(k_primary<true>, dim3(L.blocks[0]), dim3(kBlock), 0, st, tiles, L.stats + 3);
-  else
-    hipLaunchKernelGGL(k_primary<false>, dim3(L.blocks[0]), dim3(kBlock), 0, st, tiles, L.stats);
+  with_walk(L.walk, [&](auto w) {
+    hipLaunchKernelGGL(k_primary<decltype(w)::value>, dim3(L.blocks[0]), dim3(kBlock), 0, st, tiles,
+                       L.stats ? L.stats + 3 : nullptr);
+  });
   if ((rc = mark())) return rc;  // kMarkPrimary
   if (L.ris_brdf)
-    hipLaunchKernelGGL(k_ris_brdf, dim3(nb), dim3(kBlock), 0, st, pix);
+    with_walk(L.walk == kWalkCount ? kWalkBvh : L.walk, [&](auto w) {
+      constexpr int kWalk = decltype(w)::value == kWalkGrid ? kWalkGrid : kWalkBvh;  // never counted
+      hipLaunchKernelGGL(k_ris_brdf<kWalk>, dim3(nb), dim3(kBlock), 0, st, pix);
+    });
   else
     hipLaunchKernelGGL(k_ris, dim3(nb), dim3(kBlock), 0, st, pix);
   if ((rc = mark())) return rc;  // kMarkRis
@@ -2216,23 +2249,26 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
                        (1u << kCntPtQueue) | (1u << (kCntPtQueue + 1)) | (1u << kCntPtHead) | (1u << kCntQueue) |
                            (1u << kCntQueueNear) | (1u << kCntHead));
     hipLaunchKernelGGL(k_pt_begin, dim3(nb), dim3(kBlock), 0, st, pix);
-    const uint32_t grid = std::min<uint32_t>(std::min<uint32_t>(std::max<uint32_t>(nblocks(np), 1), L.trace_blocks),
-                                             L.stats ? (L.multi ? segments_resident<true, true>() : segments_resident<true, false>())
-                                                     : (L.multi ? segments_resident<false, true>() : segments_resident<false, false>()));
     for (uint32_t d = 0; d < L.pt_depth; ++d) {
       // the next queue and the fetch counter start at zero (already so at depth 0)
       if (d > 0)
         hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters,
                            (1u << (kCntPtQueue + ((d + 1) & 1u))) | (1u << kCntPtHead));
       if ((rc = seg_mark())) return rc;
-      if (L.stats && L.multi)
-        hipLaunchKernelGGL((k_trace_segments<true, true>), dim3(grid), dim3(kBlock), 0, st, pix, d, L.stats + 6);
-      else if (L.stats)
-        hipLaunchKernelGGL((k_trace_segments<true, false>), dim3(grid), dim3(kBlock), 0, st, pix, d, L.stats + 6);
-      else if (L.multi)
-        hipLaunchKernelGGL((k_trace_segments<false, true>), dim3(grid), dim3(kBlock), 0, st, pix, d, L.stats);
-      else
-        hipLaunchKernelGGL((k_trace_segments<false, false>), dim3(grid), dim3(kBlock), 0, st, pix, d, L.stats);
+      with_walk(L.walk, [&](auto w) {
+        constexpr int kWalk = decltype(w)::value;
+        auto go = [&](auto m) {
+          constexpr bool kMulti = decltype(m)::value;
+          const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(np), 1),
+                                                   trace_blocks<kWalk>(L, segments_resident<kWalk, kMulti>()));
+          hipLaunchKernelGGL((k_trace_segments<kWalk, kMulti>), dim3(grid), dim3(kBlock), 0, st, pix, d,
+                             L.stats ? L.stats + 6 : nullptr);
+        };
+        if (L.multi)
+          go(std::true_type{});
+        else
+          go(std::false_type{});
+      });
       if ((rc = seg_mark())) return rc;
       if (L.multi)
         hipLaunchKernelGGL(k_pt_step<true>, dim3(nblocks(np)), dim3(kBlock), 0, st, pix, d);
@@ -2245,13 +2281,19 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
       hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters,
                          (1u << kCntPtQueue) | (1u << (kCntPtQueue + 1)) | (1u << kCntPtHead));
       hipLaunchKernelGGL((k_pt_end<kVisRequest, true>), dim3(nb), dim3(kBlock), 0, st, pix);
-      const uint32_t rgrid =
-          std::min<uint32_t>(std::min<uint32_t>(std::max<uint32_t>(nblocks(2 * np), 1), L.trace_blocks),
-                             L.multi ? retrace_resident<true>() : retrace_resident<false>());
-      if (L.multi)
-        hipLaunchKernelGGL(k_pt_retrace<true>, dim3(rgrid), dim3(kBlock), 0, st, pix);
-      else
-        hipLaunchKernelGGL(k_pt_retrace<false>, dim3(rgrid), dim3(kBlock), 0, st, pix);
+      with_walk(L.walk, [&](auto w) {
+        constexpr int kWalk = decltype(w)::value == kWalkGrid ? kWalkGrid : kWalkBvh;  // never counted
+        auto go = [&](auto m) {
+          constexpr bool kMulti = decltype(m)::value;
+          const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(2 * np), 1),
+                                                   trace_blocks<kWalk>(L, retrace_resident<kWalk, kMulti>()));
+          hipLaunchKernelGGL((k_pt_retrace<kWalk, kMulti>), dim3(grid), dim3(kBlock), 0, st, pix);
+        };
+        if (L.multi)
+          go(std::true_type{});
+        else
+          go(std::false_type{});
+      });
       hipLaunchKernelGGL((k_pt_end<kVisEmit, true>), dim3(nb), dim3(kBlock), 0, st, pix);
     } else {
       hipLaunchKernelGGL((k_pt_end<kVisEmit, false>), dim3(nb), dim3(kBlock), 0, st, pix);
@@ -2274,14 +2316,13 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
   hipLaunchKernelGGL(k_spatial<false>, dim3(L.blocks[1]), dim3(kBlock), 0, st, runs);
   if ((rc = mark())) return rc;  // kMarkSpatialFinish
   if (L.pt_depth) {
-    if (L.stats && L.hybrid)
-      hipLaunchKernelGGL((k_pt_spatial<true, true>), dim3(nb), dim3(kBlock), 0, st, pix, L.stats);
-    else if (L.stats)
-      hipLaunchKernelGGL((k_pt_spatial<true, false>), dim3(nb), dim3(kBlock), 0, st, pix, L.stats);
-    else if (L.hybrid)
-      hipLaunchKernelGGL((k_pt_spatial<false, true>), dim3(nb), dim3(kBlock), 0, st, pix, L.stats);
-    else
-      hipLaunchKernelGGL((k_pt_spatial<false, false>), dim3(nb), dim3(kBlock), 0, st, pix, L.stats);
+    with_walk(L.walk, [&](auto w) {
+      constexpr int kWalk = decltype(w)::value;
+      if (L.hybrid)
+        hipLaunchKernelGGL((k_pt_spatial<kWalk, true>), dim3(nb), dim3(kBlock), 0, st, pix, L.stats);
+      else
+        hipLaunchKernelGGL((k_pt_spatial<kWalk, false>), dim3(nb), dim3(kBlock), 0, st, pix, L.stats);
+    });
   }
   if ((rc = mark())) return rc;  // kMarkPtSpatial
   }
@@ -2340,8 +2381,9 @@ void split_tables(const DFrame &F, uint32_t parts, std::vector<uint2> *tbl, uint
 // reached, the reservoir's path length and reconnection length, the vertex
 // at that length (instance, primitive, hit xyz bits), the vertex before it
 // (instance, primitive), and 0.
+template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_pt_replay(DFrame F, int32_t dx, int32_t dy, uint32_t *out) {
-  __shared__ uint32_t stk[(kStackLds > 0 ? kStackLds : 1) * kBlock];
+  __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint32_t px = blockIdx.x * blockDim.x + threadIdx.x;
   if (px >= F.npix) return;
   uint32_t *o = out + 12 * (size_t)px;
@@ -2365,7 +2407,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_replay(DFrame F, int32_t dx, int3
   tr.emitted = 0u;
   tr.far = 0u;
   const DI di = ld_di(F.dpos_c, F.dnrm_c, F.dorg_c, F.dhit_c, px);
-  const Replay rp = pt_replay(F, isect_from_di(F, di), r.init_seed, rc_len, tr);
+  const Replay rp = pt_replay<kWalk>(F, isect_from_di(F, di), r.init_seed, rc_len, tr);
   o[0] = rp.ok ? 1u : 0u;
   o[1] = rp.length;
   o[4] = rp.rc.inst;
@@ -2675,7 +2717,7 @@ int ct_batch_render(ct_batch *b, const ct_frame_params *params, int use_graph, v
   for (uint32_t g = 0; g < ng; ++g) {
     BatchGroup &G = b->groups[g];
     uint32_t pt_depth = 0, max_nb = 0, px = 0;
-    bool prev_trace = false, hybrid = false, ris_brdf = false;
+    bool prev_trace = false, hybrid = false, ris_brdf = false, grids = true;
     for (uint32_t i = G.first; i < G.first + G.count; ++i) {
       DFrame &F = rec[i];
       if ((rc = prepare_frame(b->ctxs[i], b->accels[i], &params[i], st, F))) return rc;
@@ -2695,6 +2737,7 @@ int ct_batch_render(ct_batch *b, const ct_frame_params *params, int use_graph, v
       prev_trace = prev_trace || F.prev_set != 0u;
       hybrid = hybrid || (F.rp.indirect && F.rp.pt_shift_mapping == CT_SHIFT_HYBRID);
       ris_brdf = ris_brdf || (F.active & CT_RIS_BRDF_BIT) != 0u;
+      grids = grids && F.S.grid.bricks != nullptr;
     }
     L[g].fb = b->frames.as<DFrame>() + G.first;
     L[g].total_px = px;
@@ -2705,6 +2748,7 @@ int ct_batch_render(ct_batch *b, const ct_frame_params *params, int use_graph, v
     L[g].prev_trace = prev_trace;
     L[g].hybrid = hybrid;
     L[g].ris_brdf = ris_brdf;
+    L[g].walk = grids ? kWalkGrid : kWalkBvh;
     L[g].counters = G.counters.as<uint32_t>();
     L[g].stats = nullptr;
   }
@@ -2756,7 +2800,8 @@ int ct_batch_render(ct_batch *b, const ct_frame_params *params, int use_graph, v
     std::vector<uint32_t> gkey = tkey;
     for (uint32_t g = 0; g < ng; ++g)
       gkey.insert(gkey.end(), {L[g].total_px, L[g].pt_depth, L[g].max_neighbors, L[g].trace_blocks, (uint32_t)L[g].multi,
-                               (uint32_t)L[g].prev_trace, (uint32_t)L[g].hybrid, (uint32_t)L[g].ris_brdf});
+                               (uint32_t)L[g].prev_trace, (uint32_t)L[g].hybrid, (uint32_t)L[g].ris_brdf,
+                               (uint32_t)L[g].walk});
     if (!b->exec || gkey != b->graph_key) {
       drop_graph(b);
       CT_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
@@ -2961,6 +3006,7 @@ int ct_frame_render(ct_ctx *c, ct_accel *a, const ct_frame_params *p, void *stre
       L[k].prev_trace = F.prev_set != 0u;
       L[k].hybrid = F.rp.indirect && F.rp.pt_shift_mapping == CT_SHIFT_HYBRID;
       L[k].ris_brdf = (F.active & CT_RIS_BRDF_BIT) != 0u;
+      L[k].walk = scene_walk(F.S, false);
       L[k].counters = FP[k].counters;
       L[k].stats = nullptr;
     }
@@ -3013,6 +3059,7 @@ int ct_frame_render(ct_ctx *c, ct_accel *a, const ct_frame_params *p, void *stre
     L.prev_trace = F.prev_set != 0u;
     L.hybrid = F.rp.indirect && F.rp.pt_shift_mapping == CT_SHIFT_HYBRID;
     L.ris_brdf = (F.active & CT_RIS_BRDF_BIT) != 0u;
+    L.walk = scene_walk(F.S, stats != nullptr);
     L.counters = F.counters;
     L.stats = stats;
     const bool ev = (c->instrument & 1u) != 0;
@@ -3075,13 +3122,11 @@ int ct_trace_bounce(ct_accel *a, uint32_t n, const float *origins, const float *
   F.aabbs = a->set.aabbs.as<ct_aabb>();
   F.prims = a->set.prims.as<ct_primitive>();
   F.n_mats = 0;  // materials live in a frame context; the records here carry indices only
-  if (stats)
-    hipLaunchKernelGGL(k_trace_bounce<true>, dim3(nblocks(n)), dim3(kBlock), 0, a->stream, F, o.as<float4>(),
-                       d.as<float4>(), n, r0.as<float4>(), r1.as<float4>(), r2.as<float4>(),
-                       st.as<unsigned long long>());
-  else
-    hipLaunchKernelGGL(k_trace_bounce<false>, dim3(nblocks(n)), dim3(kBlock), 0, a->stream, F, o.as<float4>(),
-                       d.as<float4>(), n, r0.as<float4>(), r1.as<float4>(), r2.as<float4>(), nullptr);
+  with_walk(scene_walk(F.S, stats != nullptr), [&](auto w) {
+    hipLaunchKernelGGL(k_trace_bounce<decltype(w)::value>, dim3(nblocks(n)), dim3(kBlock), 0, a->stream, F,
+                       o.as<float4>(), d.as<float4>(), n, r0.as<float4>(), r1.as<float4>(), r2.as<float4>(),
+                       stats ? st.as<unsigned long long>() : nullptr);
+  });
   CT_HIP(hipGetLastError());
   CT_HIP(hipStreamSynchronize(a->stream));
   std::vector<float4> a0(n), a1(n), a2(n);
@@ -3121,7 +3166,10 @@ int ct_pt_random_replay(ct_ctx *c, ct_accel *a, const ct_frame_params *p, int32_
   int rc = prepare_frame(c, a, p, st, F);
   if (rc) return rc;
   c->cur ^= 1;  // prepare_frame advanced the image ping-pong; a replay renders nothing
-  hipLaunchKernelGGL(k_pt_replay, dim3(nblocks(F.npix)), dim3(kBlock), 0, st, F, dx, dy, out);
+  with_walk(scene_walk(F.S, false), [&](auto w) {
+    constexpr int kWalk = decltype(w)::value == kWalkGrid ? kWalkGrid : kWalkBvh;
+    hipLaunchKernelGGL(k_pt_replay<kWalk>, dim3(nblocks(F.npix)), dim3(kBlock), 0, st, F, dx, dy, out);
+  });
   CT_HIP(hipGetLastError());
   CT_HIP(hipStreamSynchronize(st));
   return CT_OK;

@@ -270,13 +270,13 @@ CT_D uint32_t material_of(const DFrame &F, uint32_t inst, uint32_t prim) {
 // intersect(), bounce.glsl:9-130: the box tests start at the origin pushed
 // along the ray (compute_ray_origin(origin, dir)); distance and wo use the
 // un-pushed origin.
-template <bool kCount>
+template <int kWalk>
 CT_D Isect bounce_intersect(const DFrame &F, F3 origin, F3 dir, PtTrace &tr) {
   const F3 ro = compute_ray_origin(origin, dir);
   float bt = kMaxDistance;
   uint32_t bi = kInvalid, bp = kInvalid;
   ++tr.bounce_rays;
-  traverse_mode<kTraceBounce, kCount>(F.S, ro, dir, kMaxDistance, kInvalid, kInvalid, bt, bi, bp, tr.stk, kBlock,
+  traverse_mode<kTraceBounce, kWalk>(F.S, ro, dir, kMaxDistance, kInvalid, kInvalid, bt, bi, bp, tr.stk, kBlock,
                                       tr.cnt, tr.overflow);
   Isect i = isect_empty();
   i.mat_idx = 0u;
@@ -308,14 +308,14 @@ constexpr int kVisInline = 0, kVisEmit = 1, kVisFinish = 2;
 constexpr int kVisRequest = 3;
 
 // is_vertex_visible (light.glsl:82-142) on the current TLAS.
-template <bool kCount, int kVis = kVisInline>
+template <int kWalk, int kVis = kVisInline>
 CT_D bool vertex_visible(const DFrame &F, F3 o, F3 d, float dist, uint32_t ti, uint32_t tp, PtTrace &tr) {
   if (kVis == kVisRequest) return true;
   if (kVis == kVisInline) {
     float bt = 0.0f;
     uint32_t bi = kInvalid, bp = kInvalid;
     ++tr.shadow_rays;
-    return !traverse_mode<kTraceAny, kCount>(F.S, o, d, dist, ti, tp, bt, bi, bp, tr.stk, kBlock, tr.cnt, tr.overflow);
+    return !traverse_mode<kTraceAny, kWalk>(F.S, o, d, dist, ti, tp, bt, bi, bp, tr.stk, kBlock, tr.cnt, tr.overflow);
   }
   const uint32_t k = tr.slot++;
   if (k >= kRaySlots) return true;  // at most two tests per pixel; never taken
@@ -703,6 +703,7 @@ struct Replay {
   F3 rc_prev_wo, thp;
 };
 
+template <int kWalk>
 CT_D Replay pt_replay(const DFrame &F, Isect i0, uint32_t seed, uint32_t rc_len, PtTrace &tr) {
   Replay r;
   r.ok = false;
@@ -719,7 +720,7 @@ CT_D Replay pt_replay(const DFrame &F, Isect i0, uint32_t seed, uint32_t rc_len,
     r.thp = p.thp;
   }
   while (more && p.path_length < rc_len) {
-    Isect i = bounce_intersect<false>(F, p.origin, p.dir, tr);
+    Isect i = bounce_intersect<kWalk>(F, p.origin, p.dir, tr);
     wo = i.wo;
     more = pt_step(F, p, i);
     if (!i.is_hit) break;
@@ -834,7 +835,7 @@ CT_D void ld_pstate(const float4 *S, uint32_t np, uint32_t p, PState &s, bool re
 // connection is rejected; with use_cached the source side's geometry term
 // and pdfs come from the reservoir's cached Jacobian, and a successful
 // shift leaves the destination's there.
-template <bool kCount, int kVis = kVisInline>
+template <int kWalk, int kVis = kVisInline>
 CT_D F3 shift_reconnection(const DFrame &F, float &dst_jac, Isect dst, Isect src, PRes &s, bool eval_vis,
                            PtTrace &tr, bool use_hybrid = false, bool use_cached = false) {
   dst_jac = 0.0f;
@@ -850,7 +851,7 @@ CT_D F3 shift_reconnection(const DFrame &F, float &dst_jac, Isect dst, Isect src
   if (!exists) {
     F3 integrand = f3(0, 0, 0);
     if (pf_light_type(s.flags) == kGeomLightEnv && plen + 1u == rc_len && !nee) {
-      if (vertex_visible<kCount, kVis>(F, dst.P, wi, kMaxDistance, kMaxInstances, kMaxPrimitives, tr)) {
+      if (vertex_visible<kWalk, kVis>(F, dst.P, wi, kMaxDistance, kMaxInstances, kMaxPrimitives, tr)) {
         const float src_pdf1 = use_cached ? s.cj.x : material_pdf(src.n, src.wo, wi);
         const float dst_pdf1 = material_pdf(dst.n, dst.wo, wi);
         dst_cj.x = dst_pdf1;
@@ -922,7 +923,7 @@ CT_D F3 shift_reconnection(const DFrame &F, float &dst_jac, Isect dst, Isect src
   if (eval_vis) {
     const F3 dir = normalize(sub(rc.P, dst.P));
     const float dist = length(sub(dst.P, rc.P));
-    if (!vertex_visible<kCount, kVis>(F, dst.P, dir, dist, rc.inst, rc.prim, tr)) return f3(0, 0, 0);
+    if (!vertex_visible<kWalk, kVis>(F, dst.P, dir, dist, rc.inst, rc.prim, tr)) return f3(0, 0, 0);
   }
   if (has_nan_inf(integrand)) return f3(0, 0, 0);
   dst_jac = jac;
@@ -986,6 +987,7 @@ CT_D RcData ld_rc(const DFrame &F, uint32_t px, uint32_t slot) {
 // reconnection vertex.  Not invertible (ok = false) if it misses, stops
 // early, reaches a connectable vertex before that one or that vertex is
 // not rough.
+template <int kWalk>
 CT_D RcData hybrid_retrace(const DFrame &F, Isect i0, const PRes &src, PtTrace &tr) {
   RcData out;
   out.ok = false;
@@ -1000,7 +1002,7 @@ CT_D RcData hybrid_retrace(const DFrame &F, Isect i0, const PRes &src, PtTrace &
   p.replay_rc = k;
   p.last_rough = i0.mat.roughness > F.rp.roughness_threshold;  // generate_replay_primary_scatter_ray
   while (more) {
-    Isect h = bounce_intersect<false>(F, p.origin, p.dir, tr);
+    Isect h = bounce_intersect<kWalk>(F, p.origin, p.dir, tr);
     more = pt_step(F, p, h);
   }
   if (p.replay_done) {
@@ -1026,14 +1028,14 @@ CT_D RcData hybrid_retrace(const DFrame &F, Isect i0, const PRes &src, PtTrace &
 // primary vertex where the text passes an invalid hit (:376-378).  A source
 // whose reconnection vertex does not exist (the path ended first) is not
 // shifted.
-template <bool kCount, int kVis = kVisInline, bool kHybrid = false>
+template <int kWalk, int kVis = kVisInline, bool kHybrid = false>
 CT_D F3 shifted_integrand(const DFrame &F, float &dst_jac, const Isect &dst, const Isect &src, PRes &s,
                           bool eval_vis, PtTrace &tr) {
   dst_jac = 0.0f;
   if (s.weight == 0.0f) return f3(0, 0, 0);
   const uint32_t mapping = F.rp.pt_shift_mapping;
   if (!kHybrid) {
-    if (mapping == CT_SHIFT_RECONNECTION) return shift_reconnection<kCount, kVis>(F, dst_jac, dst, src, s, eval_vis, tr);
+    if (mapping == CT_SHIFT_RECONNECTION) return shift_reconnection<kWalk, kVis>(F, dst_jac, dst, src, s, eval_vis, tr);
     return f3(1.0f, 1.0f, 1.0f);
   }
   // The hybrid build reaches one reconnection for both mappings (it serves
@@ -1057,7 +1059,7 @@ CT_D F3 shifted_integrand(const DFrame &F, float &dst_jac, const Isect &dst, con
         tr.rc_req |= 1u << tr.rc_slot;
         return f3(0, 0, 0);
       }
-      rc = kVis == kVisInline ? hybrid_retrace(F, dst, s, tr) : ld_rc(F, tr.px, tr.rc_slot);
+      rc = kVis == kVisInline ? hybrid_retrace<kWalk>(F, dst, s, tr) : ld_rc(F, tr.px, tr.rc_slot);
       if (!rc.ok) return f3(0, 0, 0);
       tp = rc.tp;
       retraced = true;
@@ -1065,24 +1067,24 @@ CT_D F3 shifted_integrand(const DFrame &F, float &dst_jac, const Isect &dst, con
     if (!(tp.x > 0.0f || tp.y > 0.0f || tp.z > 0.0f)) return f3(0, 0, 0);
   }
   float rj = 0.0f;
-  const F3 r = shift_reconnection<kCount, kVis>(F, rj, retraced ? rc.prev : dst, src, s, eval_vis, tr, hyb, retraced);
+  const F3 r = shift_reconnection<kWalk, kVis>(F, rj, retraced ? rc.prev : dst, src, s, eval_vis, tr, hyb, retraced);
   dst_jac = rj;  // the hybrid shift's 1.0f * rj
   return hyb ? mulv(tp, r) : r;
 }
 // compute_shifted_integrand, shift.glsl:485-497: on a copy of the reservoir.
-template <bool kCount, int kVis = kVisInline, bool kHybrid = false>
+template <int kWalk, int kVis = kVisInline, bool kHybrid = false>
 CT_D F3 shifted_integrand_copy(const DFrame &F, float &dst_jac, const Isect &dst, const Isect &src, const PRes &s,
                                bool eval_vis, PtTrace &tr) {
   PRes t = s;
-  return shifted_integrand<kCount, kVis, kHybrid>(F, dst_jac, dst, src, t, eval_vis, tr);
+  return shifted_integrand<kWalk, kVis, kHybrid>(F, dst_jac, dst, src, t, eval_vis, tr);
 }
 
 // shift_and_merge_reservoir, shift.glsl:485-510 (force_merge, mis 1)
-template <bool kCount, int kVis = kVisInline, bool kHybrid = false>
+template <int kWalk, int kVis = kVisInline, bool kHybrid = false>
 CT_D bool shift_and_merge(const DFrame &F, float &dst_jac, const Isect &dst, PRes &dst_res, const Isect &src,
                           const PRes &src_res, uint32_t &seed, PtTrace &tr) {
   PRes tmp = src_res;
-  const F3 integrand = shifted_integrand<kCount, kVis, kHybrid>(F, dst_jac, dst, src, tmp, true, tr);
+  const F3 integrand = shifted_integrand<kWalk, kVis, kHybrid>(F, dst_jac, dst, src, tmp, true, tr);
   const bool selected = pres_merge(dst_res, integrand, dst_jac, tmp, seed, 1.0f, true);
   if (!selected) dst_res.F = f3(0, 0, 0);
   dst_res.M = src_res.M;
@@ -1095,7 +1097,7 @@ CT_D bool shift_and_merge(const DFrame &F, float &dst_jac, const Isect &dst, PRe
 // then the history shifted here) exist or not by data alone, never by an
 // earlier test's outcome, so a queued pass records the same rays in the
 // same slots as the finishing pass reads.
-template <bool kCount, int kVis = kVisInline, bool kHybrid = false>
+template <int kWalk, int kVis = kVisInline, bool kHybrid = false>
 CT_D PRes pt_temporal(const DFrame &F, const PRes &central, PRes temporal, const Isect &cur_i, const Isect &prev_i,
                       uint32_t &seed, PtTrace &tr) {
   PRes dest = pres_init(F.rp.max_depth);
@@ -1112,7 +1114,7 @@ CT_D PRes pt_temporal(const DFrame &F, const PRes &central, PRes temporal, const
       possible = tdst.weight > 0.0f;
     } else {
       tr.rc_slot = 0u;  // the history shifted to this pixel's primary hit
-      possible = shift_and_merge<kCount, kVis, kHybrid>(F, dst_jac, cur_i, tdst, prev_i, temporal, seed, tr);
+      possible = shift_and_merge<kWalk, kVis, kHybrid>(F, dst_jac, cur_i, tdst, prev_i, temporal, seed, tr);
     }
     if (possible) {
       // j = -1
@@ -1126,7 +1128,7 @@ CT_D PRes pt_temporal(const DFrame &F, const PRes &central, PRes temporal, const
       } else {
         float tj = 0.0f;
         tr.rc_slot = 1u;  // this pixel's path shifted to the previous pixel's primary hit
-        const F3 ti = shifted_integrand_copy<kCount, kVis, kHybrid>(F, tj, prev_i, cur_i, tdst, true, tr);
+        const F3 ti = shifted_integrand_copy<kWalk, kVis, kHybrid>(F, tj, prev_i, cur_i, tdst, true, tr);
         const float pp = lum601(ti) * tj;
         p_sum += pp * temporal.M;
       }
@@ -1176,7 +1178,7 @@ CT_D Isect isect_from_di(const DFrame &F, const DI &d) {
 }
 
 // indirect_illumination_spatial_reuse, indirect_illumination.glsl:312-452
-template <bool kCount, bool kHybrid = false>
+template <int kWalk, bool kHybrid = false>
 CT_D PRes pt_spatial(const DFrame &F, uint32_t x, uint32_t y, const Isect &ci, F3 camera_pos, uint32_t &seed,
                      PtTrace &tr) {
   const uint32_t cur = y * F.W + x;
@@ -1201,7 +1203,7 @@ CT_D PRes pt_spatial(const DFrame &F, uint32_t x, uint32_t y, const Isect &ci, F
     const PRes nres = ld_pres(F.pres_o, ni);
     valid++;
     float prefix_jac = 0.0f;
-    const F3 prefix = shifted_integrand_copy<kCount, kVisInline, kHybrid>(F, prefix_jac, nis, ci, central, true, tr);
+    const F3 prefix = shifted_integrand_copy<kWalk, kVisInline, kHybrid>(F, prefix_jac, nis, ci, central, true, tr);
     const float prefix_pdf = lum601(prefix) * prefix_jac;
     canonical += 1.0f;
     if (prefix_pdf > 0.0f)
@@ -1209,7 +1211,7 @@ CT_D PRes pt_spatial(const DFrame &F, uint32_t x, uint32_t y, const Isect &ci, F
                    (prefix_pdf * nres.M + central.M * lum601(central.F) / (float)ncount);
     PRes tdst = dest;
     float dst_jac = 0.0f;
-    const bool possible = shift_and_merge<kCount, kVisInline, kHybrid>(F, dst_jac, ci, tdst, nis, nres, seed, tr);
+    const bool possible = shift_and_merge<kWalk, kVisInline, kHybrid>(F, dst_jac, ci, tdst, nis, nres, seed, tr);
     float nw = 0.0f;
     if (possible) {
       nw = lum601(nres.F) / dst_jac * nres.M /

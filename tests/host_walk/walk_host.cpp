@@ -1,0 +1,161 @@
+// Host build of the cell-grid walk (csrc/ct_device.h), called through ctypes:
+// each ray by the walk and by the voxel test on every voxel, with the same
+// voxel test on the same operands.
+#include "../../cube-tracing_amd/csrc/ct_device.h"
+
+#include <vector>
+
+namespace ct {
+int fail(int code, const std::string &) { return code; }
+}  // namespace ct
+using namespace ct;
+using namespace ct::dev;
+
+namespace {
+
+struct Scene {
+  std::vector<uint4> bricks;
+  std::vector<uint2> ids;
+  std::vector<float> boxes;
+  std::vector<uint32_t> cells;
+  std::vector<DInst> inst;
+  DScene S{};
+};
+
+// cells [n][3] of one instance's voxels (object space lattice), each once
+void build(Scene &sc, const int32_t *cells, uint32_t n, const float *w2o) {
+  int32_t lo[3], hi[3];
+  for (int a = 0; a < 3; ++a) {
+    lo[a] = hi[a] = cells[a];
+    for (uint32_t i = 0; i < n; ++i) {
+      lo[a] = std::min(lo[a], cells[3 * i + a]);
+      hi[a] = std::max(hi[a], cells[3 * i + a]);
+    }
+  }
+  DGrid &G = sc.S.grid;
+  uint32_t nb = 1;
+  for (int a = 0; a < 3; ++a) {
+    G.org[a] = (lo[a] - 4) & ~15;
+    G.nblk[a] = (uint32_t)(((hi[a] + 4) | 15) + 1 - G.org[a]) / 16;
+    nb *= G.nblk[a];
+  }
+  std::memcpy(G.w2o, w2o, sizeof(G.w2o));
+  sc.bricks.assign((size_t)nb * 64, uint4{0, 0, 0, 0});
+  auto at = [&](int32_t x, int32_t y, int32_t z) -> uint4 * {
+    const uint32_t ux = (uint32_t)(x - G.org[0]), uy = (uint32_t)(y - G.org[1]), uz = (uint32_t)(z - G.org[2]);
+    if (ux >= 16 * G.nblk[0] || uy >= 16 * G.nblk[1] || uz >= 16 * G.nblk[2]) return nullptr;
+    const uint32_t b = ((uz >> 4) * G.nblk[1] + (uy >> 4)) * G.nblk[0] + (ux >> 4);
+    return &sc.bricks[((size_t)b << 6) | ((ux >> 2) & 3u) | (uy & 12u) | ((uz & 12u) << 2)];
+  };
+  auto bit = [](int32_t x, int32_t y, int32_t z) { return (uint32_t)((x & 3) | ((y & 3) << 2) | ((z & 3) << 4)); };
+  for (uint32_t i = 0; i < n; ++i) {
+    uint4 *e = at(cells[3 * i], cells[3 * i + 1], cells[3 * i + 2]);
+    const uint32_t b = bit(cells[3 * i], cells[3 * i + 1], cells[3 * i + 2]);
+    (b < 32 ? e->x : e->y) |= 1u << (b & 31u);
+  }
+  uint32_t total = 0;
+  for (uint4 &e : sc.bricks) {
+    e.z = total;
+    total += (uint32_t)(__builtin_popcount(e.x) + __builtin_popcount(e.y));
+  }
+  // the largest empty cube of bricks into each octant, by its definition
+  auto occupied = [&](int32_t x, int32_t y, int32_t z) {
+    const uint4 *e = at(x, y, z);
+    return e && (e->x | e->y) != 0u;
+  };
+  for (uint32_t b = 0; b < nb; ++b)
+    for (uint32_t l = 0; l < 64; ++l) {
+      uint4 &e = sc.bricks[(size_t)b * 64 + l];
+      if (e.x | e.y) continue;
+      const int32_t x = G.org[0] + 16 * (int32_t)(b % G.nblk[0]) + 4 * (int32_t)(l & 3),
+                    y = G.org[1] + 16 * (int32_t)((b / G.nblk[0]) % G.nblk[1]) + 4 * (int32_t)((l >> 2) & 3),
+                    z = G.org[2] + 16 * (int32_t)(b / (G.nblk[0] * G.nblk[1])) + 4 * (int32_t)(l >> 4);
+      for (uint32_t o = 0; o < 8; ++o) {
+        uint32_t side = 1;
+        for (int32_t s = 2; s <= (int32_t)kGridSkip; ++s) {
+          bool empty = true;
+          for (int32_t k = 0; k < s * s * s && empty; ++k)
+            empty = !occupied(x + ((o & 1u) ? -4 : 4) * (k % s), y + ((o & 2u) ? -4 : 4) * (k / s % s),
+                              z + ((o & 4u) ? -4 : 4) * (k / (s * s)));
+          if (!empty) break;
+          side = (uint32_t)s;
+        }
+        e.w |= side << (4 * o);
+      }
+    }
+  sc.ids.resize(n);
+  sc.boxes.resize(6 * (size_t)n);
+  sc.cells.resize(n);
+  for (uint32_t i = 0; i < n; ++i) {
+    const int32_t *c = cells + 3 * i;
+    const uint4 *e = at(c[0], c[1], c[2]);
+    const uint64_t mask = ((uint64_t)e->y << 32) | e->x;
+    sc.ids[e->z + (uint32_t)__builtin_popcountll(mask & ((1ull << bit(c[0], c[1], c[2])) - 1ull))] = uint2{0u, i};
+    sc.cells[i] = (uint32_t)((e - sc.bricks.data()) << 6) | bit(c[0], c[1], c[2]);
+    for (int a = 0; a < 3; ++a) {
+      sc.boxes[6 * (size_t)i + a] = (float)c[a] * 0.03125f;
+      sc.boxes[6 * (size_t)i + 3 + a] = (float)(c[a] + 1) * 0.03125f;
+    }
+  }
+  sc.inst.resize(1);
+  std::memset(sc.inst.data(), 0, sizeof(DInst));
+  std::memcpy(sc.inst[0].w2o, w2o, sizeof(sc.inst[0].w2o));
+  sc.inst[0].count = n;
+  sc.S.inst = sc.inst.data();
+  sc.S.n_inst = 1;
+  G.bricks = sc.bricks.data();
+  G.ids = sc.ids.data();
+  G.cells = sc.cells.data();
+}
+
+template <int kMode>
+void both(const Scene &sc, const int32_t *cells, uint32_t n, F3 o, F3 d, float limit, uint32_t target, float *t_out,
+          uint32_t *id_out, float *t_ref, uint32_t *id_ref) {
+  float bt = limit;
+  uint32_t bi = kInvalid, bp = kInvalid;
+  TraceCnt cnt;
+  bool ovf = false;
+  const bool occ = traverse_mode<kMode, kWalkGrid>(sc.S, o, d, limit, target == kInvalid ? kInvalid : 0u, target, bt, bi,
+                                                   bp, nullptr, 0u, cnt, ovf);
+  *t_out = kMode == kTraceAny || bp == kInvalid ? 0.0f : bt;
+  *id_out = kMode == kTraceAny ? (uint32_t)occ : bp;
+  const float *m = sc.S.grid.w2o;
+  const F3 oo = xform3(m, o, 1.0f), od = xform3(m, d, 0.0f);
+  const F3 dr = kMode == kTraceClosest ? mul_rot(od) : od;
+  const F3 sg = f3(-gsign(dr.x), -gsign(dr.y), -gsign(dr.z));
+  const F3 inv = f3(safe_inverse(od.x), safe_inverse(od.y), safe_inverse(od.z));
+  float rt = limit;
+  uint32_t rp = kInvalid, hit_any = 0;
+  for (uint32_t i = 0; i < n; ++i) {
+    const float *b = &sc.boxes[6 * (size_t)i];
+    const F3 c = f3((b[0] + b[3]) * 0.5f, (b[1] + b[4]) * 0.5f, (b[2] + b[5]) * 0.5f);
+    float t;
+    if (kMode == kTraceAny) {
+      if (intersect_box<false, false>(c, oo, dr, sg, inv, t) && t >= 0.0f && t <= limit && i != target) hit_any = 1;
+    } else {
+      const bool hit = kMode == kTraceClosest ? intersect_box<true, true>(c, oo, dr, sg, inv, t)
+                                              : intersect_box<true, false>(c, oo, dr, sg, inv, t);
+      if (hit && (kMode == kTraceClosest ? t > 0.0f : t >= 0.0f) && (t < rt || (t == rt && i < rp))) {
+        rt = t;
+        rp = i;
+      }
+    }
+  }
+  *t_ref = kMode == kTraceAny || rp == kInvalid ? 0.0f : rt;
+  *id_ref = kMode == kTraceAny ? hit_any : rp;
+}
+
+}  // namespace
+
+extern "C" void walk_and_brute(const int32_t *cells, uint32_t n, const float *w2o, int mode, uint32_t rays,
+                               const float *o, const float *d, const float *limit, const uint32_t *target, float *t_out,
+                               uint32_t *id_out, float *t_ref, uint32_t *id_ref) {
+  Scene sc;
+  build(sc, cells, n, w2o);
+#pragma omp parallel for schedule(dynamic, 64)
+  for (uint32_t i = 0; i < rays; ++i) {
+    const F3 ro = f3(o[3 * i], o[3 * i + 1], o[3 * i + 2]), rd = f3(d[3 * i], d[3 * i + 1], d[3 * i + 2]);
+    auto fn = mode == kTraceAny ? both<kTraceAny> : mode == kTraceClosest ? both<kTraceClosest> : both<kTraceBounce>;
+    fn(sc, cells, n, ro, rd, limit[i], target[i], t_out + i, id_out + i, t_ref + i, id_ref + i);
+  }
+}

@@ -1,0 +1,114 @@
+"""Scenes with a cell grid are walked through it, except by counted launches
+(`stats`), which walk the BVH: both must give the same hits to the bit, and a
+scene that an update takes off the lattice must leave the grid."""
+import numpy as np
+import pytest
+
+import ctamd
+from ctamd import adjoint as adj
+
+pytestmark = pytest.mark.gpu
+
+
+def _load(grid, chunk, fill=0.2, seed=5):
+    d = ctamd.SceneDesc()
+    d.grid[:] = [grid] * 3
+    d.chunk[:] = [chunk] * 3
+    d.occupied_count = max(1, round(fill * grid ** 3))
+    d.le_min = d.le_max = 1.0
+    d.albedo_min, d.albedo_max = 0.2, 0.8
+    d.seed = seed
+    d.voxel_extent = ctamd.CT_VOXEL_EXTENT
+    sc = ctamd.Scene(d)
+    acc = ctamd.Accel(max_instances=sc.info.instance_count + 8,
+                      max_primitives=sc.info.primitive_count + 32 * sc.info.instance_count + 1024, max_cube_lights=8)
+    adj._load_geometry(sc, acc)
+    return sc, acc
+
+
+def _rays(rng, n, lo, hi):
+    """Rays from around and within, a third of them through lattice planes, edges and corners or along the axes."""
+    ext = float((hi - lo).max())
+    d = rng.normal(size=(n, 3))
+    d[::6] = rng.choice([-1.0, 0.0, 1.0], size=(len(d[::6]), 3))
+    d[1::6] *= rng.choice([0.0, 1e-7, 1e-4, 1.0], size=(len(d[1::6]), 3))
+    d[np.abs(d).sum(1) == 0] = [0, 1, 0]
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    to = rng.uniform(lo, hi, (n, 3))
+    to[::3] = np.round(to[::3] * 32) / 32 + rng.choice([0, 0, 1e-6, -1e-6, 1 / 64], size=(len(to[::3]), 3))
+    o = to - d * rng.choice([0, 0.05, 1.0, 3.0], size=(n, 1)) * ext
+    return np.ascontiguousarray(o, np.float32), np.ascontiguousarray(d, np.float32)
+
+
+def _same(acc, sc, seed, n=60000):
+    rng = np.random.default_rng(seed)
+    o, d = _rays(rng, n, sc.grid_min.astype(np.float64), sc.grid_max.astype(np.float64))
+    t, ids = acc.trace_closest(o, d)
+    bt, bids, _ = acc.trace_closest(o, d, stats=True)
+    assert np.array_equal(ids, bids) and np.array_equal(t.view(np.uint32), bt.view(np.uint32))
+    assert 0.02 < (ids[:, 0] != ctamd.CT_INVALID_INDEX).mean() < 1.0
+    g, b = acc.trace_bounce(o, d), acc.trace_bounce(o, d, stats=True)
+    for k in ("ids", "pos", "nrm", "dist", "wo"):
+        assert np.array_equal(g[k].view(np.uint32), b[k].view(np.uint32)), k
+    hit = ids[:, 0] != ctamd.CT_INVALID_INDEX
+    dist = np.where(hit, t * rng.choice([0.5, 1.0, 1.5], size=n), 2.0).astype(np.float32)
+    targets = np.where((rng.random(n) < 0.5)[:, None], ids, ctamd.CT_INVALID_INDEX).astype(np.uint32)
+    for tg in (None, targets):
+        occ, (bocc, _) = acc.trace_any(o, d, dist, tg), acc.trace_any(o, d, dist, tg, stats=True)
+        assert np.array_equal(occ, bocc)
+
+
+@pytest.mark.parametrize("grid,chunk,fill", [(1, 1, 1.0), (3, 3, 0.5), (17, 5, 0.3), (64, 16, 0.2), (130, 64, 0.02)])
+def test_grid_walk_equals_bvh_walk(gpu, grid, chunk, fill):
+    sc, acc = _load(grid, chunk, fill)
+    _same(acc, sc, grid)
+
+
+def test_grid_follows_updates(gpu):
+    sc, acc = _load(48, 16)
+    _same(acc, sc, 1)
+    n = [i.primitive_count for i in acc.read_instances()]
+    big = int(np.argmax(n))
+    box = acc.read_world()["aabbs"]
+    first = [i.first_primitive_index for i in acc.read_instances()]
+    old = box[first[big]].copy()
+    acc.delete_primitive(big, 3)  # the voxel leaves the grid
+    acc.update_scene()
+    _same(acc, sc, 2)
+    acc.undo()
+    acc.update_scene()
+    _same(acc, sc, 3)
+    acc.update_blas(big, edits=[(0, old + np.float32(0.007))])  # off the lattice
+    acc.update_scene()
+    _same(acc, sc, 4)
+    acc.update_blas(big, edits=[(0, box[first[big] + 1])])  # two voxels in one cell
+    acc.update_scene()
+    _same(acc, sc, 5)
+    acc.update_blas(big, edits=[(0, old + np.float32(0.5))])  # another cell of the lattice
+    acc.update_scene()
+    _same(acc, sc, 6)
+    acc.update_blas(big, edits=[(0, old)])
+    acc.update_scene()
+    m = np.eye(4, dtype=np.float32)
+    m[3, 0] = 0.25
+    acc.update_blas(big, transform=m.reshape(16))  # instances with different transforms
+    acc.update_scene()
+    _same(acc, sc, 7)
+    m[3, 0] = -0.25
+    acc.update_blas(big, transform=m.reshape(16))
+    acc.update_scene()
+    _same(acc, sc, 8)
+
+
+def test_grid_under_one_transform(gpu):
+    """A scene placed by one rotation and translation keeps its grid."""
+    d = ctamd.hd_di(width=16, height=16, grid=48, chunk=16)
+    sc = ctamd.Scene(ctamd.scene_desc(d))
+    acc = ctamd.Accel(max_instances=sc.info.instance_count + 8,
+                      max_primitives=sc.info.primitive_count + 32 * sc.info.instance_count + 1024,
+                      max_cube_lights=sc.info.cube_light_count + 8)
+    ctx = ctamd.Ctx(16, 16)
+    c, s = np.cos(0.7), np.sin(0.7)
+    m = np.array([[c, 0, -s, 0], [0, 1, 0, 0], [s, 0, c, 0], [0.1, -0.2, 0.05, 1]], np.float32)
+    ctamd.load_scene(sc, acc, ctx, transform=m.reshape(16))
+    _same(acc, sc, 9)
