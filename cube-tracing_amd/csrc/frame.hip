@@ -20,6 +20,7 @@
 
 #include "ct_device.h"
 #include "ct_internal.h"
+#include "cube_light.h"
 
 namespace ct {
 using namespace dev;
@@ -58,6 +59,7 @@ struct DFrame {
   uint32_t W, H, npix, frame, active, afternoon;
   float time;
   uint32_t n_cube, n_point, n_env, n_mats;
+  uint32_t cube_plain;  // every cube light is of type CUBE and emits
   float inv_view[16], inv_proj[16];
   ct_restir_params rp;
   ct_light_config cfg;
@@ -331,26 +333,6 @@ CT_D float geom_fact_sa(F3 P, F3 Ps, F3 ns) {
   F3 dd = sub(Ps, P);
   return fabsf(dot(ns, dir)) / dot(dd, dd);
 }
-// prng.glsl:198-252
-CT_D F3 random_cube_normal(uint32_t &seed) {
-  uint32_t face = min(urnd_interval(seed, 0u, 6u), 5u);
-  switch (face) {
-    case 0: return f3(-1, 0, 0);
-    case 1: return f3(1, 0, 0);
-    case 2: return f3(0, -1, 0);
-    case 3: return f3(0, 1, 0);
-    case 4: return f3(0, 0, -1);
-    default: return f3(0, 0, 1);
-  }
-}
-CT_D F3 random_quad(F3 n, F3 p, float sx, float sy, uint32_t &seed) {
-  float u = rnd(seed);
-  float v = rnd(seed);
-  float qx = u * sx, qy = v * sy;
-  F3 t1 = fabsf(n.x) > fabsf(n.y) ? normalize(f3(-n.z, 0.0f, n.x)) : normalize(f3(0.0f, n.z, -n.y));
-  F3 t2 = normalize(cross(n, t1));
-  return add(add(p, muls(t1, qx)), muls(t2, qy));
-}
 CT_D F3 random_on_hemisphere(uint32_t &seed, F3 n) {
   F3 p = f3(0, 0, 0);
   for (int k = 0; k < 1024; ++k) {
@@ -365,44 +347,6 @@ CT_D F3 random_on_hemisphere(uint32_t &seed, F3 n) {
   return dot(u, n) > 0.0f ? u : neg(u);
 }
 
-// LCG state after 33 steps: s * a^33 + c * (a^32 + ... + 1) (mod 2^32).
-constexpr uint32_t lcg_mul_pow(int k) {
-  uint32_t r = 1u;
-  for (int i = 0; i < k; ++i) r *= 1664525u;
-  return r;
-}
-constexpr uint32_t lcg_add_sum(int k) {
-  uint32_t r = 0u, p = 1u;
-  for (int i = 0; i < k; ++i) {
-    r += p;
-    p *= 1664525u;
-  }
-  return r * 1013904223u;
-}
-CT_D uint32_t lcg_skip33(uint32_t s) {
-  constexpr uint32_t A = lcg_mul_pow(33), C = lcg_add_sum(33);
-  return A * s + C;
-}
-// True when the light voxel lies wholly on the back side of the surface at
-// P (axis-aligned normal n): then dot(normalize(P - x), n) >= 0 for every
-// sample point x of the voxel, light.glsl:343 rejects all draws.  The
-// 1e-4 margin covers the rounding of the sample position; near-boundary
-// cases take the full loop.
-CT_D bool light_behind_surface(F3 P, F3 n, F3 c, float half) {
-  const float m = half + 1e-4f;
-  if (n.y == 0.0f && n.z == 0.0f) {
-    if (n.x == 1.0f) return P.x >= c.x + m;
-    if (n.x == -1.0f) return P.x <= c.x - m;
-  } else if (n.x == 0.0f && n.z == 0.0f) {
-    if (n.y == 1.0f) return P.y >= c.y + m;
-    if (n.y == -1.0f) return P.y <= c.y - m;
-  } else if (n.x == 0.0f && n.y == 0.0f) {
-    if (n.z == 1.0f) return P.z >= c.z + m;
-    if (n.z == -1.0f) return P.z <= c.z - m;
-  }
-  return false;
-}
-
 struct LS {
   bool ok;      // the sample is valid before the shadow test
   bool ray;     // a shadow ray would be traced
@@ -414,6 +358,40 @@ struct LS {
   float G;
 };
 
+// The cube light of sample_lights (light.glsl:329-367) once the light is
+// neither the shaded voxel itself nor behind the surface.  na, ns: the
+// normal's axis (normal_axis).
+CT_D void sample_cube_light(const Hit &hit, int na, float ns, const PLight &l, float &pdf, uint32_t &seed,
+                            bool calc_pdf, bool visibility, LS &o) {
+  const F3 P = hit.P;
+  uint32_t face;
+  F3 l_pos;
+  const bool vis = draw_cube_point(P, hit.n, na, ns, l.pos, l.size * 0.5f, seed, face, l_pos);
+  const F3 l_wi = normalize(sub(P, l_pos));
+  l_pos = face_ray_origin(face_ray_origin(l_pos, face), face);
+  // length(P - l_pos), geom_fact_sa(P, l_pos, l_nor) and the shading
+  // direction share one square root: P - l_pos is exactly -(l_pos - P),
+  // and for the axis vector l_nor, dot(l_nor, dir) is the component of
+  // dir on that axis up to sign (the other terms are signed zeros).
+  const F3 dd = sub(l_pos, P);
+  const float d2 = dot(dd, dd);
+  o.dist = sqrtf(d2);
+  o.wi = divs(dd, o.dist);
+  if (calc_pdf) {
+    float area = l.size * l.size * 6.0f;
+    pdf /= area;
+  }
+  o.G = fabsf(component(o.wi, (int)(face >> 1))) / d2;
+  o.ray = visibility && vis;
+  o.P = P;
+  o.dir = neg(l_wi);
+  o.ti = l.inst;
+  o.tp = l.prim;
+  o.l_pos = l_pos;
+  o.Le = l.emissive;
+  o.ok = vis;
+}
+
 // sample_lights, light.glsl:295-399, without the shadow ray.
 CT_D void sample_lights(const DFrame &F, const Hit &hit, const PLight &l, float &pdf, uint32_t &seed, bool calc_pdf,
                         bool visibility, LS &o) {
@@ -422,66 +400,19 @@ CT_D void sample_lights(const DFrame &F, const Hit &hit, const PLight &l, float 
   F3 P = hit.P, n = hit.n;
   float distance = -1.0f;
   F3 l_wi = f3(0, 0, 0), l_pos = f3(0, 0, 0), l_nor = f3(0, 0, 0);
-  bool vis = true, check = false;
   F3 em = l.emissive;
   if (l.type == CT_LIGHT_CUBE) {
-    float half = l.size * 0.5f, qs = l.size;
-    if (light_behind_surface(P, n, l.pos, half)) {
+    float ns;
+    const int na = normal_axis(n, ns);
+    if (light_behind_surface(P, na, ns, l.pos, l.size * 0.5f)) {
       // Every one of the 11 draws fails the "in front of the surface" test,
       // so the result is a failed sample (its G and pdf only ever multiply
       // a zero contribution) after 11 x 3 = 33 LCG steps.
-      seed = lcg_skip33(seed);
+      seed = lcg_skip<33>(seed);
       return;
     }
-    // light.glsl:333-345.  The face normal is an axis vector, so
-    // random_quad's tangents are the exact axis vectors t1, t2 (their
-    // normalize divides by 1), and dot(normalize(P - x), axis) has the sign
-    // of (P - x) on that axis: the draw is tested by signs and only the
-    // last one is normalized.  A normal n off the axes takes the full test.
-    int na = -1;
-    float ns = 0.0f;
-    if (n.y == 0.0f && n.z == 0.0f && fabsf(n.x) == 1.0f) { na = 0; ns = n.x; }
-    else if (n.x == 0.0f && n.z == 0.0f && fabsf(n.y) == 1.0f) { na = 1; ns = n.y; }
-    else if (n.x == 0.0f && n.y == 0.0f && fabsf(n.z) == 1.0f) { na = 2; ns = n.z; }
-    const float hq = qs * 0.5f;
-    uint32_t i = 0;
-    do {
-      l_nor = random_cube_normal(seed);
-      l_pos = add(l.pos, muls(l_nor, half));
-      const float u = rnd(seed);
-      const float v = rnd(seed);
-      const float qx = u * hq, qy = v * hq;
-      const F3 t1 = fabsf(l_nor.x) > fabsf(l_nor.y) ? f3(-l_nor.z, 0.0f, l_nor.x) : f3(0.0f, l_nor.z, -l_nor.y);
-      const F3 t2 = cross(l_nor, t1);
-      l_pos = add(add(l_pos, muls(t1, qx)), muls(t2, qy));
-      const F3 w = sub(P, l_pos);
-      const float wn = l_nor.x != 0.0f ? w.x * l_nor.x : (l_nor.y != 0.0f ? w.y * l_nor.y : w.z * l_nor.z);
-      vis = wn > 0.0f;
-      if (vis) {
-        if (na >= 0) {
-          vis = (na == 0 ? w.x : (na == 1 ? w.y : w.z)) * ns < 0.0f;
-        } else {
-          vis = dot(normalize(w), n) < 0.0f;
-        }
-      }
-    } while (!vis && i++ < 10);
-    l_wi = normalize(sub(P, l_pos));
-    l_pos = compute_ray_origin(l_pos, l_nor);
-    l_pos = compute_ray_origin(l_pos, l_nor);
-    // length(P - l_pos), geom_fact_sa(P, l_pos, l_nor) and the shading
-    // direction share one square root: P - l_pos is exactly -(l_pos - P),
-    // and for the axis vector l_nor, dot(l_nor, dir) is the component of
-    // dir on that axis up to sign (the other terms are signed zeros).
-    const F3 dd = sub(l_pos, P);
-    const float d2 = dot(dd, dd);
-    distance = sqrtf(d2);
-    o.wi = divs(dd, distance);
-    if (calc_pdf) {
-      float area = qs * qs * 6.0f;
-      pdf /= area;
-    }
-    check = true;
-    o.G = fabsf(l_nor.x != 0.0f ? o.wi.x : (l_nor.y != 0.0f ? o.wi.y : o.wi.z)) / d2;
+    sample_cube_light(hit, na, ns, l, pdf, seed, calc_pdf, visibility, o);
+    return;
   } else if (l.type == CT_LIGHT_POINT) {
     // As above: normalize(l_pos - P) is exactly -normalize(P - l_pos).
     l_pos = l.pos;
@@ -502,16 +433,16 @@ CT_D void sample_lights(const DFrame &F, const Hit &hit, const PLight &l, float 
     if (calc_pdf) pdf /= kInv4Pi;
     o.G = 1.0f;
   }
-  if (l.type != CT_LIGHT_CUBE && l.type != CT_LIGHT_POINT) o.wi = normalize(sub(l_pos, P));
-  o.ray = visibility && vis;
+  if (l.type != CT_LIGHT_POINT) o.wi = normalize(sub(l_pos, P));
+  o.ray = visibility;
   o.P = P;
   o.dir = neg(l_wi);
   o.dist = distance;
-  o.ti = check ? l.inst : kInvalid;
-  o.tp = check ? l.prim : kInvalid;
+  o.ti = kInvalid;
+  o.tp = kInvalid;
   o.l_pos = l_pos;
   o.Le = em;
-  o.ok = vis;
+  o.ok = true;
 }
 
 // calculate_sampled_light, light.glsl:401-435.  With use_vis the shadow
@@ -2058,6 +1989,12 @@ int prepare_frame(Ctx *c, Accel *a, const ct_frame_params *p, hipStream_t st, DF
     CT_HIP(hipStreamSynchronize(st));  // earlier frames may still read the old table
     std::vector<float4> pk;
     pack_lights(a->cube_lights_host.data(), ncube, pk);
+    c->cube_plain = true;
+    for (uint32_t i = 0; i < ncube; ++i) {
+      const ct_light &l = a->cube_lights_host[i];
+      c->cube_plain = c->cube_plain && l.type == CT_LIGHT_CUBE &&
+                      !(l.emissive[0] <= 0.0f && l.emissive[1] <= 0.0f && l.emissive[2] <= 0.0f);
+    }
     if ((rc = cube.reserve(16 * pk.size()))) return rc;
     CT_HIP(hipMemcpy(cube.p, pk.data(), 16 * pk.size(), hipMemcpyHostToDevice));
     c->lights_accel = a;
@@ -2070,6 +2007,7 @@ int prepare_frame(Ctx *c, Accel *a, const ct_frame_params *p, hipStream_t st, DF
   F.frame = p->frame_number; F.active = p->is_active; F.afternoon = p->is_afternoon; F.time = p->time;
   F.n_cube = ncube; F.n_point = (uint32_t)c->point_host.size(); F.n_env = (uint32_t)c->env_host.size();
   F.n_mats = (uint32_t)c->mats_host.size();
+  F.cube_plain = c->cube_plain ? 1u : 0u;
   std::memcpy(F.inv_view, p->inv_view, sizeof(F.inv_view));
   std::memcpy(F.inv_proj, p->inv_proj, sizeof(F.inv_proj));
   F.rp = p->restir;
