@@ -769,7 +769,7 @@ __global__ void __launch_bounds__(64) k_grid_link(DGrid g, uint4 *bricks, uint32
 }
 
 __global__ void __launch_bounds__(kBlock) k_grid_ids(SegView sv, const uint32_t *inst, const uint4 *bricks,
-                                                     const uint32_t *cells, uint2 *ids) {
+                                                     const uint32_t *cells, uint2 *ids, uint32_t *slots) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= sv.n) return;
   const uint32_t s = find_seg(sv.off, sv.nseg, k), p = k - sv.off[s], c = cells[sv.base[s] + p];
@@ -777,7 +777,10 @@ __global__ void __launch_bounds__(kBlock) k_grid_ids(SegView sv, const uint32_t 
   const uint4 e = bricks[c >> 6];
   const unsigned long long m = ((unsigned long long)e.y << 32) | e.x;
   const uint32_t i = e.z + (uint32_t)__popcll(m & ((1ull << (c & 63u)) - 1ull));
-  if (i < sv.n) ids[i] = make_uint2(inst[s], p);
+  if (i < sv.n) {
+    ids[i] = make_uint2(inst[s], p);
+    slots[i] = sv.base[s] + p;
+  }
 }
 
 // Builds the scene's cell grid (DGrid) when it can have one: every instance
@@ -824,6 +827,7 @@ int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::
     for (int r = 0; r < 3; ++r) g.w2o[c * 3 + r] = w[c * 4 + r];
   int rc;
   if ((rc = S.grid_bricks.reserve(16 * (size_t)nrec)) || (rc = S.grid_ids.reserve(8 * (size_t)n)) ||
+      (rc = S.grid_slots.reserve(4 * (size_t)n)) ||
       (rc = S.grid_cells.reserve(4 * (size_t)S.prim_capacity)) || (rc = S.grid_work.reserve(8 + 4 * seg.size())))
     return rc;
   uint32_t *work = S.grid_work.as<uint32_t>(), *d_seg = work + 2;
@@ -835,11 +839,12 @@ int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::
                      S.grid_bricks.as<uint32_t>(), S.grid_cells.as<uint32_t>(), work);
   hipLaunchKernelGGL(k_grid_link, dim3((uint32_t)nblk), dim3(64), 0, st, g, bricks, work);
   hipLaunchKernelGGL(k_grid_ids, dim3(blocks(n)), dim3(kBlock), 0, st, sv, d_seg + 2 * nseg + 1, bricks,
-                     S.grid_cells.as<uint32_t>(), S.grid_ids.as<uint2>());
+                     S.grid_cells.as<uint32_t>(), S.grid_ids.as<uint2>(), S.grid_slots.as<uint32_t>());
   CT_HIP(hipGetLastError());
   CT_HIP(hipMemcpyAsync(&flags, work, 4, hipMemcpyDeviceToHost, st));
   g.bricks = bricks;
   g.ids = S.grid_ids.as<uint2>();
+  g.slots = S.grid_slots.as<uint32_t>();
   g.cells = S.grid_cells.as<uint32_t>();
   S.grid = g;
   return CT_OK;

@@ -26,6 +26,10 @@ namespace {
 
 constexpr int kBlockA = 256;
 constexpr float kFar = 1e9f;  // MAX_DISTANCE, defines.glsl:30
+// Lanes that wait before a wave shades (walk_stream).  Forward and backward
+// at 512^2, 16 samples: 16.2 ms with 32, 15.9 with 40, 15.8 with 48 to 56, and
+// more below 32; path tracing at 1080p 520, 505, 508, 520 us.
+constexpr int kAdjWait = 48;
 
 struct AView {
   uint32_t width, height, base;  // base: global index of the view's first pixel
@@ -38,12 +42,13 @@ struct AArgs {
   const ct_aabb *aabbs;
   const AView *views;
   const uint2 *blocks;  // per block: (view, first pixel of the view)
+  uint32_t per_lane;    // pixels per lane of a block
   uint32_t spp, max_depth, seed;
   const float *albedo;
   const float *emission;
 };
 
-struct Vertex {
+struct alignas(16) Vertex {
   uint32_t g;  // primitive slot
   F3 beta;     // throughput arriving at the vertex
 };
@@ -65,17 +70,16 @@ CT_D void view_ray(const AView &V, uint32_t x, uint32_t y, uint32_t &seed, F3 &o
   d = f3(d4[0], d4[1], d4[2]);
 }
 
-// Closest voxel of the segment from `origin` along `dir` (intersect()):
-// returns the slot and the world hit position and normal.
-template <int kWalk>
-CT_D bool segment(const AArgs &A, F3 origin, F3 dir, uint32_t *stk, uint32_t &g, F3 &pos, F3 &nrm) {
-  const F3 ro = compute_ray_origin(origin, dir);
-  float bt = kFar;
-  uint32_t bi = kInvalid, bp = kInvalid;
-  bool ovf = false;
-  TraceCnt cnt;
-  traverse_mode<kTraceBounce, kWalk>(A.S, ro, dir, kFar, kInvalid, kInvalid, bt, bi, bp, stk, kBlockA, cnt, ovf);
-  if (bi == kInvalid) return false;
+// transpose(world2obj) * vec4(n, 0) for the 3-row packing.
+CT_D F3 world_normal(const float *w, F3 n) {
+  return f3(((w[0] * n.x + w[1] * n.y) + w[2] * n.z) + 0.0f * 0.0f,
+            ((w[3] * n.x + w[4] * n.y) + w[5] * n.z) + 0.0f * 0.0f,
+            ((w[6] * n.x + w[7] * n.y) + w[8] * n.z) + 0.0f * 0.0f);
+}
+// The slot and the world hit position and normal of the segment's closest
+// voxel (bi, bp); the segment is tested from ro = compute_ray_origin(origin,
+// dir), as intersect() does.
+CT_D void segment_hit(const AArgs &A, F3 ro, F3 dir, uint32_t bi, uint32_t bp, uint32_t &g, F3 &pos, F3 &nrm) {
   const DInst &I = A.S.inst[bi];
   float w[12];
 #pragma unroll
@@ -91,85 +95,202 @@ CT_D bool segment(const AArgs &A, F3 origin, F3 dir, uint32_t *stk, uint32_t &g,
   F3 on;
   intersect_box<true, false>(c, oo, od, sg, sinv, t, &on);
   pos = add(ro, muls(dir, t));
-  nrm = f3(((w[0] * on.x + w[1] * on.y) + w[2] * on.z) + 0.0f * 0.0f,
-           ((w[3] * on.x + w[4] * on.y) + w[5] * on.z) + 0.0f * 0.0f,
-           ((w[6] * on.x + w[7] * on.y) + w[8] * on.z) + 0.0f * 0.0f);
-  return true;
+  nrm = world_normal(w, on);
 }
 
 CT_D F3 albedo_of(const AArgs &A, uint32_t g) {
   return f3(A.albedo[3 * (size_t)g], A.albedo[3 * (size_t)g + 1], A.albedo[3 * (size_t)g + 2]);
 }
 
-// Traces one sample; fills the vertices (when `path` is given) and returns
-// the sample's radiance.
+// A lane's path: its pixel, the sample of the pixel, and the segment to trace
+// next (from `o` along `d`, the k-th of the sample).
+struct Path {
+  uint32_t p, gpix, pixel_seed, s, k, seed;
+  F3 o, d, beta, L, sum;  // throughput and radiance of the sample, sum over samples
+  bool more;              // the sample goes on
+};
+
+CT_D void start_sample(const AArgs &A, const AView &V, Path &P) {
+  P.seed = tea(P.pixel_seed, P.s);
+  view_ray(V, P.p % V.width, P.p / V.width, P.seed, P.o, P.d);
+  P.beta = f3(1.0f, 1.0f, 1.0f);
+  P.L = f3(0.0f, 0.0f, 0.0f);
+  P.k = 0u;
+  P.more = true;
+}
+// Closest voxel of the path's segment: its slot, world hit position and
+// normal.
 template <int kWalk>
-CT_D F3 trace_sample(const AArgs &A, const AView &V, uint32_t x, uint32_t y, uint32_t seed, uint32_t *stk,
-                     Vertex *path, uint32_t &nv) {
-  F3 o, d;
-  view_ray(V, x, y, seed, o, d);
-  F3 beta = f3(1.0f, 1.0f, 1.0f), L = f3(0.0f, 0.0f, 0.0f);
-  nv = 0;
-  for (uint32_t k = 0; k <= A.max_depth; ++k) {
-    uint32_t g;
-    F3 pos, nrm;
-    if (!segment<kWalk>(A, o, d, stk, g, pos, nrm)) break;
-    if (path) {
-      path[k].g = g;
-      path[k].beta = beta;
-    }
-    nv = k + 1;
-    L = add(L, muls(beta, A.emission[g]));
-    if (k == A.max_depth) break;
-    beta = mulv(beta, albedo_of(A, g));
-    F3 sd = random_cosine_direction(seed, nrm);
-    if (normal_near_zero(sd)) sd = nrm;
-    d = sd;
-    o = compute_ray_origin(compute_ray_origin(pos, nrm), nrm);
+CT_D bool segment(const AArgs &A, const Path &P, uint32_t *stk, uint32_t &g, F3 &pos, F3 &nrm) {
+  const F3 ro = compute_ray_origin(P.o, P.d);
+  if constexpr (kWalk == kWalkGrid) {
+    GridWalk<kTraceBounce> w{A.S.grid};
+    w.start(A.S, ro, P.d, kFar, kInvalid, kInvalid);
+    w.run();
+    if (w.best == kInvalid) return false;
+    // the walk's box test is segment_hit's
+    g = gld(A.S.grid.slots + w.best);
+    pos = add(ro, muls(P.d, w.best_t));
+    nrm = world_normal(A.S.grid.w2o, w.best_n);
+    return true;
+  } else {
+    float bt = kFar;
+    uint32_t bi = kInvalid, bp = kInvalid;
+    bool ovf = false;
+    TraceCnt cnt;
+    traverse_mode<kTraceBounce, kWalk>(A.S, ro, P.d, kFar, kInvalid, kInvalid, bt, bi, bp, stk, kBlockA, cnt, ovf);
+    if (bi == kInvalid) return false;
+    segment_hit(A, ro, P.d, bi, bp, g, pos, nrm);
+    return true;
   }
-  return L;
 }
 
-CT_D uint32_t sample_seed(uint32_t gpix, uint32_t seed, uint32_t s) { return tea(tea(gpix, seed), s); }
+// Traces every path of the wave's A.per_lane * 64 pixels.  A lane that has
+// ended its path starts the next sample of its pixel, or takes the next pixel
+// of the wave, at once: paths of a wave have 1 to max_depth + 1 segments of 1
+// to 20 steps, and a wave that waits for its longest runs at 31% of its lanes
+// (with this 44%).  The samples of a pixel stay in order on one lane, so the
+// image is the same whatever the schedule.  hit(path, g, pos, nrm) shades a
+// vertex and returns whether the path goes on from path.o along path.d;
+// end(path) takes a finished sample (path.s, from 1 up to spp).
+//
+// Measured with the walk's new step loop: forward of 8 views at 512^2 with 16
+// samples 8.9 -> 6.3 ms, path tracing at 1080p with 1 sample 448 -> 400 us.
+template <int kWalk, class Hit, class End>
+CT_D void trace_paths(const AArgs &A, Hit hit, End end) {
+  __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
+  __shared__ uint32_t taken[kBlockA / 64];
+  if (threadIdx.x < kBlockA / 64) taken[threadIdx.x] = 0u;
+  __syncthreads();
+  const uint2 b = A.blocks[blockIdx.x];
+  const AView &V = *as_constant(A.views + b.x);
+  const uint32_t wave = threadIdx.x >> 6, first = b.y + wave * (64u * A.per_lane),
+                 last = min(first + 64u * A.per_lane, V.width * V.height);
+  Path P;
+  P.s = A.spp;
+  P.more = false;
+  F3 ro;
+  auto next = [&]() -> bool {
+    if (!P.more) {
+      if (P.s == A.spp) {
+        P.p = first + atomicAdd(&taken[wave], 1u);
+        if (P.p >= last) return false;
+        P.gpix = V.base + P.p;
+        P.pixel_seed = tea(P.gpix, A.seed);
+        P.s = 0u;
+        P.sum = f3(0, 0, 0);
+      }
+      start_sample(A, V, P);
+    }
+    ro = compute_ray_origin(P.o, P.d);
+    return true;
+  };
+  auto done = [&](bool found, uint32_t g, F3 pos, F3 nrm) {
+    P.more = found && hit(P, g, pos, nrm);
+    if (!P.more) {
+      P.sum = add(P.sum, P.L);
+      ++P.s;
+      end(P);
+    }
+  };
+  if constexpr (kWalk == kWalkGrid) {
+    GridWalk<kTraceBounce> w{A.S.grid};
+    walk_stream<kTraceBounce, kAdjWait>(
+        w,
+        [&]() -> bool {
+          if (!next()) return false;
+          w.start(A.S, ro, P.d, kFar, kInvalid, kInvalid);
+          return true;
+        },
+        [&]() {
+          // the walk's box test is segment_hit's
+          const bool found = w.best != kInvalid;
+          done(found, found ? gld(A.S.grid.slots + w.best) : 0u, add(ro, muls(P.d, w.best_t)),
+               world_normal(A.S.grid.w2o, w.best_n));
+        });
+  } else {
+    while (next()) {
+      uint32_t g = 0u;
+      F3 pos = f3(0, 0, 0), nrm = f3(0, 0, 0);
+      const bool found = segment<kWalk>(A, P, stk + threadIdx.x, g, pos, nrm);
+      done(found, g, pos, nrm);
+    }
+  }
+}
+
+// Lambertian scatter of a path at a vertex.
+CT_D void scatter(Path &P, F3 pos, F3 nrm) {
+  F3 sd = random_cosine_direction(P.seed, nrm);
+  if (normal_near_zero(sd)) sd = nrm;
+  P.d = sd;
+  P.o = compute_ray_origin(compute_ray_origin(pos, nrm), nrm);
+  ++P.k;
+}
+
+CT_D void store_pixel(const AArgs &A, const Path &P, float *image) {
+  const F3 I = divs(P.sum, (float)A.spp);
+  image[3 * (size_t)P.gpix] = I.x;
+  image[3 * (size_t)P.gpix + 1] = I.y;
+  image[3 * (size_t)P.gpix + 2] = I.z;
+}
 
 template <int kWalk>
 __global__ void __launch_bounds__(kBlockA) k_adj_forward(AArgs A, float *image) {
-  __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
-  const uint2 b = A.blocks[blockIdx.x];
-  const AView &V = A.views[b.x];
-  const uint32_t p = b.y + threadIdx.x;
-  if (p >= V.width * V.height) return;
-  const uint32_t x = p % V.width, y = p / V.width, gpix = V.base + p;
-  F3 sum = f3(0, 0, 0);
-  uint32_t nv;
-  for (uint32_t s = 0; s < A.spp; ++s)
-    sum = add(sum, trace_sample<kWalk>(A, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x, nullptr, nv));
-  const F3 I = divs(sum, (float)A.spp);
-  image[3 * (size_t)gpix] = I.x;
-  image[3 * (size_t)gpix + 1] = I.y;
-  image[3 * (size_t)gpix + 2] = I.z;
+  trace_paths<kWalk>(
+      A,
+      [&](Path &P, uint32_t g, F3 pos, F3 nrm) -> bool {
+        P.L = add(P.L, muls(P.beta, A.emission[g]));
+        if (P.k == A.max_depth) return false;
+        P.beta = mulv(P.beta, albedo_of(A, g));
+        scatter(P, pos, nrm);
+        return true;
+      },
+      [&](Path &P) {
+        if (P.s == A.spp) store_pixel(A, P, image);
+      });
 }
 
 template <int kWalk>
 __global__ void __launch_bounds__(kBlockA) k_adj_backward(AArgs A, const float *grad_image, float *grad_albedo,
                                                           float *grad_emission) {
+  // The path's vertices, max_depth + 1 per lane, vertex by vertex.
+  extern __shared__ Vertex vertices[];
   __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
+  Vertex *path = vertices + threadIdx.x;
   const uint2 b = A.blocks[blockIdx.x];
-  const AView &V = A.views[b.x];
-  const uint32_t p = b.y + threadIdx.x;
-  if (p >= V.width * V.height) return;
-  const uint32_t x = p % V.width, y = p / V.width, gpix = V.base + p;
+  const AView &V = *as_constant(A.views + b.x);
+  Path P;
+  P.p = b.y + threadIdx.x;
+  if (P.p >= V.width * V.height) return;
+  P.gpix = V.base + P.p;
+  P.pixel_seed = tea(P.gpix, A.seed);
   const float inv = 1.0f / (float)A.spp;
-  const F3 G = f3(grad_image[3 * (size_t)gpix] * inv, grad_image[3 * (size_t)gpix + 1] * inv,
-                  grad_image[3 * (size_t)gpix + 2] * inv);
-  Vertex path[CT_ADJOINT_MAX_DEPTH + 1];
-  for (uint32_t s = 0; s < A.spp; ++s) {
-    uint32_t nv;
-    trace_sample<kWalk>(A, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x, path, nv);
+  const F3 G = f3(grad_image[3 * (size_t)P.gpix] * inv, grad_image[3 * (size_t)P.gpix + 1] * inv,
+                  grad_image[3 * (size_t)P.gpix + 2] * inv);
+  // One sample of every lane at a time (not trace_paths): a voxel of a small
+  // scene sums tens of thousands of terms in 32 bits, whose rounding follows
+  // the order they come in; this keeps to samples before pixels.
+  for (P.s = 0; P.s < A.spp; ++P.s) {
+    uint32_t nv = 0;
+    start_sample(A, V, P);
+    while (P.more) {
+      uint32_t g = 0u;
+      F3 pos, nrm;
+      P.more = segment<kWalk>(A, P, stk + threadIdx.x, g, pos, nrm);
+      if (!P.more) break;
+      path[P.k * kBlockA] = Vertex{g, P.beta};
+      nv = P.k + 1u;
+      P.more = P.k < A.max_depth;
+      if (P.more) {
+        P.beta = mulv(P.beta, albedo_of(A, g));
+        scatter(P, pos, nrm);
+      }
+    }
     F3 S = f3(0, 0, 0);  // radiance from the vertices after k, relative to vertex k+1
     for (int k = (int)nv - 1; k >= 0; --k) {
-      const uint32_t g = path[k].g;
-      const F3 bk = path[k].beta;
+      const Vertex v = path[k * kBlockA];
+      const uint32_t g = v.g;
+      const F3 bk = v.beta;
       const float e = A.emission[g];
       atomicAdd(&grad_emission[g], dot(G, bk));
       if ((uint32_t)k < A.max_depth) {
@@ -286,55 +407,45 @@ CT_D bool scatter_material(const PMat &m, F3 dir, F3 nrm, uint32_t &seed, F3 &sd
 }
 
 template <int kWalk>
-CT_D F3 path_sample(const PArgs &P, const AView &V, uint32_t x, uint32_t y, uint32_t seed, uint32_t *stk) {
-  const AArgs &A = P.A;
-  F3 o, d;
-  view_ray(V, x, y, seed, o, d);
-  F3 beta = f3(1.0f, 1.0f, 1.0f), L = f3(0.0f, 0.0f, 0.0f);
-  for (uint32_t k = 0; k <= A.max_depth; ++k) {
-    uint32_t g;
-    F3 pos, nrm;
-    if (!segment<kWalk>(A, o, d, stk, g, pos, nrm)) break;
-    const uint32_t mi = P.prims[g].material_index;
-    if (mi >= P.n_mats) break;  // no material: absorbs
-    const PMat m = P.mats[mi];
-    L = add(L, mulv(beta, f3(m.emission_ior.x, m.emission_ior.y, m.emission_ior.z)));
-    if (k == A.max_depth) break;
-    F3 sd, att;
-    if (!scatter_material(m, d, nrm, seed, sd, att)) break;
-    beta = mulv(beta, att);
-    const uint32_t type = __float_as_uint(m.diffuse_type.w) & CT_MATERIAL_TYPE_MASK;
-    const F3 side = (type == 0u || dot(sd, nrm) >= 0.0f) ? nrm : neg(nrm);
-    d = sd;
-    o = compute_ray_origin(compute_ray_origin(pos, side), side);
-  }
-  return L;
+__global__ void __launch_bounds__(kBlockA) k_path_trace(PArgs Q, float *image) {
+  const AArgs &A = Q.A;
+  trace_paths<kWalk>(
+      A,
+      [&](Path &P, uint32_t g, F3 pos, F3 nrm) -> bool {
+        const uint32_t mi = Q.prims[g].material_index;
+        if (mi >= Q.n_mats) return false;  // no material: absorbs
+        const PMat m = Q.mats[mi];
+        P.L = add(P.L, mulv(P.beta, f3(m.emission_ior.x, m.emission_ior.y, m.emission_ior.z)));
+        if (P.k == A.max_depth) return false;
+        F3 sd, att;
+        if (!scatter_material(m, P.d, nrm, P.seed, sd, att)) return false;
+        P.beta = mulv(P.beta, att);
+        const uint32_t type = __float_as_uint(m.diffuse_type.w) & CT_MATERIAL_TYPE_MASK;
+        const F3 side = (type == 0u || dot(sd, nrm) >= 0.0f) ? nrm : neg(nrm);
+        P.d = sd;
+        P.o = compute_ray_origin(compute_ray_origin(pos, side), side);
+        ++P.k;
+        return true;
+      },
+      [&](Path &P) {
+        if (P.s == A.spp) store_pixel(A, P, image);
+      });
 }
 
-template <int kWalk>
-__global__ void __launch_bounds__(kBlockA) k_path_trace(PArgs P, float *image) {
-  __shared__ uint32_t stk[kWalk == kWalkGrid ? 1 : (kStackLds > 0 ? kStackLds : 1) * kBlockA];
-  const AArgs &A = P.A;
-  const uint2 b = A.blocks[blockIdx.x];
-  const AView &V = A.views[b.x];
-  const uint32_t p = b.y + threadIdx.x;
-  if (p >= V.width * V.height) return;
-  const uint32_t x = p % V.width, y = p / V.width, gpix = V.base + p;
-  F3 sum = f3(0, 0, 0);
-  for (uint32_t s = 0; s < A.spp; ++s) sum = add(sum, path_sample<kWalk>(P, V, x, y, sample_seed(gpix, A.seed, s), stk + threadIdx.x));
-  const F3 I = divs(sum, (float)A.spp);
-  image[3 * (size_t)gpix] = I.x;
-  image[3 * (size_t)gpix + 1] = I.y;
-  image[3 * (size_t)gpix + 2] = I.z;
-}
-
-int plan(Accel &a, const ct_adjoint_desc *d, const ct_adjoint_view *views, hipStream_t st, AdjPlan &P, AArgs &A) {
+// `stream`: the kernel takes per_lane pixels a lane (trace_paths).
+int plan(Accel &a, const ct_adjoint_desc *d, const ct_adjoint_view *views, bool stream, hipStream_t st, AdjPlan &P,
+         AArgs &A) {
   if (!d || !views || d->n_views == 0) return fail(CT_E_INVALID, "adjoint: no views");
   if (d->spp == 0 || d->max_depth > CT_ADJOINT_MAX_DEPTH) return fail(CT_E_INVALID, "adjoint: spp 0 or max_depth too large");
   if (a.set.tlas_count == 0) return fail(CT_E_STATE, "adjoint: empty scene");
   std::vector<AView> hv(d->n_views);
   std::vector<uint2> hb;
-  uint64_t base = 0;
+  uint64_t base = 0, total = 0;
+  for (uint32_t v = 0; v < d->n_views; ++v) total += (uint64_t)views[v].width * views[v].height;
+  // One lane takes several pixels where that leaves every SIMD 8 waves (256
+  // CUs of 4 SIMDs): a wave then refills from 64 * per_lane paths.
+  A.per_lane = stream ? (uint32_t)std::min<uint64_t>(std::max<uint64_t>(total / (64u * 8u * 1024u), 1u), 8u) : 1u;
+  const uint64_t run = (uint64_t)kBlockA * A.per_lane;
   for (uint32_t v = 0; v < d->n_views; ++v) {
     const ct_adjoint_view &cv = views[v];
     if (cv.width == 0 || cv.height == 0) return fail(CT_E_INVALID, "adjoint: empty view");
@@ -346,7 +457,7 @@ int plan(Accel &a, const ct_adjoint_desc *d, const ct_adjoint_view *views, hipSt
     std::memcpy(V.inv_view, cv.inv_view, sizeof(V.inv_view));
     std::memcpy(V.inv_proj, cv.inv_proj, sizeof(V.inv_proj));
     const uint64_t np = (uint64_t)cv.width * cv.height;
-    for (uint64_t p = 0; p < np; p += kBlockA) hb.push_back(make_uint2(v, (uint32_t)p));
+    for (uint64_t p = 0; p < np; p += run) hb.push_back(make_uint2(v, (uint32_t)p));
     base += np;
     if (base >= (1ull << 31)) return fail(CT_E_INVALID, "adjoint: too many pixels");
   }
@@ -380,7 +491,7 @@ int ct_adjoint_render(ct_accel *a, const ct_adjoint_desc *d, const ct_adjoint_vi
   AdjPlan P;
   AArgs A;
   int rc;
-  if ((rc = plan(*a, d, views, st, P, A))) return rc;
+  if ((rc = plan(*a, d, views, true, st, P, A))) return rc;
   A.albedo = albedo;
   A.emission = emission;
   if (A.S.grid.bricks)
@@ -402,7 +513,7 @@ int ct_path_trace(ct_accel *a, const ct_adjoint_desc *d, const ct_adjoint_view *
   AdjPlan P;
   PArgs PA;
   int rc;
-  if ((rc = plan(*a, d, views, st, P, PA.A))) return rc;
+  if ((rc = plan(*a, d, views, true, st, P, PA.A))) return rc;
   if (materials) {  // pack and keep them for later calls with materials == NULL
     std::vector<PMat> pm(std::max<uint32_t>(material_count, 1));
     for (uint32_t i = 0; i < material_count; ++i) {
@@ -443,14 +554,15 @@ int ct_adjoint_backward(ct_accel *a, const ct_adjoint_desc *d, const ct_adjoint_
   AdjPlan P;
   AArgs A;
   int rc;
-  if ((rc = plan(*a, d, views, st, P, A))) return rc;
+  if ((rc = plan(*a, d, views, false, st, P, A))) return rc;
   A.albedo = albedo;
   A.emission = emission;
+  const size_t lds = sizeof(Vertex) * kBlockA * (size_t)(A.max_depth + 1);
   if (A.S.grid.bricks)
-    hipLaunchKernelGGL(k_adj_backward<kWalkGrid>, dim3(P.nblocks), dim3(kBlockA), 0, st, A, grad_image, grad_albedo,
+    hipLaunchKernelGGL(k_adj_backward<kWalkGrid>, dim3(P.nblocks), dim3(kBlockA), lds, st, A, grad_image, grad_albedo,
                        grad_emission);
   else
-    hipLaunchKernelGGL(k_adj_backward<kWalkBvh>, dim3(P.nblocks), dim3(kBlockA), 0, st, A, grad_image, grad_albedo,
+    hipLaunchKernelGGL(k_adj_backward<kWalkBvh>, dim3(P.nblocks), dim3(kBlockA), lds, st, A, grad_image, grad_albedo,
                        grad_emission);
   CT_HIP(hipGetLastError());
   CT_HIP(hipStreamSynchronize(st));

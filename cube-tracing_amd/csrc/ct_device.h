@@ -31,6 +31,12 @@ CT_D F3 neg(F3 a) { return f3(-a.x, -a.y, -a.z); }
 CT_D float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 CT_D float length(F3 a) { return sqrtf(dot(a, a)); }
 CT_D F3 normalize(F3 a) { return divs(a, length(a)); }
+// normalize of what is mostly an axis vector already: its length is 1, and
+// the square root and the divisions by 1 (45 instructions) are left out.
+CT_D F3 normalize_axis(F3 a) {
+  const float d = dot(a, a);
+  return d == 1.0f ? a : divs(a, sqrtf(d));
+}
 CT_D F3 cross(F3 a, F3 b) {
   return f3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
 }
@@ -43,7 +49,22 @@ CT_D F3 mix3(F3 x, F3 y, float a) { return f3(mixf(x.x, y.x, a), mixf(x.y, y.y, 
 CT_D float gsign(float x) { return x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f); }
 CT_D F3 xyz(float4 v) { return f3(v.x, v.y, v.z); }
 
-// Saturating conversions (NaN -> 0).
+// Saturating conversions (NaN -> 0), which the hardware's are (a C++ cast
+// leaves values out of range undefined, and guarding it takes 8 instructions;
+// compute_ray_origin converts three values, and each pass calls it 2 to 6
+// times a pixel).
+#if defined(__HIP_DEVICE_COMPILE__)
+CT_D uint32_t f2u_sat(float x) {
+  uint32_t r;
+  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+CT_D int32_t f2i_sat(float x) {
+  int32_t r;
+  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+  return r;
+}
+#else
 CT_D uint32_t f2u_sat(float x) {
   if (!(x > 0.0f)) return 0u;
   if (x >= 4294967296.0f) return 0xFFFFFFFFu;
@@ -54,6 +75,14 @@ CT_D int32_t f2i_sat(float x) {
   if (x >= 2147483648.0f) return 0x7FFFFFFF;
   if (x <= -2147483648.0f) return (int32_t)0x80000000;
   return (int32_t)x;
+}
+#endif
+
+// Memory that no kernel of the launch writes, as constant memory: uniform
+// reads of it are then scalar loads, also after stores and inside loops.
+template <class T>
+CT_D const T *as_constant(const T *p) {
+  return (const T *)(const __attribute__((address_space(4))) T *)p;
 }
 
 // Column-major 4x4 (m[c*4 + r]): out_r = ((m0r*v0 + m1r*v1) + m2r*v2) + m3r*v3.
@@ -121,10 +150,12 @@ CT_D F3 mul_rot(F3 v) {
 // primitives.glsl:273-355 with rotation = identity and radius = h on all
 // axes.  `dr` is the (rotated) direction and `sg` = -sign(dr), both
 // independent of the box.  oriented: divide by dr; else multiply by inv.
-template <bool kCanStart, bool kOriented>
+// finite: ro - c is finite, so the rotation leaves it (but for the sign of a
+// zero, which no test below sees).
+template <bool kCanStart, bool kOriented, bool kFinite = false>
 CT_D bool intersect_box(F3 c, F3 ro, F3 dr, F3 sg, F3 inv, float &dist, F3 *normal = nullptr) {
   const float r = kHalfVoxel, ir = 64.0f;  // safeInverse(HALF_VOXEL_EXTENT)
-  F3 o = rot_mul(sub(ro, c));
+  F3 o = kFinite ? sub(ro, c) : rot_mul(sub(ro, c));
   float winding = 1.0f;
   if (kCanStart) {
     F3 rb = muls(vabs(o), ir);
@@ -228,7 +259,7 @@ CT_D F3 random_cosine_direction(uint32_t &seed, F3 n) {
   const float x = cp * sqrtf(r2);
   const float y = sp * sqrtf(r2);
   F3 u = fabsf(n.x) > 0.1f ? f3(0.0f, 1.0f, 0.0f) : f3(1.0f, 0.0f, 0.0f);
-  u = normalize(cross(n, u));
+  u = normalize_axis(cross(n, u));
   F3 v = cross(n, u);
   return add(add(muls(u, x), muls(v, y)), muls(n, z));
 }
@@ -524,7 +555,10 @@ constexpr float kU = 5.9604644775390625e-8f;  // 2^-24
 constexpr float kNearMax = 0.015625f;
 constexpr float kDeadAxis = 9.094947017729282e-13f;  // 2^-40: an axis that is never crossed
 
-CT_D float med3f(float a, float b, float c) { return gmax(gmin(a, b), gmin(gmax(a, b), c)); }
+// The lanes of the wave where b holds (the same value on every lane).
+CT_D uint64_t ballot(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+CT_D float med3f(float a, float b, float c) { return __builtin_amdgcn_fmed3f(a, b, c); }
+CT_D float fractf(float x) { return __builtin_amdgcn_fractf(x); }  // x - floor(x), below 1
 CT_D int32_t imin(int32_t a, int32_t b) { return a < b ? a : b; }
 CT_D int32_t imax(int32_t a, int32_t b) { return a > b ? a : b; }
 CT_D int32_t clampi(int32_t x, int32_t lo, int32_t hi) { return imax(imin(x, lo), imin(imax(x, lo), hi)); }
@@ -538,6 +572,7 @@ struct GridWalk {
   uint32_t target;               // any hit: the target voxel's cell (DGrid::cells)
   float limit, best_t;
   uint32_t best;                 // index in ids of the closest voxel
+  F3 best_n;                     // the normal of the face it is hit at
   bool occluded;
 
   // The brick record of a (negated) cell and its index (times 64); false
@@ -565,11 +600,12 @@ struct GridWalk {
     const F3 c = f3(((float)cx + 0.5f) * 0.03125f, ((float)cy + 0.5f) * 0.03125f, ((float)cz + 0.5f) * 0.03125f);
     float t;
     if (kAny) {
-      const bool hit = intersect_box<false, false>(c, oo, dr, sg, sinv, t);
+      const bool hit = intersect_box<false, false, true>(c, oo, dr, sg, sinv, t);
       if (hit && (t >= 0.0f) && (t <= limit) && (base | bit) != target) occluded = true;
     } else {
-      const bool hit = kMode == kTraceClosest ? intersect_box<true, true>(c, oo, dr, sg, sinv, t)
-                                              : intersect_box<true, false>(c, oo, dr, sg, sinv, t);
+      F3 n;
+      const bool hit = kMode == kTraceClosest ? intersect_box<true, true, true>(c, oo, dr, sg, sinv, t, &n)
+                                              : intersect_box<true, false, true>(c, oo, dr, sg, sinv, t, &n);
       if (hit && (kMode == kTraceClosest ? t > 0.0f : t >= 0.0f) && t <= best_t) {
         const uint64_t mask = ((uint64_t)e.y << 32) | e.x;
         const uint32_t idx = e.z + (uint32_t)__popcll(mask & ((1ull << bit) - 1ull));
@@ -581,28 +617,36 @@ struct GridWalk {
         if (better) {
           best_t = t;
           best = idx;
+          best_n = n;
         }
       }
     }
   }
 
-  // The state of a walk between its steps; `done` once it has ended.
+  // The state of a walk between its steps.
+  static constexpr uint32_t kStepping = 0, kAtVoxel = 1, kEnded = 2, kNone = 3;  // kNone: no ray
+  uint32_t state;
+  uint4 e;                       // the cell's brick, its index and the cell's bit in it
+  uint32_t cell_base, cell_bit;
+  int32_t box_m, box_ext;        // the empty box: to the cell (i | box_m) + box_ext
   int32_t ix, iy, iz;            // the cell
-  float px, py, pz, p;           // the position the ray entered it at, and p there
-  bool near, done;
+  float t_in;                    // where the ray entered it
+  uint32_t near;                 // 1: within p of a plane there
   float vx, vy, vz, qx, qy, qz, ivx, ivy, ivz, t_unit, t_end, k1;
   uint32_t octant;               // shift of the ray's nibble
 
   // Whether a position is within `m` of a lattice plane on an axis other
   // than the crossed one (always near its own plane); `any`: on any axis.
   CT_D static bool near_plane(float x, float y, float z, float m, bool any) {
-    const float fx = fabsf((x - floorf(x)) - 0.5f), fy = fabsf((y - floorf(y)) - 0.5f), fz = fabsf((z - floorf(z)) - 0.5f);
+    const float fx = fabsf(fractf(x) - 0.5f), fy = fabsf(fractf(y) - 0.5f), fz = fabsf(fractf(z) - 0.5f);
     return (any ? gmax(gmax(fx, fy), fz) : med3f(fx, fy, fz)) > 0.5f - m;
   }
 
   // Tests the cells across the edges within p of the position the ray
   // entered the cell at.
   CT_D void test_near() {
+    const float p = gmin(__builtin_fmaf(10.0f * kU, t_in, k1), kNearMax), px = __builtin_fmaf(vx, t_in, qx),
+                py = __builtin_fmaf(vy, t_in, qy), pz = __builtin_fmaf(vz, t_in, qz);
     const float fx = px - (float)ix, fy = py - (float)iy, fz = pz - (float)iz;
     const int32_t ax = fx < p ? -1 : (fx > 1.0f - p ? 1 : 0), ay = fy < p ? -1 : (fy > 1.0f - p ? 1 : 0),
                   az = fz < p ? -1 : (fz > 1.0f - p ? 1 : 0);
@@ -634,9 +678,20 @@ struct GridWalk {
     return t;
   }
 
-  // Sets the walk up; `done` at once when the ray misses the grid.
-  CT_D void start(const DScene &S, F3 o, F3 d, uint32_t ti, uint32_t tp) {
-    done = true;
+  // Sets the walk up for a ray and its limit (any hit: of the distance; else
+  // of the closest t); ended at once when the ray misses the grid.
+  CT_D void start(const DScene &S, F3 o, F3 d, float max_t, uint32_t ti, uint32_t tp) {
+    state = kEnded;
+    limit = max_t;
+    best_t = max_t;
+    best = kInvalid;
+    best_n = f3(0.0f, 0.0f, 0.0f);
+    occluded = false;
+    e = make_uint4(0u, 0u, 0u, 0u);
+    cell_base = 0u;
+    cell_bit = 0u;
+    box_m = 0;
+    box_ext = 0;
     float m[12];
 #pragma unroll
     for (int k = 0; k < 12; ++k) m[k] = G.w2o[k];
@@ -685,97 +740,125 @@ struct GridWalk {
     t_end = (kAny ? limit : best_t) * t_unit;
     const float t = gmax(tn, 0.0f);
     if (!(t <= tf) || t > t_end + kNearMax) return;
-    done = false;
     const float gm = gmax(gmax(gmax(fabsf((float)l0x), fabsf((float)hx)), gmax(fabsf((float)l0y), fabsf((float)hy))),
                           gmax(fabsf((float)l0z), fabsf((float)hz)));
     k1 = kU * (1.5f * gmax(qmax, gm) + gmax(gmax(lx ? ivx : 0.0f, ly ? ivy : 0.0f), lz ? ivz : 0.0f) + 4.0f);
-    px = __builtin_fmaf(vx, t, qx);
-    py = __builtin_fmaf(vy, t, qy);
-    pz = __builtin_fmaf(vz, t, qz);
+    t_in = t;
+    const float px = __builtin_fmaf(vx, t, qx), py = __builtin_fmaf(vy, t, qy), pz = __builtin_fmaf(vz, t, qz);
     ix = clampi((int32_t)floorf(px), l0x, hx);
     iy = clampi((int32_t)floorf(py), l0y, hy);
     iz = clampi((int32_t)floorf(pz), l0z, hz);
-    p = gmin(__builtin_fmaf(10.0f * kU, t, k1), kNearMax);
-    near = near_plane(px, py, pz, p, true);  // an origin in the grid has crossed no axis
+    const float p = gmin(__builtin_fmaf(10.0f * kU, t, k1), kNearMax);
+    near = near_plane(px, py, pz, p, true) ? 1u : 0u;  // an origin in the grid has crossed no axis
+    look(~0);
   }
 
-  // Lanes step until each has come to a voxel or ended (a cell's neighbours,
-  // rare, are tested on the spot); the voxel tests then run together, and
-  // nearly all accept.
-  CT_D void run(const DScene &S, F3 o, F3 d, uint32_t ti, uint32_t tp) {
-    constexpr uint32_t kStepping = 0, kAtVoxel = 1, kEnded = 2;
-    start(S, o, d, ti, tp);
-    if (done) return;
-    uint4 e = make_uint4(0u, 0u, 0u, 0u);
-    uint32_t base = 0, bit = 0, tested = kInvalid;  // the cell tested last
-    int32_t moved = ~0;  // bits of the cell that the last step changed
-    for (;;) {
-      uint32_t state = kStepping;
-      while (state == kStepping) {
-        if ((moved & ~3) != 0 && !brick(ix, iy, iz, e, base)) {
-          state = kEnded;
-          break;
-        }
-        if (near) {
-          test_near();
-          if (!kAny) t_end = best_t * t_unit;
-          if (kAny && occluded) {
-            state = kEnded;
-            break;
-          }
-        }
-        // the cell, the 2x2x2 cells around it when all are empty, or the
-        // empty cube of bricks
-        int32_t m = 3, ext = (int32_t)((e.w >> octant) & 15u) * 4 - 4;
-        if ((e.x | e.y) != 0u) {
-          bit = bit_of(ix, iy, iz);
-          const uint32_t w = (uint32_t)((((uint64_t)e.y << 32) | e.x) >> (bit & 0x2Au));
-          if (((w >> (bit & 0x15u)) & 1u) != 0u && (base | bit) != tested) {
-            state = kAtVoxel;
-            break;
-          }
-          m = (w & 0x00330033u) == 0u ? 1 : 0;
-          ext = 0;
-        }
-        if (near) m = ext = 0;
-        int32_t fx = (ix | m) + ext, fy = (iy | m) + ext, fz = (iz | m) + ext;
-        float tx, ty, tz, x, y, z, pn;
-        float t = leave(fx, fy, fz, tx, ty, tz, x, y, z, pn);
-        bool nr = near_plane(x, y, z, pn * (tx <= t ? ivx : (ty <= t ? ivy : ivz)), false);
-        if (nr && m != 0) {
-          fx = ix;
-          fy = iy;
-          fz = iz;
-          t = leave(fx, fy, fz, tx, ty, tz, x, y, z, pn);
-          nr = near_plane(x, y, z, pn * (tx <= t ? ivx : (ty <= t ? ivy : ivz)), false);
-        }
-        if (t > t_end + pn) {
-          state = kEnded;
-          break;
-        }
-        const int32_t nx = tx <= t ? fx + 1 : clampi((int32_t)floorf(x), ix, fx),
-                      ny = ty <= t ? fy + 1 : clampi((int32_t)floorf(y), iy, fy),
-                      nz = tz <= t ? fz + 1 : clampi((int32_t)floorf(z), iz, fz);
-        moved = (ix ^ nx) | (iy ^ ny) | (iz ^ nz);
-        ix = nx;
-        iy = ny;
-        iz = nz;
-        px = x;
-        py = y;
-        pz = z;
-        p = pn;
-        near = nr;
-      }
-      if (state == kEnded) return;
-      test(ix, iy, iz, e, base, bit);
-      if (kAny && occluded) return;
+  // The cell the walk has entered: its brick (when it is another one), the
+  // neighbours within p of its edges (rare, tested on the spot), and whether
+  // it is a voxel.  Else the empty box to step over: the cell, the 2x2x2
+  // cells around it when all are empty, or the empty cube of bricks.
+  // Written, as `move`, without early exits: each exit of a divergent loop
+  // costs a copy of the walk's state in every step.
+  CT_D void look(int32_t moved) {
+    bool ended = false;
+    if ((moved & ~3) != 0) ended = !brick(ix, iy, iz, e, cell_base);
+    if (near != 0u && !ended) {
+      test_near();
       if (!kAny) t_end = best_t * t_unit;
-      tested = base | bit;
-      near = false;  // its neighbours are done too
-      moved = 0;
+      if (kAny) ended = occluded;
+    }
+    const bool empty = (e.x | e.y) == 0u;
+    cell_bit = bit_of(ix, iy, iz);
+    const uint32_t w = (uint32_t)((((uint64_t)e.y << 32) | e.x) >> (cell_bit & 0x2Au));
+    const bool at_voxel = ((w >> (cell_bit & 0x15u)) & 1u) != 0u;
+    box_m = (w & 0x00330033u) == 0u ? 1 : 0;
+    box_m = empty ? 3 : box_m;
+    box_m = near != 0u ? 0 : box_m;
+    box_ext = empty && near == 0u ? (int32_t)((e.w >> octant) & 15u) * 4 - 4 : 0;
+    state = ended ? kEnded : (at_voxel ? kAtVoxel : kStepping);
+  }
+
+  // One step of a stepping walk: out of the empty box into the next cell.
+  CT_D void advance() {
+    int32_t fx = (ix | box_m) + box_ext, fy = (iy | box_m) + box_ext, fz = (iz | box_m) + box_ext;
+    float tx, ty, tz, x, y, z, pn;
+    float t = leave(fx, fy, fz, tx, ty, tz, x, y, z, pn);
+    bool nr = near_plane(x, y, z, pn * (tx <= t ? ivx : (ty <= t ? ivy : ivz)), false);
+    if (nr && box_m != 0) {
+      fx = ix;
+      fy = iy;
+      fz = iz;
+      t = leave(fx, fy, fz, tx, ty, tz, x, y, z, pn);
+      nr = near_plane(x, y, z, pn * (tx <= t ? ivx : (ty <= t ? ivy : ivz)), false);
+    }
+    const int32_t cx = clampi((int32_t)floorf(x), ix, fx), cy = clampi((int32_t)floorf(y), iy, fy),
+                  cz = clampi((int32_t)floorf(z), iz, fz);
+    const int32_t nx = tx <= t ? fx + 1 : cx, ny = ty <= t ? fy + 1 : cy, nz = tz <= t ? fz + 1 : cz;
+    const int32_t moved = (ix ^ nx) | (iy ^ ny) | (iz ^ nz);
+    ix = nx;
+    iy = ny;
+    iz = nz;
+    t_in = t;
+    near = nr ? 1u : 0u;
+    state = kEnded;
+    if (!(t > t_end + pn)) look(moved);
+  }
+
+  // The test of a walk at a voxel.  A closest walk whose hit lies before the
+  // cell's end has ended.
+  CT_D void test_voxel() {
+    test(ix, iy, iz, e, cell_base, cell_bit);
+    near = 0u;  // its neighbours are done too
+    box_m = 0;
+    box_ext = 0;
+    state = kAny && occluded ? kEnded : kStepping;
+    if (!kAny) {
+      t_end = best_t * t_unit;
+      float tx, ty, tz, x, y, z, pn;
+      if (leave(ix, iy, iz, tx, ty, tz, x, y, z, pn) > t_end + pn) state = kEnded;
+    }
+  }
+
+  // Lanes step until each has come to a voxel or ended; the voxel tests then
+  // run together, and nearly all accept.  (The ballot also keeps the
+  // compiler from testing each lane's voxel inside the stepping loop.)
+  CT_D void run() {
+    for (;;) {
+      while (state == kStepping) advance();
+      if (ballot(state == kAtVoxel) == 0ull) return;
+      if (state == kAtVoxel) test_voxel();
     }
   }
 };
+
+// Walks a stream of rays per lane: `next` starts the lane's next ray (false:
+// it has none left) and `done` takes the result of one that has ended.
+// Rays of a wave take 3 to 30 steps, and a wave that waits for its longest
+// ray runs at 30% of its lanes.  Here the stepping loop leaves once kWait
+// lanes wait, tests those at a voxel and gives those that have ended their
+// next ray; kWait balances idle lanes in the loop against the same in the
+// (about five times longer) code between the loops.
+template <int kMode, int kWait, class Next, class Done>
+CT_D void walk_stream(GridWalk<kMode> &w, Next next, Done done) {
+  using W = GridWalk<kMode>;
+  if (!next()) w.state = W::kNone;
+  for (;;) {
+    const int keep = __popcll(ballot(w.state != W::kNone)) - kWait;
+    if (w.state == W::kStepping) {
+      do w.advance();
+      while ((int)(w.state == W::kStepping) & (int)(__popcll(ballot(w.state == W::kStepping)) > keep));
+    }
+    if (w.state == W::kAtVoxel) w.test_voxel();
+    const int stepping = __popcll(ballot(w.state == W::kStepping)), ended = __popcll(ballot(w.state == W::kEnded));
+    if ((int)(stepping == 0) | (int)(ended >= kWait / 2)) {
+      if (w.state == W::kEnded) {
+        done();
+        if (!next()) w.state = W::kNone;
+      }
+      if (ballot(w.state != W::kNone) == 0ull) return;
+    }
+  }
+}
 
 // How a kernel is built to walk: the BVH, the BVH with counters, or the cell
 // grid (scenes that have one; the counters are the BVH's, so counted
@@ -791,11 +874,8 @@ CT_D bool traverse_mode(const DScene &S, F3 o, F3 d, float limit, uint32_t ti, u
                         uint32_t stride, TraceCnt &cnt, bool &overflow) {
   if constexpr (kWalk == kWalkGrid) {
     GridWalk<kMode> w{S.grid};
-    w.limit = limit;
-    w.best_t = best_t;
-    w.best = kInvalid;
-    w.occluded = false;
-    w.run(S, o, d, ti, tp);
+    w.start(S, o, d, kMode == kTraceAny ? limit : best_t, ti, tp);
+    w.run();
     if (kMode != kTraceAny && w.best != kInvalid) {
       const uint2 id = gld(S.grid.ids + w.best);
       best_t = w.best_t;

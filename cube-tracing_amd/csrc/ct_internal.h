@@ -80,6 +80,7 @@ constexpr uint32_t kGridSkip = 4;
 struct DGrid {
   const uint4 *bricks;   // null: the scene has no grid and is walked as a BVH
   const uint2 *ids;      // (instance, primitive)
+  const uint32_t *slots; // primitive slot, by the same index
   const uint32_t *cells; // by primitive slot: brick record << 6 | bit
   int32_t org[3];        // lattice cell of the grid's first cell, a multiple of 16
   uint32_t nblk[3];      // blocks per axis
@@ -179,7 +180,7 @@ struct BvhSet {
   uint32_t prim_capacity = 0;
   uint32_t cube_light_count = 0;
   uint32_t cube_light_hw = 0;   // entries held: deleted lights leave stale records past the count
-  DevBuf grid_bricks, grid_ids, grid_cells, grid_work;
+  DevBuf grid_bricks, grid_ids, grid_slots, grid_cells, grid_work;
   DGrid grid{};                 // bricks null: no grid
 };
 

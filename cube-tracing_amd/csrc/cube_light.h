@@ -92,7 +92,7 @@ CT_D F3 face_ray_origin(F3 p, uint32_t face) {
 // one LCG step of three numbers and a bit test, and only voxels level with P
 // compute its point.  A wave draws until its slowest lane is done, about 7
 // times, and 11 full draws of 90 instructions each were most of k_ris: at
-// 256^2 pixels and 32 candidates 203 us, with this 139 us (one wave a SIMD,
+// 256^2 pixels and 32 candidates 203 us, with this 111 us (one wave a SIMD,
 // bound by the chain of dependent instructions and light loads).
 CT_D bool draw_cube_point(F3 P, F3 n, int na, float ns, F3 c, float half, uint32_t &seed, uint32_t &face, F3 &pos) {
   uint32_t faces = (P.x < c.x - half ? 1u : 0u) | (P.x > c.x + half ? 2u : 0u) | (P.y < c.y - half ? 4u : 0u) |

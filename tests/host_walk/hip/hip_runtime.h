@@ -18,6 +18,9 @@ inline uint4 make_uint4(uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return
 inline uint32_t __float_as_uint(float f) { uint32_t u; std::memcpy(&u, &f, 4); return u; }
 inline float __uint_as_float(uint32_t u) { float f; std::memcpy(&f, &u, 4); return f; }
 inline uint32_t min(uint32_t a, uint32_t b) { return a < b ? a : b; }
+#define __builtin_amdgcn_ballot_w64(b) ((b) ? 1ull : 0ull)  // a wave of one lane
+inline float __builtin_amdgcn_fmed3f(float a, float b, float c) { return std::fmax(std::fmin(a, b), std::fmin(std::fmax(a, b), c)); }
+inline float __builtin_amdgcn_fractf(float x) { return std::fmin(x - std::floor(x), 0.99999994f); }
 inline int __popcll(uint64_t v) { return __builtin_popcountll(v); }
 inline int __ffs(int v) { return __builtin_ffs(v); }
 using std::isnan;

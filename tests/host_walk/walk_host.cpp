@@ -117,8 +117,23 @@ void both(const Scene &sc, const int32_t *cells, uint32_t n, F3 o, F3 d, float l
   bool ovf = false;
   const bool occ = traverse_mode<kMode, kWalkGrid>(sc.S, o, d, limit, target == kInvalid ? kInvalid : 0u, target, bt, bi,
                                                    bp, nullptr, 0u, cnt, ovf);
+  // the same ray three times in one stream
+  GridWalk<kMode> w{sc.S.grid};
+  int left = 3, off = 0;
+  walk_stream<kMode, 1>(
+      w,
+      [&]() -> bool {
+        if (left-- == 0) return false;
+        w.start(sc.S, o, d, limit, target == kInvalid ? kInvalid : 0u, target);
+        return true;
+      },
+      [&]() {
+        if (kMode == kTraceAny) off += w.occluded != occ;
+        else off += (w.best == kInvalid) != (bp == kInvalid) || (bp != kInvalid && (sc.ids[w.best].y != bp || w.best_t != bt));
+      });
+  if (off != 0 || left != -1) bp = kInvalid - 1u;  // reported as a difference
   *t_out = kMode == kTraceAny || bp == kInvalid ? 0.0f : bt;
-  *id_out = kMode == kTraceAny ? (uint32_t)occ : bp;
+  *id_out = kMode == kTraceAny && bp == kInvalid ? (uint32_t)occ : bp;
   const float *m = sc.S.grid.w2o;
   const F3 oo = xform3(m, o, 1.0f), od = xform3(m, d, 0.0f);
   const F3 dr = kMode == kTraceClosest ? mul_rot(od) : od;
