@@ -320,7 +320,7 @@ CT_D bool vertex_visible(const DFrame &F, F3 o, F3 d, float dist, uint32_t ti, u
   const uint32_t k = tr.slot++;
   if (k >= kRaySlots) return true;  // at most two tests per pixel; never taken
   if (kVis == kVisEmit) {
-    const uint32_t idx = tr.px * kRaySlots + k;
+    const size_t idx = ray_at(F, tr.px, k);
     F.ray_o[idx] = make_float4(o.x, o.y, o.z, dist);
     F.ray_d[idx] = make_float4(d.x, d.y, d.z, __uint_as_float(ti));
     F.ray_t[idx] = tp;
