@@ -67,6 +67,18 @@ struct alignas(16) DInst {
   uint32_t pad;
 };
 
+// A pointer to device memory kept in a record that kernels read: the loads
+// and stores through it are global instructions.  Through a plain pointer
+// from memory they are flat ones, which also wait on LDS, in order, and take
+// no scalar base.
+template <class T>
+struct GPtr {
+  __attribute__((address_space(1))) T *p;
+  GPtr() = default;
+  __host__ __device__ GPtr(T *q) : p((__attribute__((address_space(1))) T *)q) {}
+  __host__ __device__ operator T *() const { return (T *)p; }
+};
+
 // Cell grid of a scene whose voxels all sit on the 2^-5 lattice of one object
 // space (host side: build_grid).  Cells are grouped in bricks of 4x4x4 and
 // blocks of 4x4x4 bricks; the bricks of a block are contiguous, 64 records
@@ -78,21 +90,21 @@ struct alignas(16) DInst {
 // itself is not empty).  Everything outside the grid is empty.
 constexpr uint32_t kGridSkip = 4;
 struct DGrid {
-  const uint4 *bricks;   // null: the scene has no grid and is walked as a BVH
-  const uint2 *ids;      // (instance, primitive)
-  const uint32_t *slots; // primitive slot, by the same index
-  const uint32_t *cells; // by primitive slot: brick record << 6 | bit
+  GPtr<const uint4> bricks;   // null: the scene has no grid and is walked as a BVH
+  GPtr<const uint2> ids;      // (instance, primitive)
+  GPtr<const uint32_t> slots; // primitive slot, by the same index
+  GPtr<const uint32_t> cells; // by primitive slot: brick record << 6 | bit
   int32_t org[3];        // lattice cell of the grid's first cell, a multiple of 16
   uint32_t nblk[3];      // blocks per axis
   float w2o[12];         // world-to-object, shared by every instance (DInst::w2o)
 };
 
 struct DScene {
-  const DNode *blas_nodes;
-  const float4 *blas_leaves;  // (centre.xyz, prim id bits), Morton order
-  const DInst *inst;
-  const DNode *tlas_nodes;
-  const uint32_t *tlas_inst;  // instance id per TLAS leaf
+  GPtr<const DNode> blas_nodes;
+  GPtr<const float4> blas_leaves;  // (centre.xyz, prim id bits), Morton order
+  GPtr<const DInst> inst;
+  GPtr<const DNode> tlas_nodes;
+  GPtr<const uint32_t> tlas_inst;  // instance id per TLAS leaf
   uint32_t tlas_root;
   uint32_t n_inst;            // entries of `inst` (instance slots)
   DGrid grid;

@@ -66,44 +66,48 @@ struct DFrame {
   DScene S;
   DScene Sp;          // the scene before the last update (get_previous_tlas) when prev_set, else S
   uint32_t prev_set;  // CT_REMAP_BIT with a distinct previous set: temporal slot-1 queries trace Sp
-  const ct_aabb *aabbs;
-  const ct_primitive *prims;
-  const float4 *mats;   // [2 per material]: (diffuse, type), (emission, roughness)
-  const float4 *cube;   // [3 per light]: (pos, size), (emissive, type), (inst, prim, -, -)
-  const float4 *point;
-  const float4 *env;
-  const float *geo_t;   // [16 per instance] geometry_T = previous model * inverse(model)
-  const uint32_t *remap_prim, *remap_light, *prev_first;  // remapping tables, previous first indices
+  GPtr<const ct_aabb> aabbs;
+  GPtr<const ct_primitive> prims;
+  GPtr<const float4> mats;   // [2 per material]: (diffuse, type), (emission, roughness)
+  GPtr<const float4> cube;   // [3 per light]: (pos, size), (emissive, type), (inst, prim, -, -)
+  GPtr<const float4> point;
+  GPtr<const float4> env;
+  GPtr<const float> geo_t;   // [16 per instance] geometry_T = previous model * inverse(model)
+  GPtr<const uint32_t> remap_prim, remap_light, prev_first;  // remapping tables, previous first indices
   uint32_t remap_cap, remap_light_cap;
   float prev_vp[16];    // inverse(prev_inv_proj) * inverse(prev_inv_view)
-  float4 *dpos_c, *dnrm_c, *dorg_c;
-  uint4 *dhit_c;
-  float4 *dpos_p, *dnrm_p, *dorg_p;
-  uint4 *dhit_p;
-  uint4 *rA_i; float4 *rB_i; float *rC_i;
-  uint4 *rA_p; float4 *rB_p; float *rC_p;
-  float2 *vel;
-  float4 *img;
-  const float4 *img_prev;
-  float4 *taa;
-  float4 *hit;
-  uint32_t *pidx;
-  uint32_t *mask;
-  float4 *ray_o, *ray_d;
-  uint32_t *ray_t;
-  uint32_t *queue;   // [queue_cap]: far rays from the front, near rays from the back
+  GPtr<float4> dpos_c, dnrm_c, dorg_c;
+  GPtr<uint4> dhit_c;
+  GPtr<float4> dpos_p, dnrm_p, dorg_p;
+  GPtr<uint4> dhit_p;
+  GPtr<uint4> rA_i;
+  GPtr<float4> rB_i;
+  GPtr<float> rC_i;
+  GPtr<uint4> rA_p;
+  GPtr<float4> rB_p;
+  GPtr<float> rC_p;
+  GPtr<float2> vel;
+  GPtr<float4> img;
+  GPtr<const float4> img_prev;
+  GPtr<float4> taa;
+  GPtr<float4> hit;
+  GPtr<uint32_t> pidx;
+  GPtr<uint32_t> mask;
+  GPtr<float4> ray_o, ray_d;
+  GPtr<uint32_t> ray_t;
+  GPtr<uint32_t> queue;   // [queue_cap]: far rays from the front, near rays from the back
   uint32_t queue_cap;
-  uint32_t *counters;
-  float4 *gat;  // [8 per pixel] neighbour record, see st_gather
-  float4 *spc;  // spatial reuse's per-neighbour results, see spc_at
-  float4 *tpc;  // temporal reuse's two targets and flags, [2 per pixel], see temporal_emit
-  float4 *pres_o;    // [6 per pixel] output path reservoirs (this frame)
-  float4 *pres_t;    // [6 per pixel] temporal path reservoirs (history)
-  float4 *indirect;  // indirect colour of the first pass
-  float4 *pst;       // path state between the wavefront kernels (14 float4 per pixel)
-  float4 *rc;        // hybrid shift: retrace records, 2 slots of 5 float4 per pixel
-  uint32_t *ptq[2];  // path-segment queues (tagged pixel ids) of even / odd depths
-  float4 *seg_o, *seg_d, *seg_hit;  // path segments and their hits by queue position
+  GPtr<uint32_t> counters;
+  GPtr<float4> gat;  // [8 per pixel] neighbour record, see st_gather
+  GPtr<float4> spc;  // spatial reuse's per-neighbour results, see spc_at
+  GPtr<float4> tpc;  // temporal reuse's two targets and flags, [2 per pixel], see temporal_emit
+  GPtr<float4> pres_o;    // [6 per pixel] output path reservoirs (this frame)
+  GPtr<float4> pres_t;    // [6 per pixel] temporal path reservoirs (history)
+  GPtr<float4> indirect;  // indirect colour of the first pass
+  GPtr<float4> pst;       // path state between the wavefront kernels (14 float4 per pixel)
+  GPtr<float4> rc;        // hybrid shift: retrace records, 2 slots of 5 float4 per pixel
+  GPtr<uint32_t> ptq[2];  // path-segment queues (tagged pixel ids) of even / odd depths
+  GPtr<float4> seg_o, seg_d, seg_hit;  // path segments and their hits by queue position
   uint32_t qtag;     // frame index << kViewShift when frames are batched, else 0
   uint32_t taa_w, taa_h;  // TAA dispatch size (main.cpp:1642-1643 truncation applied)
   float far_ray;     // shadow rays at least this long are queued (and traced) first
@@ -116,6 +120,16 @@ struct FrameSet {
   const DFrame *fb;   // device array of frames
   const uint2 *blk;   // per block: (frame, first pixel or tile)
 };
+
+// A frame's record, which no kernel of the frame writes, as constant memory:
+// reads of its fields are scalar loads and their values sit in scalar
+// registers, also after the kernel's own stores (through plain memory each is
+// a vector load again).  `i` is the same on every lane.
+CT_D const DFrame &frame_at(const FrameSet &FS, uint32_t i) {
+  const __attribute__((address_space(4))) DFrame *p;
+  asm("" : "=s"(p) : "0"(FS.fb + i));  // else the casts cancel out
+  return *(const DFrame *)p;
+}
 
 struct PLight {
   F3 pos;
@@ -880,7 +894,7 @@ template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_primary(FrameSet FS, unsigned long long *stats) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   const uint32_t tid = threadIdx.x, lane = tid & 63u, w = tid >> 6;
   const uint32_t tiles_x = (F.W + 15) / 16;
   const uint32_t bx = blk_.y % tiles_x, by = blk_.y / tiles_x;
@@ -1011,7 +1025,7 @@ template <bool kBrdf, int kWalk>
 CT_D void ris_pass(const FrameSet &FS) {
   __shared__ uint32_t stk[kBrdf ? kStackWords<kWalk> : 1];
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px;
   const bool mine = pass_pixel(F, blk_, px);
   uint32_t emitted = 0, far = 0, ris_ray = 0, brdf_rays = 0, ris_mask = 0;
@@ -1136,7 +1150,7 @@ k_ris_brdf(FrameSet FS) {
 // queries made, not the rays traced for them.
 __global__ void __launch_bounds__(kBlock) k_temporal_finish(FrameSet FS) {
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px;
   const bool mine = pass_pixel(F, blk_, px);
   uint32_t queries = 0;
@@ -1181,7 +1195,7 @@ __global__ void __launch_bounds__(kBlock) k_temporal_finish(FrameSet FS) {
 template <bool kEmit>
 __global__ void __launch_bounds__(kBlock) k_spatial(FrameSet FS) {
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px = blk_.y + threadIdx.x;
   const bool mine = kEmit ? pass_pixel(F, blk_, px) : px < F.npix;
   uint32_t emitted = 0, far = 0;
@@ -1262,7 +1276,7 @@ CT_D uint32_t queue_push(bool active, uint32_t *count, uint32_t *also) {
 // (depth & 1) holds the length of the queue of that depth.
 __global__ void __launch_bounds__(kBlock) k_pt_begin(FrameSet FS) {
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px;
   const bool mine = pass_pixel(F, blk_, px);
   bool more = false;
@@ -1308,7 +1322,7 @@ struct RayBatches {
 template <int kWalk, bool kMulti>
 __global__ void __launch_bounds__(kBlock) k_trace_segments(FrameSet FS, uint32_t d, unsigned long long *stats) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
-  const DFrame &F0 = FS.fb[0];
+  const DFrame &F0 = frame_at(FS, 0u);
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t n = F0.counters[kCntPtQueue + (d & 1u)];
   TraceCnt cnt;
@@ -1320,7 +1334,7 @@ __global__ void __launch_bounds__(kBlock) k_trace_segments(FrameSet FS, uint32_t
       float bt = kMaxDistance;
       uint32_t bi = kInvalid, bp = kInvalid;
       bool ovf = false;
-      traverse_mode<kTraceBounce, kWalk>(FS.fb[view].S, xyz(o), xyz(dd), kMaxDistance, kInvalid, kInvalid, bt, bi,
+      traverse_mode<kTraceBounce, kWalk>((kMulti ? FS.fb[view] : F0).S, xyz(o), xyz(dd), kMaxDistance, kInvalid, kInvalid, bt, bi,
                                          bp, stk + tid, kBlock, cnt, ovf);
       F0.seg_hit[q] = make_float4(bt, __uint_as_float(bi), __uint_as_float(bp), 0.0f);
     }
@@ -1331,7 +1345,7 @@ __global__ void __launch_bounds__(kBlock) k_trace_segments(FrameSet FS, uint32_t
 // One path-loop iteration for every path of queue `d & 1`.
 template <bool kMulti>
 __global__ void __launch_bounds__(kBlock) k_pt_step(FrameSet FS, uint32_t d) {
-  const DFrame &F0 = FS.fb[0];
+  const DFrame &F0 = frame_at(FS, 0u);
   const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t n = F0.counters[kCntPtQueue + (d & 1u)];
   bool more = false;
@@ -1339,7 +1353,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_step(FrameSet FS, uint32_t d) {
   F3 ro, rd;
   if (q < n) {
     entry = F0.ptq[d & 1u][q];
-    const DFrame &F = FS.fb[kMulti ? (entry >> kViewShift) : 0u];
+    const DFrame &F = kMulti ? FS.fb[entry >> kViewShift] : F0;
     const uint32_t px = kMulti ? (entry & kSlotMask) : entry;
     PState p;
     ld_pstate(F.pst, F.npix, px, p, false);
@@ -1373,7 +1387,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_step(FrameSet FS, uint32_t d) {
 template <int kVis, bool kHybrid>
 __global__ void __launch_bounds__(kBlock) k_pt_end(FrameSet FS) {
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px;
   const bool mine = pass_pixel(F, blk_, px);
   PtTrace tr;
@@ -1442,7 +1456,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_end(FrameSet FS) {
 template <int kWalk, bool kMulti>
 __global__ void __launch_bounds__(kBlock) k_pt_retrace(FrameSet FS) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
-  const DFrame &F0 = FS.fb[0];
+  const DFrame &F0 = frame_at(FS, 0u);
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t n0 = F0.counters[kCntPtQueue], n = n0 + F0.counters[kCntPtQueue + 1];
   PtTrace tr;
@@ -1455,7 +1469,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_retrace(FrameSet FS) {
     if (q < n) {
       const uint32_t slot = q < n0 ? 0u : 1u;
       const uint32_t e = F0.ptq[slot][slot ? q - n0 : q];
-      const DFrame &F = FS.fb[kMulti ? (e >> kViewShift) : 0u];
+      const DFrame &F = kMulti ? FS.fb[e >> kViewShift] : F0;
       const uint32_t px = kMulti ? (e & kSlotMask) : e;
       const float4 req = rc_rec(F, px, slot)[0];
       const uint32_t di_index = __float_as_uint(req.x);
@@ -1476,7 +1490,7 @@ template <int kWalk, bool kHybrid>
 __global__ void __launch_bounds__(kBlock) k_pt_spatial(FrameSet FS, unsigned long long *stats) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px;
   const bool mine = pass_pixel(F, blk_, px);
   PtTrace tr;
@@ -1542,7 +1556,7 @@ __global__ void __launch_bounds__(kBlock) k_trace_bounce(DFrame F, const float4 
 // taa.glsl:16-108 over the dispatch region.
 __global__ void __launch_bounds__(kBlock) k_taa(FrameSet FS) {
   const uint2 blk_ = FS.blk[blockIdx.x];
-  const DFrame &F = FS.fb[blk_.x];
+  const DFrame &F = frame_at(FS, blk_.x);
   if (!(F.active & CT_TAA_BIT)) return;
   const uint32_t tw = F.taa_w, th = F.taa_h;
   const uint32_t t = blk_.y + threadIdx.x;
@@ -1663,7 +1677,7 @@ template <int kWalk, bool kMulti, int kSel = kSelAll>
 __global__ void __launch_bounds__(kBlock) k_trace_any_frames(FrameSet FS, uint32_t max_rays,
                                                              unsigned long long *stats) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
-  const DFrame &F0 = FS.fb[0];
+  const DFrame &F0 = frame_at(FS, 0u);
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t nfar = F0.counters[kCntQueue];
   uint32_t count = nfar + F0.counters[kCntQueueNear];
@@ -1674,7 +1688,7 @@ __global__ void __launch_bounds__(kBlock) k_trace_any_frames(FrameSet FS, uint32
     if (q < count) {
       // far rays from the front, then near rays from the back end down
       const uint32_t e = F0.queue[q < nfar ? q : F0.queue_cap - 1u - (q - nfar)];
-      const DFrame &F = FS.fb[kMulti ? (e >> kViewShift) : 0u];
+      const DFrame &F = kMulti ? FS.fb[e >> kViewShift] : F0;
       const uint32_t idx = kMulti ? (e & kSlotMask) : e;
       const bool mine = kSel == kSelAll || ((F.prev_set != 0u && idx % kRaySlots == 1u) == (kSel == kSelPrevious));
       if (mine) {
