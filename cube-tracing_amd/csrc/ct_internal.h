@@ -377,7 +377,6 @@ struct TraceAnyArgs {
   const uint32_t *ray_t; // target primitive
   const uint32_t *queue; // ray indices, or null: index = queue position
   const uint32_t *count; // device count (queue length)
-  uint32_t *head;        // device work counter, zeroed by the launch
   uint32_t *mask;        // per-pixel occlusion bits (index / 16, bit index % 16)
   uint8_t *occ;          // alternatively one byte per ray (index), may be null
   unsigned long long *stats;  // nodes, leaves, instances (instrumented launch) or null

@@ -45,8 +45,8 @@ enum {
 // counters[] slots
 // kCntQueue counts the far rays at the front of the ray queue, kCntQueueNear
 // the near rays stored from its back end down (see queue_flush).
-constexpr int kCntQueue = 0, kCntHead = 1, kCntRis = 2, kCntTemporal = 3, kCntSpatial = 4, kCntPtBounce = 5,
-              kCntPtShadow = 6, kCntQueueNear = 7, kCntPtQueue = 8 /* and 9 */, kCntPtHead = 10;
+constexpr int kCntQueue = 0, kCntRis = 2, kCntTemporal = 3, kCntSpatial = 4, kCntPtBounce = 5,
+              kCntPtShadow = 6, kCntQueueNear = 7, kCntPtQueue = 8 /* and 9 */;
 #ifndef CT_FAR_RAY
 #define CT_FAR_RAY 2.0f
 #endif
@@ -817,11 +817,20 @@ CT_D void camera_ray(const DFrame &F, uint32_t x, uint32_t y, F3 &o, F3 &d) {
 
 #include "restir_pt.h"
 
-// Sums a per-lane count over the wave; lane 0 adds it to `dst`.
-CT_D void wave_add(uint32_t v, uint32_t *dst) {
+// Adds a per-lane count over the block to `dst` with one atomic (one a wave
+// took 2% of a frame: the counters share a line that 8 L2s hand around).
+// Every thread of the block calls it.
+CT_D void block_add(uint32_t v, uint32_t *dst) {
+  __shared__ uint32_t s_sum[kBlock / 64];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off);
-  if (__lane_id() == 0 && v) atomicAdd(dst, v);
+  if (__lane_id() == 0) s_sum[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint32_t tot = 0;
+    for (int i = 0; i < kBlock / 64; ++i) tot += s_sum[i];
+    if (tot) atomicAdd(dst, tot);
+  }
 }
 CT_D void wave_add_cnt(const TraceCnt &c, unsigned long long *dst) {
   unsigned long long a = c.nodes, b = c.leaves, d = c.insts;
@@ -840,13 +849,12 @@ CT_D void wave_add_cnt(const TraceCnt &c, unsigned long long *dst) {
 
 // ----------------------------------------------------------- queue push
 // Appends this thread's emitted slots (bit k -> ray pixel*16 + k) to the
-// ray queue with two atomics per block and adds their number to counter
-// `counter` (none when negative). Slots in `far` (rays of at least kFarRay)
+// ray queue with two atomics per block. Slots in `far` (rays of at least kFarRay)
 // fill the queue from the front (count kCntQueue), the others from the back
 // end down (count kCntQueueNear): the traversal takes far rays first, so
 // the long walks start early and waves hold rays of like length. Every
 // thread of the block calls it.
-CT_D void queue_flush(const DFrame &F, uint32_t px, uint32_t emitted, uint32_t far, int counter) {
+CT_D void queue_flush(const DFrame &F, uint32_t px, uint32_t emitted, uint32_t far) {
   __shared__ uint32_t s_wsum[kBlock / 64];
   __shared__ uint32_t s_base_far, s_base_near;
   const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
@@ -871,7 +879,6 @@ CT_D void queue_flush(const DFrame &F, uint32_t px, uint32_t emitted, uint32_t f
     const uint32_t tf = tot & 0xFFFFu, tn = tot >> 16;
     s_base_far = tf ? atomicAdd(&F.counters[kCntQueue], tf) : 0u;
     s_base_near = tn ? atomicAdd(&F.counters[kCntQueueNear], tn) : 0u;
-    if ((tf + tn) && counter >= 0) atomicAdd(&F.counters[counter], tf + tn);
   }
   __syncthreads();
   const uint32_t before = s_wsum[w] + incl - c;
@@ -1125,9 +1132,12 @@ CT_D void ris_pass(const FrameSet &FS) {
     st_di(F.dpos_c, F.dnrm_c, F.dorg_c, F.dhit_c, px, di);
     F.mask[px] = ris_mask;
   }
-  wave_add(ris_ray, &F.counters[kCntRis]);
-  if (kBrdf) wave_add(brdf_rays, &F.counters[kCntPtBounce]);
-  queue_flush(F, px, emitted, far, -1);
+  block_add(ris_ray, &F.counters[kCntRis]);
+  if (kBrdf) {
+    __syncthreads();
+    block_add(brdf_rays, &F.counters[kCntPtBounce]);
+  }
+  queue_flush(F, px, emitted, far);
 }
 // Five waves per SIMD (at most 96 VGPRs, a few dwords spilled) run the
 // VALU-heavy pass faster than four without spills.  With the BRDF
@@ -1153,6 +1163,12 @@ __global__ void __launch_bounds__(kBlock) k_temporal_finish(FrameSet FS) {
   const DFrame &F = frame_at(FS, blk_.x);
   uint32_t px;
   const bool mine = pass_pixel(F, blk_, px);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // the ray queue is traced, the segment queues start
+    F.counters[kCntQueue] = 0u;
+    F.counters[kCntQueueNear] = 0u;
+    F.counters[kCntPtQueue] = 0u;
+    F.counters[kCntPtQueue + 1] = 0u;
+  }
   uint32_t queries = 0;
   if (mine) {
     const float4 pd = F.dpos_c[px];
@@ -1185,7 +1201,7 @@ __global__ void __launch_bounds__(kBlock) k_temporal_finish(FrameSet FS) {
       st_gather(F.gat, px, pd, pn, po, ph.x, ph.y, r);
     }
   }
-  wave_add(queries, &F.counters[kCntTemporal]);
+  block_add(queries, &F.counters[kCntTemporal]);
 }
 
 // Shading pass: spatial reuse (EMIT / FINISH) then shade and store.
@@ -1240,12 +1256,12 @@ __global__ void __launch_bounds__(kBlock) k_spatial(FrameSet FS) {
     }
     if (kEmit) F.mask[px] = 0u;
   }
-  if (kEmit) queue_flush(F, px, emitted, far, kCntSpatial);
+  if (kEmit) queue_flush(F, px, emitted, far);
 }
 
 // Appends this thread's item (when `active`) to a queue with one atomic per
 // block; returns its position.  Every thread of the block calls it.
-CT_D uint32_t queue_push(bool active, uint32_t *count, uint32_t *also) {
+CT_D uint32_t queue_push(bool active, uint32_t *count) {
   __shared__ uint32_t s_wsum[kBlock / 64];
   __shared__ uint32_t s_base;
   const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
@@ -1261,7 +1277,6 @@ CT_D uint32_t queue_push(bool active, uint32_t *count, uint32_t *also) {
       tot += t;
     }
     s_base = tot ? atomicAdd(count, tot) : 0u;
-    if (tot && also) atomicAdd(also, tot);
   }
   __syncthreads();
   return active ? s_base + s_wsum[w] + before : kInvalid;
@@ -1289,7 +1304,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_begin(FrameSet FS) {
     ro = compute_ray_origin(p.origin, p.dir);
     rd = p.dir;
   }
-  const uint32_t pos = queue_push(more, &F.counters[kCntPtQueue], &F.counters[kCntPtBounce]);
+  const uint32_t pos = queue_push(more, &F.counters[kCntPtQueue]);
   if (more) {
     F.ptq[0][pos] = F.qtag | px;
     F.seg_o[pos] = make_float4(ro.x, ro.y, ro.z, 0.0f);
@@ -1297,24 +1312,21 @@ __global__ void __launch_bounds__(kBlock) k_pt_begin(FrameSet FS) {
   }
 }
 
-// Batches of 64 queued rays for a persistent wave. The first batch is the
-// wave's own index in the grid, taken without an atomic; later batches come
-// from the shared head, offset by the rays the first batches cover. With a
-// grid of resident blocks every first batch starts at once, so a launch with
-// few rays costs about one batch, not one atomic per wave of the grid.
+// Batches of 64 queued rays for a persistent wave: its own index in the grid,
+// then a grid further.  A shared counter instead (each wave taking its next
+// batch with an atomic) was the bound of these kernels: with a resident grid
+// a wave has 1 to 3 batches, so almost every one paid an atomic on one
+// address that 8 L2s hand around, about 16 ns each and 11 k a launch, while
+// the launch order already mixes far and near rays.  k_trace_any of a 1080p
+// frame 250 -> 171 us a launch, 8 frames 19.8 -> 17.7 ms.
 struct RayBatches {
   uint32_t base, count, stride;
-  uint32_t *head;
-  CT_D RayBatches(uint32_t count_, uint32_t *head_) : count(count_), head(head_) {
+  CT_D explicit RayBatches(uint32_t count_) : count(count_) {
     stride = gridDim.x * (kBlock / 64u) * 64u;
     base = (blockIdx.x * (kBlock / 64u) + (threadIdx.x >> 6)) * 64u;
   }
   CT_D bool valid() const { return base < count; }
-  CT_D void next() {
-    uint32_t b = 0xFFFFFFFFu;
-    if ((threadIdx.x & 63u) == 0u) b = atomicAdd(head, 64u) + stride;
-    base = __shfl(b, 0);
-  }
+  CT_D void next() { base += stride; }
 };
 
 // Closest voxel of each queued path segment (intersect() semantics), one
@@ -1325,8 +1337,12 @@ __global__ void __launch_bounds__(kBlock) k_trace_segments(FrameSet FS, uint32_t
   const DFrame &F0 = frame_at(FS, 0u);
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t n = F0.counters[kCntPtQueue + (d & 1u)];
+  if (blockIdx.x == 0 && tid == 0) {  // for k_pt_step, which fills the other queue next
+    F0.counters[kCntPtBounce] += n;
+    F0.counters[kCntPtQueue + ((d + 1u) & 1u)] = 0u;
+  }
   TraceCnt cnt;
-  for (RayBatches rb(n, &F0.counters[kCntPtHead]); rb.valid(); rb.next()) {
+  for (RayBatches rb(n); rb.valid(); rb.next()) {
     const uint32_t q = rb.base + lane;
     if (q < n) {
       const uint32_t view = kMulti ? (F0.ptq[d & 1u][q] >> kViewShift) : 0u;
@@ -1369,7 +1385,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_step(FrameSet FS, uint32_t d) {
     ro = compute_ray_origin(p.origin, p.dir);
     rd = p.dir;
   }
-  const uint32_t pos = queue_push(more, &F0.counters[kCntPtQueue + ((d + 1u) & 1u)], &F0.counters[kCntPtBounce]);
+  const uint32_t pos = queue_push(more, &F0.counters[kCntPtQueue + ((d + 1u) & 1u)]);
   if (more) {
     F0.ptq[(d + 1u) & 1u][pos] = entry;
     F0.seg_o[pos] = make_float4(ro.x, ro.y, ro.z, 0.0f);
@@ -1403,6 +1419,10 @@ __global__ void __launch_bounds__(kBlock) k_pt_end(FrameSet FS) {
   tr.rc_slot = 0u;
   tr.rc_prev = 0u;
   tr.rc_req = 0u;
+  if (kVis == kVisFinish && blockIdx.x == 0 && threadIdx.x == 0) {  // the ray queue is traced
+    F.counters[kCntQueue] = 0u;
+    F.counters[kCntQueueNear] = 0u;
+  }
   if (mine) {
     if (F.dpos_c[px].w > 0.0f) {
       const uint32_t x = px % F.W, y = px / F.W;
@@ -1437,14 +1457,14 @@ __global__ void __launch_bounds__(kBlock) k_pt_end(FrameSet FS) {
     }
     if (kVis == kVisEmit) F.mask[px] = 0u;
   }
-  if (kVis == kVisEmit) queue_flush(F, px, tr.emitted, tr.far, kCntPtShadow);
+  if (kVis == kVisEmit) queue_flush(F, px, tr.emitted, tr.far);
   if (kVis == kVisRequest) {
     // the segment queues are idle after the path loop: slot k's retraces
     // go to queue k
     const bool r0 = (tr.rc_req & 1u) != 0u, r1 = (tr.rc_req & 2u) != 0u;
-    const uint32_t p0 = queue_push(r0, &F.counters[kCntPtQueue], nullptr);
+    const uint32_t p0 = queue_push(r0, &F.counters[kCntPtQueue]);
     if (r0) F.ptq[0][p0] = F.qtag | px;
-    const uint32_t p1 = queue_push(r1, &F.counters[kCntPtQueue + 1], nullptr);
+    const uint32_t p1 = queue_push(r1, &F.counters[kCntPtQueue + 1]);
     if (r1) F.ptq[1][p1] = F.qtag | px;
   }
 }
@@ -1464,7 +1484,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_retrace(FrameSet FS) {
   tr.bounce_rays = 0u;
   tr.shadow_rays = 0u;
   tr.overflow = false;
-  for (RayBatches rb(n, &F0.counters[kCntPtHead]); rb.valid(); rb.next()) {
+  for (RayBatches rb(n); rb.valid(); rb.next()) {
     const uint32_t q = rb.base + lane;
     if (q < n) {
       const uint32_t slot = q < n0 ? 0u : 1u;
@@ -1527,7 +1547,7 @@ __global__ void __launch_bounds__(kBlock) k_pt_spatial(FrameSet FS, unsigned lon
     if (F.active & CT_TAA_BIT) F.taa[px] = fp;
     F.dorg_p[px].w = __uint_as_float(seed);
   }
-  wave_add(tr.shadow_rays, &F.counters[kCntPtShadow]);
+  block_add(tr.shadow_rays, &F.counters[kCntPtShadow]);
   if (kWalk == kWalkCount) wave_add_cnt(tr.cnt, stats + 9);
 }
 
@@ -1636,7 +1656,7 @@ __global__ void __launch_bounds__(kBlock) k_trace_any(DScene S, TraceAnyArgs A) 
   uint32_t count = *A.count;
   if (count > A.max_rays) count = A.max_rays;
   TraceCnt cnt;
-  for (RayBatches rb(count, A.head); rb.valid(); rb.next()) {
+  for (RayBatches rb(count); rb.valid(); rb.next()) {
     const uint32_t q = rb.base + lane;
     if (q < count) {
       uint32_t idx = A.queue ? A.queue[q] : q;
@@ -1667,23 +1687,25 @@ __global__ void __launch_bounds__(kBlock) k_trace_any(DScene S, TraceAnyArgs A) 
 }
 
 // The frame path's any-hit traversal: the queue holds tagged slots of the
-// frames' ray buffers.
+// frames' ray buffers.  The queue's length is added to counter `counter`
+// (none when negative).
 // Queries of the launch after k_ris: kSel 0 traces every ray in the frame's
 // scene; in a frame that traces the previous set (prev_set), kSel 1 skips
 // its slot-1 rays (temporal reuse's target at the previous pixel) and kSel
 // 2 traces only those, in the previous set.
 constexpr int kSelAll = 0, kSelCurrent = 1, kSelPrevious = 2;
 template <int kWalk, bool kMulti, int kSel = kSelAll>
-__global__ void __launch_bounds__(kBlock) k_trace_any_frames(FrameSet FS, uint32_t max_rays,
+__global__ void __launch_bounds__(kBlock) k_trace_any_frames(FrameSet FS, uint32_t max_rays, int counter,
                                                              unsigned long long *stats) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
   const DFrame &F0 = frame_at(FS, 0u);
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
   const uint32_t nfar = F0.counters[kCntQueue];
   uint32_t count = nfar + F0.counters[kCntQueueNear];
+  if (counter >= 0 && blockIdx.x == 0 && tid == 0) F0.counters[counter] += count;
   if (count > max_rays) count = max_rays;
   TraceCnt cnt;
-  for (RayBatches rb(count, &F0.counters[kCntHead]); rb.valid(); rb.next()) {
+  for (RayBatches rb(count); rb.valid(); rb.next()) {
     const uint32_t q = rb.base + lane;
     if (q < count) {
       // far rays from the front, then near rays from the back end down
@@ -1801,7 +1823,6 @@ void with_walk(int walk, F f) {
 }  // namespace
 
 int launch_trace_any(const DScene &s, const TraceAnyArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, a.head, 0, 1);
   with_walk(scene_walk(s, a.stats != nullptr), [&](auto w) {
     constexpr int kWalk = decltype(w)::value;
     const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(a.max_rays), 1), any_single_resident<kWalk>());
@@ -2133,10 +2154,10 @@ uint32_t trace_blocks(const Launch &L, uint32_t resident) {
   return kWalk == kWalkGrid ? resident : std::min<uint32_t>(L.trace_blocks, resident);
 }
 
-// The queue length and the fetch head (kCntHead) are zeroed by the caller
-// before the pass that fills the queue.  The previous set has no grid.
+// The queue length is zeroed before the pass that fills the queue, by the
+// pass before it (k_temporal_finish, k_pt_end).  The previous set has no grid.
 template <int kSel = kSelAll>
-void launch_any(const Launch &L, FrameSet fs, uint32_t max_rays, hipStream_t st) {
+void launch_any(const Launch &L, FrameSet fs, uint32_t max_rays, int counter, hipStream_t st) {
   with_walk(kSel == kSelPrevious && L.walk == kWalkGrid ? kWalkBvh : L.walk, [&](auto w) {
     constexpr int kWalk = decltype(w)::value;
     auto go = [&](auto m) {
@@ -2144,7 +2165,7 @@ void launch_any(const Launch &L, FrameSet fs, uint32_t max_rays, hipStream_t st)
       const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(max_rays), 1),
                                                trace_blocks<kWalk>(L, any_resident<kWalk, kMulti, kSel>()));
       hipLaunchKernelGGL((k_trace_any_frames<kWalk, kMulti, kSel>), dim3(grid), dim3(kBlock), 0, st, fs, max_rays,
-                         L.stats);
+                         counter, L.stats);
     };
     if (L.multi)
       go(std::true_type{});
@@ -2171,7 +2192,7 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
   const FrameSet pix = kTiled ? tiles : runs;
   const uint32_t np = L.total_px, nb = kTiled ? L.blocks[0] : L.blocks[1];
   if (phases & kPhaseFirst) {
-  // queue, fetch head and the ray statistics
+  // the ray queue and the ray statistics
   hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, L.counters, 0, 8);
   if (L.stats) hipLaunchKernelGGL(k_reset_u64, dim3(1), dim3(64), 0, st, L.stats, 12);
   if ((rc = mark())) return rc;  // kMarkStart
@@ -2191,27 +2212,17 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
   if (L.prev_trace) {
     // RIS and temporal reuse visibility; the target-at-previous queries of
     // frames that trace the previous set in a second pass over the queue
-    launch_any<kSelCurrent>(L, pix, 3 * np, st);
-    hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters, 1u << kCntHead);
-    launch_any<kSelPrevious>(L, pix, 3 * np, st);
+    launch_any<kSelCurrent>(L, pix, 3 * np, -1, st);
+    launch_any<kSelPrevious>(L, pix, 3 * np, -1, st);
   } else {
-    launch_any(L, pix, 3 * np, st);  // RIS and temporal reuse visibility
+    launch_any(L, pix, 3 * np, -1, st);  // RIS and temporal reuse visibility
   }
   if ((rc = mark())) return rc;  // kMarkTraceRis
   hipLaunchKernelGGL(k_temporal_finish, dim3(nb), dim3(kBlock), 0, st, pix);
   if ((rc = mark())) return rc;  // kMarkTemporalFinish
   if (L.pt_depth) {
-    // both segment queues and their head, and the ray queue and head that
-    // path-reuse visibility uses after the path loop
-    hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters,
-                       (1u << kCntPtQueue) | (1u << (kCntPtQueue + 1)) | (1u << kCntPtHead) | (1u << kCntQueue) |
-                           (1u << kCntQueueNear) | (1u << kCntHead));
     hipLaunchKernelGGL(k_pt_begin, dim3(nb), dim3(kBlock), 0, st, pix);
     for (uint32_t d = 0; d < L.pt_depth; ++d) {
-      // the next queue and the fetch counter start at zero (already so at depth 0)
-      if (d > 0)
-        hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters,
-                           (1u << (kCntPtQueue + ((d + 1) & 1u))) | (1u << kCntPtHead));
       if ((rc = seg_mark())) return rc;
       with_walk(L.walk, [&](auto w) {
         constexpr int kWalk = decltype(w)::value;
@@ -2237,7 +2248,7 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
       // the retraces temporal path reuse needs: requested into the idle
       // segment queues, traced at full waves, read by both passes below
       hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters,
-                         (1u << kCntPtQueue) | (1u << (kCntPtQueue + 1)) | (1u << kCntPtHead));
+                         (1u << kCntPtQueue) | (1u << (kCntPtQueue + 1)));
       hipLaunchKernelGGL((k_pt_end<kVisRequest, true>), dim3(nb), dim3(kBlock), 0, st, pix);
       with_walk(L.walk, [&](auto w) {
         constexpr int kWalk = decltype(w)::value == kWalkGrid ? kWalkGrid : kWalkBvh;  // never counted
@@ -2258,18 +2269,16 @@ int enqueue_frames(const Launch &L, hipStream_t st, Mark mark, SegMark seg_mark,
     }
   }
   if ((rc = mark())) return rc;  // kMarkPtEmit
-  if (L.pt_depth) launch_any(L, pix, 2 * np, st);
+  if (L.pt_depth) launch_any(L, pix, 2 * np, kCntPtShadow, st);
   if ((rc = mark())) return rc;  // kMarkTracePt
   if (L.pt_depth && L.hybrid) hipLaunchKernelGGL((k_pt_end<kVisFinish, true>), dim3(nb), dim3(kBlock), 0, st, pix);
   if (L.pt_depth && !L.hybrid) hipLaunchKernelGGL((k_pt_end<kVisFinish, false>), dim3(nb), dim3(kBlock), 0, st, pix);
   if ((rc = mark())) return rc;  // kMarkPt
   }
   if (phases & kPhaseSpatial) {
-  hipLaunchKernelGGL(k_reset_mask, dim3(1), dim3(64), 0, st, L.counters,
-                     (1u << kCntQueue) | (1u << kCntQueueNear) | (1u << kCntHead));
   hipLaunchKernelGGL(k_spatial<true>, dim3(nb), dim3(kBlock), 0, st, pix);
   if ((rc = mark())) return rc;  // kMarkSpatialEmit
-  launch_any(L, pix, 2 * L.max_neighbors * np, st);
+  launch_any(L, pix, 2 * L.max_neighbors * np, kCntSpatial, st);
   if ((rc = mark())) return rc;  // kMarkTraceSpatial
   hipLaunchKernelGGL(k_spatial<false>, dim3(L.blocks[1]), dim3(kBlock), 0, st, runs);
   if ((rc = mark())) return rc;  // kMarkSpatialFinish

@@ -99,7 +99,6 @@ int ct_trace_any_noalloc(ct_accel *a, uint32_t n, const float *origins, const fl
   t.ray_t = rt;
   t.queue = nullptr;
   t.count = cnt;
-  t.head = cnt + 1;  // zeroed by the launch
   t.mask = nullptr;
   t.occ = occluded_out;
   t.stats = nullptr;
@@ -182,7 +181,6 @@ int ct_trace_any(ct_accel *a, uint32_t n, const float *origins, const float *dir
   t.ray_t = s.t.as<uint32_t>();
   t.queue = nullptr;
   t.count = s.cnt.as<uint32_t>();
-  t.head = s.cnt.as<uint32_t>() + 1;
   t.mask = nullptr;
   t.occ = s.occ.as<uint8_t>();
   t.stats = stats ? s.stats.as<unsigned long long>() : nullptr;
