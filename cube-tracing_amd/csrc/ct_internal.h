@@ -10,6 +10,8 @@
 #include <memory>
 #include <deque>
 #include <queue>
+#include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -283,6 +285,9 @@ struct Accel {
   DevBuf pt_mats;
   uint32_t pt_mat_count = 0;
   BuildScratch scratch;
+  std::mutex io_mu;                         // held by through_device, which uses the two below
+  DevBuf io_dev;
+  PinnedBuf io_host;
   PinnedBuf readback;                       // GPU deletions' slots on their way to the host mirror
   DevBuf upload;                            // packed slot records and remapping writes on their way in
   uint32_t status = CT_AS_IDLE;
@@ -370,29 +375,35 @@ DScene scene_view(const Accel &a);
 DScene previous_scene_view(const Accel &a);
 bool previous_distinct(const Accel &a);
 
-// Launch the any-hit traversal over a ray queue (frame.hip / trace.hip).
+// Traversal launches over packed ray arrays on the device (frame.hip), three
+// floats per origin and direction.
 struct TraceAnyArgs {
-  const float4 *ray_o;   // (origin, distance)
-  const float4 *ray_d;   // (direction, target instance bits)
-  const uint32_t *ray_t; // target primitive
-  const uint32_t *queue; // ray indices, or null: index = queue position
-  const uint32_t *count; // device count (queue length)
-  uint32_t *mask;        // per-pixel occlusion bits (index / 16, bit index % 16)
-  uint8_t *occ;          // alternatively one byte per ray (index), may be null
+  const float *o, *d, *dist;
+  const uint32_t *targets;    // (instance, primitive) per ray, or null
+  uint8_t *occ;
   unsigned long long *stats;  // nodes, leaves, instances (instrumented launch) or null
-  uint32_t max_rays;
+  uint32_t n;
 };
 int launch_trace_any(const DScene &s, const TraceAnyArgs &args, hipStream_t stream);
 
 struct TraceClosestArgs {
-  const float4 *ray_o;   // (origin, -)
-  const float4 *ray_d;   // (direction, -)
+  const float *o, *d;
   float tmax;
   uint32_t n;
-  float4 *hit;           // (t, instance bits, primitive bits, -)
+  float *t;       // -1: no hit
+  uint32_t *ids;  // (instance, primitive) per ray
   unsigned long long *stats;
 };
 int launch_trace_closest(const DScene &s, const TraceClosestArgs &args, hipStream_t stream);
+
+// Host arrays on their way to the device and back (trace.hip).  Copies every
+// `in` array into one block and the block's `out` arrays back after
+// launch(device address of each array, in order) has enqueued its work on the
+// accel's stream.  Arrays start at multiples of 16 bytes.
+struct HostIn { const void *p; size_t bytes; };
+struct HostOut { void *p; size_t bytes; };
+int through_device(Accel &a, const std::vector<HostIn> &in, const std::vector<HostOut> &out,
+                   const std::function<int(const std::vector<void *> &)> &launch);
 
 int device_count_gfx950();
 

@@ -1551,11 +1551,26 @@ __global__ void __launch_bounds__(kBlock) k_pt_spatial(FrameSet FS, unsigned lon
   if (kWalk == kWalkCount) wave_add_cnt(tr.cnt, stats + 9);
 }
 
+CT_D F3 packed3(const float *p, uint32_t i) {
+  const float *q = p + 3 * (size_t)i;
+  return f3(q[0], q[1], q[2]);
+}
+CT_D void store3(float *p, uint32_t i, F3 v) {
+  float *q = p + 3 * (size_t)i;
+  q[0] = v.x;
+  q[1] = v.y;
+  q[2] = v.z;
+}
+
 // Path segments on caller rays (ct_trace_bounce).
+struct BounceArgs {
+  const float *o, *d;
+  uint32_t *ids;
+  float *pos, *nrm, *dist, *wo;
+  uint32_t n;
+};
 template <int kWalk>
-__global__ void __launch_bounds__(kBlock) k_trace_bounce(DFrame F, const float4 *ro, const float4 *rd, uint32_t n,
-                                                        float4 *pos_dist, float4 *nrm_ids, float4 *wo_prim,
-                                                        unsigned long long *stats) {
+__global__ void __launch_bounds__(kBlock) k_trace_bounce(DFrame F, BounceArgs A, unsigned long long *stats) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   PtTrace tr;
@@ -1563,12 +1578,14 @@ __global__ void __launch_bounds__(kBlock) k_trace_bounce(DFrame F, const float4 
   tr.bounce_rays = 0u;
   tr.shadow_rays = 0u;
   tr.overflow = false;
-  if (i < n) {
-    const Isect h = bounce_intersect<kWalk>(F, xyz(ro[i]), xyz(rd[i]), tr);
-    const uint32_t inst = h.is_hit ? h.inst : kInvalid, prim = h.is_hit ? h.prim : kInvalid;
-    pos_dist[i] = make_float4(h.P.x, h.P.y, h.P.z, h.distance);
-    nrm_ids[i] = make_float4(h.n.x, h.n.y, h.n.z, __uint_as_float(inst));
-    wo_prim[i] = make_float4(h.wo.x, h.wo.y, h.wo.z, __uint_as_float(prim));
+  if (i < A.n) {
+    const Isect h = bounce_intersect<kWalk>(F, packed3(A.o, i), packed3(A.d, i), tr);
+    A.ids[2 * (size_t)i] = h.is_hit ? h.inst : kInvalid;
+    A.ids[2 * (size_t)i + 1] = h.is_hit ? h.prim : kInvalid;
+    store3(A.pos, i, h.P);
+    store3(A.nrm, i, h.n);
+    A.dist[i] = h.distance;
+    store3(A.wo, i, h.wo);
   }
   if (kWalk == kWalkCount) wave_add_cnt(tr.cnt, stats);
 }
@@ -1648,27 +1665,26 @@ __global__ void k_store_frame(DFrame F, DFrame *dst) {
   for (uint32_t i = threadIdx.x; i < sizeof(DFrame) / 4; i += blockDim.x) d[i] = src[i];
 }
 
-// Any-hit traversal over a ray queue; each wave fetches 64 rays at a time.
+// Any-hit traversal over an array of rays; each wave fetches 64 at a time.
 template <int kWalk>
 __global__ void __launch_bounds__(kBlock) k_trace_any(DScene S, TraceAnyArgs A) {
   __shared__ uint32_t stk[kStackWords<kWalk>];
   const uint32_t tid = threadIdx.x, lane = tid & 63u;
-  uint32_t count = *A.count;
-  if (count > A.max_rays) count = A.max_rays;
   TraceCnt cnt;
-  for (RayBatches rb(count); rb.valid(); rb.next()) {
+  for (RayBatches rb(A.n); rb.valid(); rb.next()) {
     const uint32_t q = rb.base + lane;
-    if (q < count) {
-      uint32_t idx = A.queue ? A.queue[q] : q;
-      float4 o = A.ray_o[idx], d = A.ray_d[idx];
-      uint32_t tp = A.ray_t[idx];
+    if (q < A.n) {
+      uint32_t ti = kInvalid, tp = kInvalid;
+      if (A.targets) {
+        ti = A.targets[2 * (size_t)q];
+        tp = A.targets[2 * (size_t)q + 1];
+      }
       float bt = 0.0f;
       uint32_t bi = 0, bp = 0;
       bool ovf = false;
-      bool occ = traverse_mode<kTraceAny, kWalk>(S, f3(o.x, o.y, o.z), f3(d.x, d.y, d.z), o.w, __float_as_uint(d.w), tp,
-                                                 bt, bi, bp, stk + tid, kBlock, cnt, ovf);
-      if (occ && A.mask) atomicOr(&A.mask[idx / kRaySlots], 1u << (idx % kRaySlots));
-      if (A.occ) A.occ[idx] = occ ? 1 : 0;
+      const bool occ = traverse_mode<kTraceAny, kWalk>(S, packed3(A.o, q), packed3(A.d, q), A.dist[q], ti, tp, bt, bi,
+                                                       bp, stk + tid, kBlock, cnt, ovf);
+      A.occ[q] = occ ? 1 : 0;
     }
   }
   if (kWalk == kWalkCount) {
@@ -1737,13 +1753,14 @@ __global__ void __launch_bounds__(kBlock) k_trace_closest(DScene S, TraceClosest
   const uint32_t i = blockIdx.x * blockDim.x + tid;
   TraceCnt cnt;
   if (i < A.n) {
-    float4 o = A.ray_o[i], d = A.ray_d[i];
     float bt = A.tmax;
     uint32_t bi = kInvalid, bp = kInvalid;
     bool ovf = false;
-    traverse_mode<kTraceClosest, kWalk>(S, f3(o.x, o.y, o.z), f3(d.x, d.y, d.z), A.tmax, kInvalid, kInvalid, bt, bi, bp,
+    traverse_mode<kTraceClosest, kWalk>(S, packed3(A.o, i), packed3(A.d, i), A.tmax, kInvalid, kInvalid, bt, bi, bp,
                                         stk + tid, kBlock, cnt, ovf);
-    A.hit[i] = make_float4(bi != kInvalid ? bt : -1.0f, __uint_as_float(bi), __uint_as_float(bp), 0.0f);
+    A.t[i] = bi != kInvalid ? bt : -1.0f;
+    A.ids[2 * (size_t)i] = bi;
+    A.ids[2 * (size_t)i + 1] = bp;
   }
   if (kWalk == kWalkCount) {
     unsigned long long a = cnt.nodes, b = cnt.leaves, c = cnt.insts;
@@ -1825,7 +1842,7 @@ void with_walk(int walk, F f) {
 int launch_trace_any(const DScene &s, const TraceAnyArgs &a, hipStream_t st) {
   with_walk(scene_walk(s, a.stats != nullptr), [&](auto w) {
     constexpr int kWalk = decltype(w)::value;
-    const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(a.max_rays), 1), any_single_resident<kWalk>());
+    const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(a.n), 1), any_single_resident<kWalk>());
     hipLaunchKernelGGL(k_trace_any<kWalk>, dim3(grid), dim3(kBlock), 0, st, s, a);
   });
   CT_HIP(hipGetLastError());
@@ -3068,55 +3085,44 @@ int ct_trace_bounce(ct_accel *a, uint32_t n, const float *origins, const float *
   if (a->set.tlas_count == 0) return fail(CT_E_STATE, "ct_trace_bounce: empty scene");
   if (n == 0) return CT_OK;
   CT_HIP(hipSetDevice(a->device));
-  DevBuf o, d, r0, r1, r2, st;
-  int rc;
-  if ((rc = o.reserve(16 * (size_t)n)) || (rc = d.reserve(16 * (size_t)n)) || (rc = r0.reserve(16 * (size_t)n)) ||
-      (rc = r1.reserve(16 * (size_t)n)) || (rc = r2.reserve(16 * (size_t)n)) ||
-      (rc = st.reserve(3 * sizeof(unsigned long long))))
-    return rc;
-  std::vector<float4> ho(n), hd(n);
-  for (uint32_t i = 0; i < n; ++i) {
-    ho[i] = make_float4(origins[3 * i], origins[3 * i + 1], origins[3 * i + 2], 0.0f);
-    hd[i] = make_float4(directions[3 * i], directions[3 * i + 1], directions[3 * i + 2], 0.0f);
-  }
-  CT_HIP(hipMemcpy(o.p, ho.data(), 16 * (size_t)n, hipMemcpyHostToDevice));
-  CT_HIP(hipMemcpy(d.p, hd.data(), 16 * (size_t)n, hipMemcpyHostToDevice));
-  CT_HIP(hipMemset(st.p, 0, 3 * sizeof(unsigned long long)));
-  DFrame F;
-  std::memset(&F, 0, sizeof(F));
-  F.S = scene_view(*a);
-  F.Sp = F.S;
-  F.aabbs = a->set.aabbs.as<ct_aabb>();
-  F.prims = a->set.prims.as<ct_primitive>();
-  F.n_mats = 0;  // materials live in a frame context; the records here carry indices only
-  with_walk(scene_walk(F.S, stats != nullptr), [&](auto w) {
-    hipLaunchKernelGGL(k_trace_bounce<decltype(w)::value>, dim3(nblocks(n)), dim3(kBlock), 0, a->stream, F,
-                       o.as<float4>(), d.as<float4>(), n, r0.as<float4>(), r1.as<float4>(), r2.as<float4>(),
-                       stats ? st.as<unsigned long long>() : nullptr);
-  });
-  CT_HIP(hipGetLastError());
-  CT_HIP(hipStreamSynchronize(a->stream));
-  std::vector<float4> a0(n), a1(n), a2(n);
-  CT_HIP(hipMemcpy(a0.data(), r0.p, 16 * (size_t)n, hipMemcpyDeviceToHost));
-  CT_HIP(hipMemcpy(a1.data(), r1.p, 16 * (size_t)n, hipMemcpyDeviceToHost));
-  CT_HIP(hipMemcpy(a2.data(), r2.p, 16 * (size_t)n, hipMemcpyDeviceToHost));
-  for (uint32_t i = 0; i < n; ++i) {
-    pos_out[3 * i] = a0[i].x; pos_out[3 * i + 1] = a0[i].y; pos_out[3 * i + 2] = a0[i].z;
-    dist_out[i] = a0[i].w;
-    nrm_out[3 * i] = a1[i].x; nrm_out[3 * i + 1] = a1[i].y; nrm_out[3 * i + 2] = a1[i].z;
-    std::memcpy(&ids_out[2 * i], &a1[i].w, 4);
-    wo_out[3 * i] = a2[i].x; wo_out[3 * i + 1] = a2[i].y; wo_out[3 * i + 2] = a2[i].z;
-    std::memcpy(&ids_out[2 * i + 1], &a2[i].w, 4);
-  }
+  const size_t m = n;
+  unsigned long long v[3] = {0, 0, 0};
+  std::vector<HostIn> in{{origins, 12 * m}, {directions, 12 * m}};
+  std::vector<HostOut> out{{ids_out, 8 * m}, {pos_out, 12 * m}, {nrm_out, 12 * m}, {dist_out, 4 * m}, {wo_out, 12 * m}};
   if (stats) {
-    unsigned long long v[3];
-    CT_HIP(hipMemcpy(v, st.p, sizeof(v), hipMemcpyDeviceToHost));
+    in.push_back({v, sizeof(v)});
+    out.push_back({v, sizeof(v)});
+  }
+  const int rc = through_device(*a, in, out, [&](const std::vector<void *> &p) -> int {
+    const size_t k = in.size();
+    const BounceArgs A{static_cast<float *>(p[0]),     static_cast<float *>(p[1]),     static_cast<uint32_t *>(p[k]),
+                       static_cast<float *>(p[k + 1]), static_cast<float *>(p[k + 2]), static_cast<float *>(p[k + 3]),
+                       static_cast<float *>(p[k + 4]), n};
+    unsigned long long *cnt = nullptr;
+    if (stats) {
+      cnt = static_cast<unsigned long long *>(p.back());
+      CT_HIP(hipMemcpyAsync(cnt, p[2], sizeof(v), hipMemcpyDeviceToDevice, a->stream));
+    }
+    DFrame F;
+    std::memset(&F, 0, sizeof(F));
+    F.S = scene_view(*a);
+    F.Sp = F.S;
+    F.aabbs = a->set.aabbs.as<ct_aabb>();
+    F.prims = a->set.prims.as<ct_primitive>();
+    F.n_mats = 0;  // materials live in a frame context; the records here carry indices only
+    with_walk(scene_walk(F.S, stats != nullptr), [&](auto w) {
+      hipLaunchKernelGGL(k_trace_bounce<decltype(w)::value>, dim3(nblocks(n)), dim3(kBlock), 0, a->stream, F, A, cnt);
+    });
+    CT_HIP(hipGetLastError());
+    return CT_OK;
+  });
+  if (!rc && stats) {
     stats->rays = n;
     stats->nodes = v[0];
     stats->leaves = v[1];
     stats->instances = v[2];
   }
-  return CT_OK;
+  return rc;
 }
 
 int ct_pt_random_replay(ct_ctx *c, ct_accel *a, const ct_frame_params *p, int32_t dx, int32_t dy, uint32_t *out,

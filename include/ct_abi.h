@@ -415,10 +415,7 @@ int ct_trace_any(ct_accel *accel, uint32_t n, const float *origins,
  * capture, tight serving loops).  Same rays, same result bytes as
  * ct_trace_any, but every array is in DEVICE memory and the call is only
  * enqueued on `stream` (null: the accel's stream); nothing is copied back
- * and nothing is waited for.  The staged rays and the work counters live in
- * a fixed 36 MiB device array per GPU, so n is at most 2^20 (CT_E_CAPACITY
- * above); the array is shared by every call on that GPU, so calls that
- * overlap on one GPU race. */
+ * and nothing is waited for.  n is at most 2^20 (CT_E_CAPACITY above). */
 int ct_trace_any_noalloc(ct_accel *accel, uint32_t n, const float *origins,
                          const float *directions, const float *distances,
                          const uint32_t *targets, uint8_t *occluded_out,
