@@ -825,27 +825,37 @@ int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::
   if ((uint64_t)nrec > 4ull * n + (1u << 20)) return CT_OK;
   for (int c = 0; c < 4; ++c)
     for (int r = 0; r < 3; ++r) g.w2o[c * 3 + r] = w[c * 4 + r];
+  // One allocation: each takes and gives back about 0.4 ms, which a small
+  // world's load would feel.
+  size_t total = 0;
+  auto place = [&](size_t bytes) {
+    const size_t at = total;
+    total += (bytes + 255) & ~(size_t)255;
+    return at;
+  };
+  const size_t o_bricks = place(16 * (size_t)nrec), o_ids = place(8 * (size_t)n), o_slots = place(4 * (size_t)n),
+               o_cells = place(4 * (size_t)S.prim_capacity), o_work = place(8 + 4 * seg.size());
   int rc;
-  if ((rc = S.grid_bricks.reserve(16 * (size_t)nrec)) || (rc = S.grid_ids.reserve(8 * (size_t)n)) ||
-      (rc = S.grid_slots.reserve(4 * (size_t)n)) ||
-      (rc = S.grid_cells.reserve(4 * (size_t)S.prim_capacity)) || (rc = S.grid_work.reserve(8 + 4 * seg.size())))
-    return rc;
-  uint32_t *work = S.grid_work.as<uint32_t>(), *d_seg = work + 2;
+  if ((rc = S.grid_mem.reserve(total))) return rc;
+  unsigned char *mem = S.grid_mem.as<unsigned char>();
+  uint4 *bricks = reinterpret_cast<uint4 *>(mem + o_bricks);
+  uint2 *d_ids = reinterpret_cast<uint2 *>(mem + o_ids);
+  uint32_t *slots = reinterpret_cast<uint32_t *>(mem + o_slots), *cells = reinterpret_cast<uint32_t *>(mem + o_cells),
+           *work = reinterpret_cast<uint32_t *>(mem + o_work), *d_seg = work + 2;
   CT_HIP(hipMemcpyAsync(d_seg, seg.data(), 4 * seg.size(), hipMemcpyHostToDevice, st));
   const SegView sv{d_seg, d_seg + nseg + 1, nullptr, (uint32_t)nseg, n};
-  uint4 *bricks = S.grid_bricks.as<uint4>();
   hipLaunchKernelGGL(k_grid_clear, dim3(blocks(nrec)), dim3(kBlock), 0, st, bricks, nrec, work);
   hipLaunchKernelGGL(k_grid_mark, dim3(blocks(n)), dim3(kBlock), 0, st, sv, S.aabbs.as<ct_aabb>(), g,
-                     S.grid_bricks.as<uint32_t>(), S.grid_cells.as<uint32_t>(), work);
+                     reinterpret_cast<uint32_t *>(bricks), cells, work);
   hipLaunchKernelGGL(k_grid_link, dim3((uint32_t)nblk), dim3(64), 0, st, g, bricks, work);
   hipLaunchKernelGGL(k_grid_ids, dim3(blocks(n)), dim3(kBlock), 0, st, sv, d_seg + 2 * nseg + 1, bricks,
-                     S.grid_cells.as<uint32_t>(), S.grid_ids.as<uint2>(), S.grid_slots.as<uint32_t>());
+                     cells, d_ids, slots);
   CT_HIP(hipGetLastError());
   CT_HIP(hipMemcpyAsync(&flags, work, 4, hipMemcpyDeviceToHost, st));
   g.bricks = bricks;
-  g.ids = S.grid_ids.as<uint2>();
-  g.slots = S.grid_slots.as<uint32_t>();
-  g.cells = S.grid_cells.as<uint32_t>();
+  g.ids = d_ids;
+  g.slots = slots;
+  g.cells = cells;
   S.grid = g;
   return CT_OK;
 }

@@ -194,7 +194,7 @@ struct BvhSet {
   uint32_t prim_capacity = 0;
   uint32_t cube_light_count = 0;
   uint32_t cube_light_hw = 0;   // entries held: deleted lights leave stale records past the count
-  DevBuf grid_bricks, grid_ids, grid_slots, grid_cells, grid_work;
+  DevBuf grid_mem;              // the cell grid's arrays
   DGrid grid{};                 // bricks null: no grid
 };
 
@@ -285,9 +285,8 @@ struct Accel {
   DevBuf pt_mats;
   uint32_t pt_mat_count = 0;
   BuildScratch scratch;
-  std::mutex io_mu;                         // held by through_device, which uses the two below
+  std::mutex io_mu;                         // held by through_device, which uses io_dev
   DevBuf io_dev;
-  PinnedBuf io_host;
   PinnedBuf readback;                       // GPU deletions' slots on their way to the host mirror
   DevBuf upload;                            // packed slot records and remapping writes on their way in
   uint32_t status = CT_AS_IDLE;

@@ -13,54 +13,38 @@ using namespace ct;
 
 namespace ct {
 
-// The block and its pinned copy are kept between calls up to this size (a
-// larger call allocates and copies piece by piece, as its time is the copies').
-// 100 k rays through closest, bounce and any hit: 490, 880 and 640 us with an
-// allocation, a repacking loop on the host and a pageable copy per array, 200,
-// 430 and 155 us with one copy each way of the arrays as they are.
+// The block is kept between calls up to this size; a larger one is the call's
+// own.  The copies are pageable: pinned memory halves their time, but its
+// allocation and release (3 ms) would be paid by every accel, and one that is
+// built, asked once and closed is a usual one.
+// 100 k rays through closest, bounce and any hit took 490, 880 and 640 us with
+// an allocation and a repacking loop on the host per array.
 constexpr size_t kIoKeep = (size_t)64 << 20;
 
 int through_device(Accel &a, const std::vector<HostIn> &in, const std::vector<HostOut> &out,
                    const std::function<int(const std::vector<void *> &)> &launch) {
   std::vector<size_t> at;
-  size_t total = 0, in_bytes = 0;
+  size_t total = 0;
   auto place = [&](size_t bytes) {
     at.push_back(total);
     total += (bytes + 15) & ~(size_t)15;
   };
   for (const HostIn &i : in) place(i.bytes);
-  in_bytes = total;
   for (const HostOut &o : out) place(o.bytes);
   const std::lock_guard<std::mutex> lock(a.io_mu);
   DevBuf own;
-  const bool keep = total <= kIoKeep && a.io_host.reserve(total) == CT_OK;
-  DevBuf &dev = keep ? a.io_dev : own;
+  DevBuf &dev = total <= kIoKeep ? a.io_dev : own;
   int rc;
   if ((rc = dev.reserve(total))) return rc;
-  unsigned char *d = dev.as<unsigned char>(), *h = keep ? a.io_host.as<unsigned char>() : nullptr;
-  if (keep) {
-    for (size_t k = 0; k < in.size(); ++k) std::memcpy(h + at[k], in[k].p, in[k].bytes);
-    CT_HIP(hipMemcpyAsync(d, h, in_bytes, hipMemcpyHostToDevice, a.stream));
-  } else {
-    for (size_t k = 0; k < in.size(); ++k) CT_HIP(hipMemcpy(d + at[k], in[k].p, in[k].bytes, hipMemcpyHostToDevice));
-  }
   std::vector<void *> ptr;
-  for (size_t o : at) ptr.push_back(d + o);
+  for (size_t o : at) ptr.push_back(dev.as<unsigned char>() + o);
+  for (size_t k = 0; k < in.size(); ++k) CT_HIP(hipMemcpy(ptr[k], in[k].p, in[k].bytes, hipMemcpyHostToDevice));
   rc = launch(ptr);
-  if (!rc && keep) {
-    const hipError_t e = hipMemcpyAsync(h + in_bytes, d + in_bytes, total - in_bytes, hipMemcpyDeviceToHost, a.stream);
-    if (e != hipSuccess) rc = fail(CT_E_HIP, std::string("hipMemcpyAsync: ") + hipGetErrorString(e));
-  }
   const hipError_t e = hipStreamSynchronize(a.stream);  // the block is the next call's
   if (!rc && e != hipSuccess) rc = fail(CT_E_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
   if (rc) return rc;
-  for (size_t k = 0; k < out.size(); ++k) {
-    const size_t o = at[in.size() + k];
-    if (keep)
-      std::memcpy(out[k].p, h + o, out[k].bytes);
-    else
-      CT_HIP(hipMemcpy(out[k].p, d + o, out[k].bytes, hipMemcpyDeviceToHost));
-  }
+  for (size_t k = 0; k < out.size(); ++k)
+    CT_HIP(hipMemcpy(out[k].p, ptr[in.size() + k], out[k].bytes, hipMemcpyDeviceToHost));
   return CT_OK;
 }
 
