@@ -18,6 +18,7 @@
 
 #include "ct_device.h"
 #include "ct_internal.h"
+#include "grid_reach.h"
 
 namespace ct {
 
@@ -800,7 +801,9 @@ int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::
   const size_t nseg = ids.size();
   for (size_t q = 0; q < nseg; ++q) {
     const uint32_t id = ids[q];
-    if (std::memcmp(w, &a.w2o[16 * id], 16 * sizeof(float)) != 0) return CT_OK;
+    if (std::memcmp(w, &a.w2o[16 * id], 16 * sizeof(float)) != 0 ||
+        std::memcmp(a.instances[ids[0]].transform, a.instances[id].transform, 16 * sizeof(float)) != 0)
+      return CT_OK;
     for (int c = 0; c < 3; ++c) {
       lo[c] = std::fmin(lo[c], a.blas_root_box[6 * id + c]);
       hi[c] = std::fmax(hi[c], a.blas_root_box[6 * id + 3 + c]);
@@ -1052,6 +1055,7 @@ int build_tlas(Accel &a, hipStream_t st) {
   int rc;
   const std::vector<uint32_t> ids = used_ids(a);
   S.tlas_count = (uint32_t)ids.size();
+  for (int k = 0; k < 3; ++k) S.world_lo[k] = S.world_hi[k] = 0.0f;
   uint32_t dmax = 0;
   for (uint32_t id : ids) dmax = std::max(dmax, a.blas_depth[id]);
   S.blas_depth_max = dmax;
@@ -1080,6 +1084,8 @@ int build_tlas(Accel &a, hipStream_t st) {
       l[k] = wl[k] - kLeafPad;
       h[k] = wh[k] + kLeafPad;
       c[k] = (l[k] + h[k]) * 0.5f;
+      S.world_lo[k] = q ? std::fmin(S.world_lo[k], l[k]) : l[k];
+      S.world_hi[k] = q ? std::fmax(S.world_hi[k], h[k]) : h[k];
     }
     tc[q] = make_float4(c[0], c[1], c[2], 0.0f);
     tlo[q] = make_float4(l[0], l[1], l[2], 0.0f);
@@ -1219,6 +1225,11 @@ int commit(Accel &a, const Dirty &d) {
   if (!rc) rc = build_tlas(a, st);
   const hipError_t e = hipStreamSynchronize(st);  // grid_seg was read, grid_flags has arrived
   if (rc || e != hipSuccess || grid_flags) S.grid = DGrid{};
+  if (S.grid.bricks) {
+    const uint32_t id = used_ids(a)[0];
+    S.grid.max_o = world_reach(a.instances[id].transform, &a.w2o[16 * id], S.world_lo, S.world_hi);
+    if (!(S.grid.max_o > 0.0f)) S.grid = DGrid{};
+  }
   if (!rc && e != hipSuccess) return fail(CT_E_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
   return rc;
 }

@@ -467,6 +467,9 @@ int plan(Accel &a, const ct_adjoint_desc *d, const ct_adjoint_view *views, bool 
   CT_HIP(hipMemcpyAsync(P.blocks.p, hb.data(), sizeof(uint2) * hb.size(), hipMemcpyHostToDevice, st));
   P.nblocks = (uint32_t)hb.size();
   A.S = scene_view(a);
+  Reach from;
+  from.add(a.set.world_lo, a.set.world_hi);
+  for (uint32_t v = 0; v < d->n_views; ++v) keep_served(A.S.grid, from, views[v].inv_view);
   A.aabbs = a.set.aabbs.as<ct_aabb>();
   A.views = P.views.as<AView>();
   A.blocks = P.blocks.as<uint2>();

@@ -12,6 +12,7 @@
 #include <cstdint>
 
 #include "ct_internal.h"
+#include "grid_reach.h"
 
 namespace ct {
 namespace dev {
@@ -535,9 +536,16 @@ struct Walker {
 // cells on the fastest axis and iv the crossing times of a cell:
 //   walk:  (plane - q) * iv, then q + v T:         3 u T + u |q + v T|
 //   test:  ro - c, +-r, * inv, o + dr t:     6 u T + u max(iv) / 2 + 2 u
-// hence p = 10 u T + u (1.5 max|position| + max(iv) + 4).  Past 1/64 cell it
-// is cut off: there the BVH's own boxes (padded by 2^-12, 1/128 cell) do not
-// bound the test's rounding either.
+// hence p = 10 u T + u (1.5 max|position| + max(iv) + 4), cut off at 1/64
+// cell.  The term of iv may be cut: an error of u iv in the time a plane is
+// crossed at moves the ray by u along that plane's axis, so it is still
+// within p of the plane where the test places the crossing.  The other terms
+// may not, and where they pass 1/128 cell the BVH's boxes (padded by 2^-12)
+// do not bound the test's rounding either, so that what the BVH walk finds
+// depends on its boxes.  Rays from far away (about 200 units on) or through
+// as much of a grid are therefore walked through the BVH: ray queries look
+// at each ray (kChecked, kWalkQuery), frames and path tracing at the camera
+// and the scene, whose surfaces every other ray starts from (grid_reach.h).
 //
 // An empty box may be stepped over when neither its entry nor its exit lies
 // within p iv_a of a lattice plane of an axis other than the crossed one, a.
@@ -563,7 +571,8 @@ CT_D int32_t imin(int32_t a, int32_t b) { return a < b ? a : b; }
 CT_D int32_t imax(int32_t a, int32_t b) { return a > b ? a : b; }
 CT_D int32_t clampi(int32_t x, int32_t lo, int32_t hi) { return imax(imin(x, lo), imin(imax(x, lo), hi)); }
 
-template <int kMode>
+// kChecked: rays that this walk does not serve end as kWide.
+template <int kMode, bool kChecked = false>
 struct GridWalk {
   static constexpr bool kAny = kMode == kTraceAny;
   const DGrid &G;
@@ -624,7 +633,8 @@ struct GridWalk {
   }
 
   // The state of a walk between its steps.
-  static constexpr uint32_t kStepping = 0, kAtVoxel = 1, kEnded = 2, kNone = 3;  // kNone: no ray
+  // kNone: no ray; kWide: walk this ray through the BVH.
+  static constexpr uint32_t kStepping = 0, kAtVoxel = 1, kEnded = 2, kNone = 3, kWide = 4;
   uint32_t state;
   uint4 e;                       // the cell's brick, its index and the cell's bit in it
   uint32_t cell_base, cell_bit;
@@ -708,8 +718,15 @@ struct GridWalk {
     sg = f3(-gsign(dr.x), -gsign(dr.y), -gsign(dr.z));
     const float qmax = gmax(gmax(fabsf(oo.x), fabsf(oo.y)), fabsf(oo.z)) * kCellsPerUnit;
     const float dmax = gmax(gmax(fabsf(od.x), fabsf(od.y)), fabsf(od.z));
-    // A direction of zero length or with a term that is not finite, or an
-    // origin whose cells are not distinct floats, hits nothing.
+    if (kChecked) {
+      state = kWide;
+      // the times below are normal floats for these
+      if (!(gmax(gmax(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) <= G.max_o) || !(dmax > 1e-20f) ||
+          !((fabsf(od.x) + fabsf(od.y)) + fabsf(od.z) < 1e20f))
+        return;
+    }
+    // A direction of zero length or with a term that is not finite hits
+    // nothing.
     if (!(dmax > 0.0f) || !((fabsf(od.x) + fabsf(od.y)) + fabsf(od.z) < INFINITY) ||
         !((fabsf(oo.x) + fabsf(oo.y)) + fabsf(oo.z) < 1e9f))
       return;
@@ -738,10 +755,15 @@ struct GridWalk {
     const float tf = gmin(gmin(((float)(hx + 1) - qx) * ivx, ((float)(hy + 1) - qy) * ivy), ((float)(hz + 1) - qz) * ivz);
     t_unit = ldexpf(1.0f, ex + 5);  // T of one unit of t
     t_end = (kAny ? limit : best_t) * t_unit;
-    const float t = gmax(tn, 0.0f);
-    if (!(t <= tf) || t > t_end + kNearMax) return;
     const float gm = gmax(gmax(gmax(fabsf((float)l0x), fabsf((float)hx)), gmax(fabsf((float)l0y), fabsf((float)hy))),
                           gmax(fabsf((float)l0z), fabsf((float)hz)));
+    if (kChecked) {
+      const float last = t_end < tf ? t_end : tf;
+      if (!((10.0f * last + 1.5f * gmax(qmax, gm)) + 4.0f <= kWideMax)) return;
+      state = kEnded;
+    }
+    const float t = gmax(tn, 0.0f);
+    if (!(t <= tf) || t > t_end + kNearMax) return;
     k1 = kU * (1.5f * gmax(qmax, gm) + gmax(gmax(lx ? ivx : 0.0f, ly ? ivy : 0.0f), lz ? ivz : 0.0f) + 4.0f);
     t_in = t;
     const float px = __builtin_fmaf(vx, t, qx), py = __builtin_fmaf(vy, t, qy), pz = __builtin_fmaf(vz, t, qz);
@@ -862,8 +884,9 @@ CT_D void walk_stream(GridWalk<kMode> &w, Next next, Done done) {
 
 // How a kernel is built to walk: the BVH, the BVH with counters, or the cell
 // grid (scenes that have one; the counters are the BVH's, so counted
-// launches walk it).
-constexpr int kWalkBvh = 0, kWalkCount = 1, kWalkGrid = 2;
+// launches walk it), or the cell grid where it serves the ray and else the
+// BVH (queries of any rays).
+constexpr int kWalkBvh = 0, kWalkCount = 1, kWalkGrid = 2, kWalkQuery = 3;
 
 // The whole walk of one ray.  Returns true when an any-hit query is
 // occluded; a closest query leaves its hit in best_t/best_i/best_p (which
@@ -872,10 +895,13 @@ template <int kMode, int kWalk>
 CT_D bool traverse_mode(const DScene &S, F3 o, F3 d, float limit, uint32_t ti, uint32_t tp,
                         float &best_t, uint32_t &best_i, uint32_t &best_p, uint32_t *stk,
                         uint32_t stride, TraceCnt &cnt, bool &overflow) {
-  if constexpr (kWalk == kWalkGrid) {
-    GridWalk<kMode> w{S.grid};
+  if constexpr (kWalk == kWalkGrid || kWalk == kWalkQuery) {
+    using W = GridWalk<kMode, kWalk == kWalkQuery>;
+    W w{S.grid};
     w.start(S, o, d, kMode == kTraceAny ? limit : best_t, ti, tp);
     w.run();
+    if (kWalk == kWalkQuery && w.state == W::kWide)
+      return traverse_mode<kMode, kWalkBvh>(S, o, d, limit, ti, tp, best_t, best_i, best_p, stk, stride, cnt, overflow);
     if (kMode != kTraceAny && w.best != kInvalid) {
       const uint2 id = gld(S.grid.ids + w.best);
       best_t = w.best_t;

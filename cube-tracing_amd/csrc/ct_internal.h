@@ -99,6 +99,7 @@ struct DGrid {
   int32_t org[3];        // lattice cell of the grid's first cell, a multiple of 16
   uint32_t nblk[3];      // blocks per axis
   float w2o[12];         // world-to-object, shared by every instance (DInst::w2o)
+  float max_o;           // rays from world coordinates past this are not for this walk (world_reach)
 };
 
 struct DScene {
@@ -196,6 +197,7 @@ struct BvhSet {
   uint32_t cube_light_hw = 0;   // entries held: deleted lights leave stale records past the count
   DevBuf grid_mem;              // the cell grid's arrays
   DGrid grid{};                 // bricks null: no grid
+  float world_lo[3] = {0, 0, 0}, world_hi[3] = {0, 0, 0};  // the instances' padded world boxes (build_tlas)
 };
 
 // The scene as the frames before an update saw it: the traversable state
@@ -319,6 +321,18 @@ struct FrameBufs {
   bool pt_ready = false;     // allocated (and zeroed) on the first frame with indirect light
 };
 
+// A world box of ray origins.  It starts with the world's origin, where
+// records of pixels without a hit lie.
+struct Reach {
+  float lo[3] = {0.0f, 0.0f, 0.0f}, hi[3] = {0.0f, 0.0f, 0.0f};
+  void add(const float *l, const float *h) {
+    for (int k = 0; k < 3; ++k) {
+      lo[k] = !(lo[k] <= l[k]) ? l[k] : lo[k];
+      hi[k] = !(hi[k] >= h[k]) ? h[k] : hi[k];
+    }
+  }
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -342,6 +356,7 @@ struct Ctx {
   DevBuf frame_dev, blk_dev;    // the frame record and its block tables on the device
   uint32_t blk_key[4] = {0, 0, 0, 0};
   uint32_t blk_counts[3] = {0, 0, 0};
+  Reach reach;                  // the scenes this context has rendered since its reset
   const void *lights_accel = nullptr;  // accel and build whose cube lights were uploaded
   uint32_t lights_generation = 0;
   bool cube_plain = false;             // every uploaded cube light is of type CUBE and emits

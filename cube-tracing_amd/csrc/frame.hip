@@ -1826,6 +1826,8 @@ uint32_t retrace_resident() {
 // How a launch over a scene walks it: with counters (the BVH's) when they
 // are asked for, through the cell grid when the scene has one.
 int scene_walk(const DScene &s, bool counted) { return counted ? kWalkCount : (s.grid.bricks ? kWalkGrid : kWalkBvh); }
+// The same for any rays.
+int query_walk(const DScene &s, bool counted) { return counted ? kWalkCount : (s.grid.bricks ? kWalkQuery : kWalkBvh); }
 // Calls f with the walk as a compile-time constant.
 template <class F>
 void with_walk(int walk, F f) {
@@ -1836,11 +1838,20 @@ void with_walk(int walk, F f) {
   else
     f(std::integral_constant<int, kWalkBvh>{});
 }
+template <class F>
+void with_query_walk(int walk, F f) {
+  if (walk == kWalkQuery)
+    f(std::integral_constant<int, kWalkQuery>{});
+  else if (walk == kWalkCount)
+    f(std::integral_constant<int, kWalkCount>{});
+  else
+    f(std::integral_constant<int, kWalkBvh>{});
+}
 
 }  // namespace
 
 int launch_trace_any(const DScene &s, const TraceAnyArgs &a, hipStream_t st) {
-  with_walk(scene_walk(s, a.stats != nullptr), [&](auto w) {
+  with_query_walk(query_walk(s, a.stats != nullptr), [&](auto w) {
     constexpr int kWalk = decltype(w)::value;
     const uint32_t grid = std::min<uint32_t>(std::max<uint32_t>(nblocks(a.n), 1), any_single_resident<kWalk>());
     hipLaunchKernelGGL(k_trace_any<kWalk>, dim3(grid), dim3(kBlock), 0, st, s, a);
@@ -1851,7 +1862,7 @@ int launch_trace_any(const DScene &s, const TraceAnyArgs &a, hipStream_t st) {
 
 int launch_trace_closest(const DScene &s, const TraceClosestArgs &a, hipStream_t st) {
   if (a.n == 0) return CT_OK;
-  with_walk(scene_walk(s, a.stats != nullptr), [&](auto w) {
+  with_query_walk(query_walk(s, a.stats != nullptr), [&](auto w) {
     hipLaunchKernelGGL(k_trace_closest<decltype(w)::value>, dim3(nblocks(a.n)), dim3(kBlock), 0, st, s, a);
   });
   CT_HIP(hipGetLastError());
@@ -2072,6 +2083,9 @@ int prepare_frame(Ctx *c, Accel *a, const ct_frame_params *p, hipStream_t st, DF
   F.cfg = c->cfg;
   F.cfg.cube_light_count = ncube;  // the manager owns this count (accel_struct_mngr.cpp:2580)
   F.S = scene_view(*a);
+  // Rays start at the camera and at hits of this frame and of earlier ones.
+  c->reach.add(a->set.world_lo, a->set.world_hi);
+  keep_served(F.S.grid, c->reach, p->inv_view);
   F.prev_set = ((p->is_active & CT_REMAP_BIT) && previous_distinct(*a)) ? 1u : 0u;
   F.Sp = F.prev_set ? previous_scene_view(*a) : F.S;
   F.aabbs = a->set.aabbs.as<ct_aabb>();
@@ -2517,6 +2531,7 @@ int ct_ctx_reset(ct_ctx *c, void *stream) {
   CT_HIP(hipSetDevice(c->device));
   hipStream_t st = stream ? static_cast<hipStream_t>(stream) : c->stream;
   c->cur = 1;
+  c->reach = Reach{};
   return zero_frame(*c, st);
 }
 
@@ -3110,7 +3125,7 @@ int ct_trace_bounce(ct_accel *a, uint32_t n, const float *origins, const float *
     F.aabbs = a->set.aabbs.as<ct_aabb>();
     F.prims = a->set.prims.as<ct_primitive>();
     F.n_mats = 0;  // materials live in a frame context; the records here carry indices only
-    with_walk(scene_walk(F.S, stats != nullptr), [&](auto w) {
+    with_query_walk(query_walk(F.S, stats != nullptr), [&](auto w) {
       hipLaunchKernelGGL(k_trace_bounce<decltype(w)::value>, dim3(nblocks(n)), dim3(kBlock), 0, a->stream, F, A, cnt);
     });
     CT_HIP(hipGetLastError());

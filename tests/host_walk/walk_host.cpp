@@ -1,8 +1,10 @@
 // Host build of the cell-grid walk (csrc/ct_device.h), called through ctypes:
 // each ray by the walk and by the voxel test on every voxel, with the same
-// voxel test on the same operands.
+// voxel test on the same operands, or by the walk of ray queries and by the
+// BVH walk; and the rays each walk may take (csrc/grid_reach.h).
 #include "../../cube-tracing_amd/csrc/ct_device.h"
 
+#include <type_traits>
 #include <vector>
 
 namespace ct {
@@ -19,8 +21,43 @@ struct Scene {
   std::vector<float> boxes;
   std::vector<uint32_t> cells;
   std::vector<DInst> inst;
+  std::vector<DNode> nodes;
+  std::vector<float4> leaves;
+  uint32_t tlas_inst = 0;
   DScene S{};
 };
+
+// A BVH of the leaves [a, b), split at the median of the longest axis;
+// returns the ref of its root (an internal node's index is its split's).
+uint32_t build_bvh(Scene &sc, uint32_t a, uint32_t b, float *lo, float *hi) {
+  auto axis = [](const float4 &v, int k) { return k == 0 ? v.x : (k == 1 ? v.y : v.z); };
+  for (int k = 0; k < 3; ++k) {
+    lo[k] = hi[k] = axis(sc.leaves[a], k);
+    for (uint32_t i = a; i < b; ++i) {
+      lo[k] = std::min(lo[k], axis(sc.leaves[i], k));
+      hi[k] = std::max(hi[k], axis(sc.leaves[i], k));
+    }
+  }
+  int k = 0;
+  for (int c = 1; c < 3; ++c)
+    if (hi[c] - lo[c] > hi[k] - lo[k]) k = c;
+  for (int c = 0; c < 3; ++c) {
+    lo[c] -= kHalfVoxel + kLeafPad;
+    hi[c] += kHalfVoxel + kLeafPad;
+  }
+  if (b - a == 1) return kLeaf | a;
+  const uint32_t m = (a + b) / 2;
+  std::nth_element(sc.leaves.begin() + a, sc.leaves.begin() + m, sc.leaves.begin() + b,
+                   [&](const float4 &p, const float4 &q) { return axis(p, k) < axis(q, k); });
+  float l[6], h[6];
+  const uint32_t c0 = build_bvh(sc, a, m, l, h), c1 = build_bvh(sc, m, b, l + 3, h + 3);
+  DNode &n = sc.nodes[m];
+  n.a = float4{l[0], l[1], l[2], h[0]};
+  n.b = float4{h[1], h[2], l[3], l[4]};
+  n.c = float4{l[5], h[3], h[4], h[5]};
+  n.d = uint4{c0, c1, 0u, 0u};
+  return m;
+}
 
 // cells [n][3] of one instance's voxels (object space lattice), each once
 void build(Scene &sc, const int32_t *cells, uint32_t n, const float *w2o) {
@@ -103,6 +140,18 @@ void build(Scene &sc, const int32_t *cells, uint32_t n, const float *w2o) {
   sc.inst[0].count = n;
   sc.S.inst = sc.inst.data();
   sc.S.n_inst = 1;
+  for (uint32_t i = 0; i < n; ++i) {
+    const float *b = &sc.boxes[6 * (size_t)i];
+    sc.leaves.push_back(float4{(b[0] + b[3]) * 0.5f, (b[1] + b[4]) * 0.5f, (b[2] + b[5]) * 0.5f, __uint_as_float(i)});
+  }
+  sc.nodes.resize(n);
+  float lo3[3], hi3[3];
+  sc.inst[0].root = build_bvh(sc, 0, n, lo3, hi3);
+  sc.S.blas_nodes = sc.nodes.data();
+  sc.S.blas_leaves = sc.leaves.data();
+  sc.S.tlas_inst = &sc.tlas_inst;
+  sc.S.tlas_root = kLeaf;
+  G.max_o = INFINITY;
   G.bricks = sc.bricks.data();
   G.ids = sc.ids.data();
   G.cells = sc.cells.data();
@@ -160,7 +209,56 @@ void both(const Scene &sc, const int32_t *cells, uint32_t n, F3 o, F3 d, float l
   *id_ref = kMode == kTraceAny ? hit_any : rp;
 }
 
+// A ray query's walk against the BVH walk; whether the query took the BVH.
+template <int kMode>
+bool query(const Scene &sc, F3 o, F3 d, float limit, uint32_t target, float *t_out, uint32_t *id_out, float *t_ref,
+           uint32_t *id_ref) {
+  const uint32_t ti = target == kInvalid ? kInvalid : 0u;
+  auto one = [&](auto walk, float *t, uint32_t *id) {
+    uint32_t stk[kStackLds], bi = kInvalid, bp = kInvalid;
+    float bt = limit;
+    TraceCnt cnt;
+    bool ovf = false;
+    const bool occ = traverse_mode<kMode, decltype(walk)::value>(sc.S, o, d, limit, ti, target, bt, bi, bp, stk, 1u, cnt, ovf);
+    *t = kMode == kTraceAny || bp == kInvalid ? 0.0f : bt;
+    *id = kMode == kTraceAny ? (uint32_t)occ : bp;
+    if (ovf) *id = kInvalid - 1u;
+  };
+  one(std::integral_constant<int, kWalkQuery>{}, t_out, id_out);
+  one(std::integral_constant<int, kWalkBvh>{}, t_ref, id_ref);
+  GridWalk<kMode, true> w{sc.S.grid};
+  w.start(sc.S, o, d, limit, ti, target);
+  return w.state == GridWalk<kMode, true>::kWide;
+}
+
 }  // namespace
+
+extern "C" void query_and_bvh(const int32_t *cells, uint32_t n, const float *w2o, int mode, uint32_t rays, const float *o,
+                              const float *d, const float *limit, const uint32_t *target, float *t_out, uint32_t *id_out,
+                              float *t_ref, uint32_t *id_ref, uint8_t *wide) {
+  Scene sc;
+  build(sc, cells, n, w2o);
+#pragma omp parallel for schedule(dynamic, 64)
+  for (uint32_t i = 0; i < rays; ++i) {
+    const F3 ro = f3(o[3 * i], o[3 * i + 1], o[3 * i + 2]), rd = f3(d[3 * i], d[3 * i + 1], d[3 * i + 2]);
+    auto fn = mode == kTraceAny ? query<kTraceAny> : mode == kTraceClosest ? query<kTraceClosest> : query<kTraceBounce>;
+    wide[i] = fn(sc, ro, rd, limit[i], target[i], t_out + i, id_out + i, t_ref + i, id_ref + i);
+  }
+}
+
+extern "C" float reach_of(const float *m, const float *w, const float *lo, const float *hi) { return world_reach(m, w, lo, hi); }
+
+// Whether a scene's grid stays for rays from its surfaces and a camera.
+extern "C" int served(const int32_t *cells, uint32_t n, const float *w2o, float max_o, const float *lo, const float *hi,
+                      const float *inv_view) {
+  Scene sc;
+  build(sc, cells, n, w2o);
+  sc.S.grid.max_o = max_o;
+  Reach from;
+  from.add(lo, hi);
+  keep_served(sc.S.grid, from, inv_view);
+  return sc.S.grid.bricks != nullptr;
+}
 
 extern "C" void walk_and_brute(const int32_t *cells, uint32_t n, const float *w2o, int mode, uint32_t rays,
                                const float *o, const float *d, const float *limit, const uint32_t *target, float *t_out,

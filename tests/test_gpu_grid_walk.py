@@ -112,3 +112,55 @@ def test_grid_under_one_transform(gpu):
     m = np.array([[c, 0, -s, 0], [0, 1, 0, 0], [s, 0, c, 0], [0.1, -0.2, 0.05, 1]], np.float32)
     ctamd.load_scene(sc, acc, ctx, transform=m.reshape(16))
     _same(acc, sc, 9)
+
+
+def test_far_rays_take_the_bvh(gpu):
+    """Rays from up to 10^10 units away, of odd lengths and not finite: the
+    counted walk's hits, to the bit (the grid's own differ from about 5600
+    units on)."""
+    sc, acc = _load(16, 16, 0.4)
+    rng = np.random.default_rng(4)
+    n = 200000
+    lo, hi = sc.grid_min.astype(np.float64), sc.grid_max.astype(np.float64)
+    for far in (300.0, 2e4, 1e6, 3e9):
+        d = rng.normal(size=(n, 3))
+        d /= np.linalg.norm(d, axis=1, keepdims=True)
+        o = np.ascontiguousarray(rng.uniform(lo, hi, (n, 3)) - d * far, np.float32)
+        d = np.ascontiguousarray(d * np.where(rng.random((n, 1)) < 0.1, 10.0 ** rng.uniform(-30, 30, (n, 1)), 1), np.float32)
+        d[:40] = rng.choice(np.array([0, -0.0, np.inf, np.nan, 1, 1e-42, 1e38], np.float32), size=(40, 3))
+        o[20:40] = rng.choice(np.array([0, np.inf, np.nan, 0.25, 1e38], np.float32), size=(20, 3))
+        t, ids = acc.trace_closest(o, d, tmax=1e30)
+        bt, bids, _ = acc.trace_closest(o, d, tmax=1e30, stats=True)
+        assert np.array_equal(ids, bids) and np.array_equal(t.view(np.uint32), bt.view(np.uint32))
+        g, b = acc.trace_bounce(o, d), acc.trace_bounce(o, d, stats=True)
+        for k in ("ids", "pos", "nrm", "dist", "wo"):
+            assert np.array_equal(g[k].view(np.uint32), b[k].view(np.uint32)), k
+        dist = np.full(n, np.float32(far * 1.5))
+        occ, (bocc, _) = acc.trace_any(o, d, dist, ids), acc.trace_any(o, d, dist, ids, stats=True)
+        assert np.array_equal(occ, bocc)
+
+
+@pytest.mark.parametrize("far", [12.0, 2e4])
+def test_frames_of_far_cameras(gpu, far):
+    """Frames from a camera far outside the scene: the bits of frames that walk
+    the BVH (instrumented ones)."""
+    w = ctamd.hd_di(width=160, height=96, grid=32, chunk=16)
+    scenes = [ctamd.Scene(ctamd.scene_desc(w)) for _ in range(2)]
+    lo, hi = scenes[0].grid_min.astype(np.float64), scenes[0].grid_max.astype(np.float64)
+    eye = (lo + hi) / 2 + far * np.array([0.6, 0.0, 0.8])
+    w.camera = lambda f: (tuple(eye.tolist()), (-0.6, 0.0, -0.8), (0.0, 1.0, 0.0))
+    w.fov_radians = 1.2 * float((hi - lo).max()) / far
+    images = []
+    for k in range(2):
+        sc = scenes[k]
+        acc = ctamd.Accel(max_instances=sc.info.instance_count + 8,
+                          max_primitives=sc.info.primitive_count + 32 * sc.info.instance_count + 1024,
+                          max_cube_lights=sc.info.cube_light_count + 8)
+        ctx = ctamd.Ctx(w.width, w.height)
+        ctamd.load_scene(sc, acc, ctx)
+        ctx.set_instrumentation(2 if k else 0)
+        for f in range(2):
+            ctx.render(acc, ctamd.frame_params(w, f))
+        images.append((ctx.read(ctamd.CT_BUF_IMAGE, w.width, w.height), bytes(ctx.read(ctamd.CT_BUF_DI, w.width, w.height))))
+    assert np.array_equal(images[0][0].view(np.uint32), images[1][0].view(np.uint32))
+    assert images[0][1] == images[1][1]

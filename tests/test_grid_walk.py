@@ -1,6 +1,8 @@
 """The cell-grid walk (csrc/ct_device.h, GridWalk), built for the host, against
 the voxel test on every voxel: the same hits to the bit, whatever the rays do
-at the lattice's planes, edges and corners."""
+at the lattice's planes, edges and corners.  Rays the walk does not serve (from
+far away, of odd lengths, not finite) are walked through the BVH: a ray query
+gets the BVH walk's hit whatever the ray."""
 import ctypes as C
 import os
 import shutil
@@ -109,3 +111,112 @@ def test_rays_that_hit_nothing(walk):
         bad, ref = _both(walk, cells, IDENTITY, mode, o, d, limit, target)
         assert not bad.any()
         assert (ref == (0 if mode == 0 else NONE)).all()
+
+
+# origins up to 10^10 units away, where the grid walk's own hits differ from the
+# BVH walk's at a few rays in 10^4 from about 5600 units on; a long grid,
+# where the distance within it counts
+@pytest.mark.parametrize("far", [30.0, 400.0, 5000.0, 2e4, 1e6, 3e9, 1e10])
+@pytest.mark.parametrize("n,org", [(16, (0, 0, 0)), (12, (6000, -9000, 14000)), (0, (0, 0, 0))])
+def test_queries_equal_the_bvh_walk(walk, far, n, org):
+    rng = np.random.default_rng(int(far) % 1000 + n)
+    if n:
+        cells = np.argwhere(rng.random((n, n, n)) < 0.4) + np.array(org)
+    else:
+        cells = np.unique(rng.integers(0, 12, (3000, 3)) * [1, 1, 900], axis=0)
+    cells, rays = np.ascontiguousarray(cells, np.int32), 20000
+    lo, hi = cells.min(0) / 32.0, (cells.max(0) + 1) / 32.0
+    d = rng.normal(size=(rays, 3))
+    d[::5] = rng.choice([-1.0, 0.0, 1.0, 1e-6], size=(len(d[::5]), 3))
+    d[np.abs(d).sum(1) == 0] = [1, 0, 0]
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    to = cells[rng.integers(0, len(cells), rays)] / 32.0 + rng.uniform(0, 1 / 32.0, (rays, 3))
+    o = np.ascontiguousarray(to - d * far * rng.uniform(0.5, 1.0, (rays, 1)), np.float32)
+    d = np.ascontiguousarray(d * np.where(rng.random((rays, 1)) < 0.1, 10.0 ** rng.uniform(-35, 35, (rays, 1)), 1), np.float32)
+    odd = slice(0, 40)
+    d[odd] = rng.choice(np.array([0, -0.0, np.inf, -np.inf, np.nan, 1, 1e-42, 1e38], np.float32), size=(40, 3))
+    o[20:40] = rng.choice(np.array([0, np.inf, np.nan, 0.25, 1e38], np.float32), size=(20, 3))
+    for mode in (0, 1, 2):
+        limit, target = np.full(rays, 1e30, np.float32), np.full(rays, NONE, np.uint32)
+        limit[::11] = np.inf
+        if mode == 0:
+            limit[::2] = (far * rng.uniform(0.4, 1.2, len(limit[::2]))).astype(np.float32)
+            target[::3] = rng.integers(0, len(cells), len(target[::3]))
+        t, i, tr, ir = (np.zeros(rays, k) for k in (np.float32, np.uint32, np.float32, np.uint32))
+        wide = np.zeros(rays, np.uint8)
+        walk.query_and_bvh(_p(cells), len(cells), _p(IDENTITY), mode, rays, _p(o), _p(d), _p(limit), _p(target), _p(t),
+                           _p(i), _p(tr), _p(ir), _p(wide))
+        bad = (i != ir) | (t.view(np.uint32) != tr.view(np.uint32))
+        assert not bad.any(), (mode, int(bad.sum()), o[bad][:3], d[bad][:3])
+        if n == 16 and far == 30.0:  # ordinary rays stay in the grid
+            assert wide[40:].mean() < 0.1
+        if far >= 2e4:
+            assert wide.mean() > 0.9
+
+
+def _m44(rot, t):
+    m = np.eye(4, dtype=np.float64)
+    m[:3, :3], m[:3, 3] = rot, t
+    return m
+
+
+def _colmajor(m):
+    return np.ascontiguousarray(m.T.reshape(16), np.float32)
+
+
+def test_reach_of_transforms(walk):
+    """How far from the world's origin rays may start: anywhere under the
+    identity, nearer the further the instances lie, nowhere when the two
+    matrices are not each other's inverses."""
+    walk.reach_of.restype = C.c_float
+    lo, hi = np.full(3, -4, np.float32), np.full(3, 4, np.float32)
+
+    def reach(m, w=None):
+        w = np.linalg.inv(m.astype(np.float32).astype(np.float64)) if w is None else w
+        return walk.reach_of(_p(_colmajor(m)), _p(_colmajor(w)), _p(lo), _p(hi))
+
+    rng = np.random.default_rng(3)
+    q = np.linalg.qr(rng.normal(size=(3, 3)))[0]
+    eye = np.eye(3)
+    assert reach(_m44(eye, 0)) == np.inf
+    near, far = reach(_m44(eye, [3, 0, 0])), reach(_m44(eye, [60, -20, 7]))
+    assert 20 < far < near < 215
+    assert 20 < reach(_m44(q, [0.1, 0, 0])) < 215
+    assert 20 < reach(_m44(q * 3.0, 0)) < 215
+    assert reach(_m44(eye, [500, 0, 0])) == 0.0
+    assert reach(_m44(q, 0), _m44(eye, 0)) == 0.0
+    assert reach(_m44(eye, 0), _m44(eye, [1e-3, 0, 0])) == 0.0
+    assert reach(_m44(eye * 0.0, 0), _m44(eye * 0.0, 0)) == 0.0
+    assert reach(_m44(q * 1e12, 0)) == 0.0
+    p = _m44(eye, 0)
+    p[3, 0] = 0.1
+    assert reach(p) == 0.0
+    assert reach(_m44(eye, [np.nan, 0, 0]), _m44(eye, 0)) == 0.0
+
+
+def test_served_cameras_have_no_wide_ray(walk):
+    """A grid that a frame keeps serves every ray from its camera and its
+    scene; far and odd cameras lose it."""
+    rng = np.random.default_rng(11)
+    cells = np.ascontiguousarray(np.argwhere(rng.random((24, 24, 24)) < 0.2) + [-12, 5, 3000], np.int32)
+    lo, hi = (cells.min(0) / 32.0).astype(np.float32), ((cells.max(0) + 1) / 32.0).astype(np.float32)
+    kept = []
+    for dist in (0.0, 1.0, 30.0, 80.0, 150.0, 300.0, 1e4, 1e9, np.inf, np.nan):
+        for scale in (1.0, 1e-12, 1e12, 0.0, np.nan):
+            rot = np.linalg.qr(rng.normal(size=(3, 3)))[0] * scale
+            eye = (lo + hi) / 2 + np.array([dist, 0, 0])
+            view = _colmajor(_m44(rot, eye))
+            if walk.served(_p(cells), len(cells), _p(IDENTITY), C.c_float(np.inf), _p(lo), _p(hi), _p(view)):
+                kept.append((dist, scale))
+                n = 3000
+                o = np.where(rng.random((n, 1)) < 0.5, eye, rng.uniform(lo, hi, (n, 3)))
+                o, d = np.ascontiguousarray(o, np.float32), np.ascontiguousarray(rng.normal(size=(n, 3)), np.float32)
+                out = [np.zeros(n, k) for k in (np.float32, np.uint32, np.float32, np.uint32, np.uint8)]
+                limit, target = np.full(n, 1e9, np.float32), np.full(n, NONE, np.uint32)
+                walk.query_and_bvh(_p(cells), len(cells), _p(IDENTITY), 1, n, _p(o), _p(d), _p(limit), _p(target),
+                                   *(_p(x) for x in out))
+                assert not out[4].any(), (dist, scale, o[out[4] > 0][:3], d[out[4] > 0][:3])
+    assert {(k, 1.0) for k in (0.0, 1.0, 30.0)} <= set(kept)
+    assert all(k[0] < 300 and k[1] == 1.0 for k in kept)
+    view = _colmajor(_m44(np.array([[1, 1, 0], [0, 1e-6, 0], [0, 0, 1]]), (lo + hi) / 2))
+    assert not walk.served(_p(cells), len(cells), _p(IDENTITY), C.c_float(np.inf), _p(lo), _p(hi), _p(view))
