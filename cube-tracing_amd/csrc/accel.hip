@@ -1234,6 +1234,11 @@ int commit(Accel &a, const Dirty &d) {
   return rc;
 }
 
+bool recording(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
 int device_count_gfx950() {
   int n = 0;
   if (hipGetDeviceCount(&n) != hipSuccess) return 0;

@@ -385,6 +385,10 @@ struct Ctx {
 
 // Kernel-side views used by trace.hip and frame.hip.
 DScene scene_view(const Accel &a);
+// Whether work enqueued on `st` is recorded for replays, which may follow
+// updates of the scene.  An update in place keeps the BVH's arrays where they
+// are, but not the cell grid's: recorded launches walk the BVH.
+bool recording(hipStream_t st);
 // The previous set's traversal view while SETTLING (else the current one).
 DScene previous_scene_view(const Accel &a);
 bool previous_distinct(const Accel &a);

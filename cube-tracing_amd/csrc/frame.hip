@@ -2086,6 +2086,7 @@ int prepare_frame(Ctx *c, Accel *a, const ct_frame_params *p, hipStream_t st, DF
   // Rays start at the camera and at hits of this frame and of earlier ones.
   c->reach.add(a->set.world_lo, a->set.world_hi);
   keep_served(F.S.grid, c->reach, p->inv_view);
+  if (recording(st)) F.S.grid.bricks = nullptr;
   F.prev_set = ((p->is_active & CT_REMAP_BIT) && previous_distinct(*a)) ? 1u : 0u;
   F.Sp = F.prev_set ? previous_scene_view(*a) : F.S;
   F.aabbs = a->set.aabbs.as<ct_aabb>();

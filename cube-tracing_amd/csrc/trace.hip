@@ -79,7 +79,9 @@ int ct_trace_any_noalloc(ct_accel *a, uint32_t n, const float *origins, const fl
   CT_HIP(hipSetDevice(a->device));
   hipStream_t st = stream ? static_cast<hipStream_t>(stream) : a->stream;
   const TraceAnyArgs t{origins, directions, distances, targets, occluded_out, nullptr, n};
-  return launch_trace_any(scene_view(*a), t, st);
+  DScene s = scene_view(*a);
+  if (recording(st)) s.grid.bricks = nullptr;
+  return launch_trace_any(s, t, st);
 }
 
 int ct_trace_closest(ct_accel *a, uint32_t n, const float *origins, const float *directions, float tmax,

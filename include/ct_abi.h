@@ -415,7 +415,10 @@ int ct_trace_any(ct_accel *accel, uint32_t n, const float *origins,
  * capture, tight serving loops).  Same rays, same result bytes as
  * ct_trace_any, but every array is in DEVICE memory and the call is only
  * enqueued on `stream` (null: the accel's stream); nothing is copied back
- * and nothing is waited for.  n is at most 2^20 (CT_E_CAPACITY above). */
+ * and nothing is waited for.  n is at most 2^20 (CT_E_CAPACITY above).  A
+ * captured call walks the BVH, so its replays follow the updates that keep
+ * the accel's arrays in place (deletions, refits, rebuilt BLAS); capture it
+ * again after instances or more primitives than ever before are added. */
 int ct_trace_any_noalloc(ct_accel *accel, uint32_t n, const float *origins,
                          const float *directions, const float *distances,
                          const uint32_t *targets, uint8_t *occluded_out,
