@@ -266,6 +266,12 @@ CT_D F3 random_cosine_direction(uint32_t &seed, F3 n) {
 }
 
 
+// A strided loop's next index below `count`, else `count`: base + stride may
+// pass 2^32, and a wrapped index would start the loop again.
+CT_D uint32_t next_batch(uint32_t base, uint32_t count, uint32_t stride) {
+  return count - base > stride ? base + stride : count;
+}
+
 // ------------------------------------------------------------ traversal
 constexpr uint32_t kMaxTraversalSteps = 1u << 22;
 

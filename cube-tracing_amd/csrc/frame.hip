@@ -1326,7 +1326,7 @@ struct RayBatches {
     base = (blockIdx.x * (kBlock / 64u) + (threadIdx.x >> 6)) * 64u;
   }
   CT_D bool valid() const { return base < count; }
-  CT_D void next() { base += stride; }
+  CT_D void next() { base = next_batch(base, count, stride); }
 };
 
 // Closest voxel of each queued path segment (intersect() semantics), one

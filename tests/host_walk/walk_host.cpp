@@ -246,6 +246,14 @@ extern "C" void query_and_bvh(const int32_t *cells, uint32_t n, const float *w2o
   }
 }
 
+// Batches a wave takes, from `base` on (at most `most`, so that a loop without
+// an end shows).
+extern "C" uint32_t batches(uint32_t base, uint32_t count, uint32_t stride, uint32_t most) {
+  uint32_t n = 0;
+  for (; base < count && n < most; base = next_batch(base, count, stride)) ++n;
+  return n;
+}
+
 extern "C" float reach_of(const float *m, const float *w, const float *lo, const float *hi) { return world_reach(m, w, lo, hi); }
 
 // Whether a scene's grid stays for rays from its surfaces and a camera.

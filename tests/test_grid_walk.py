@@ -220,3 +220,11 @@ def test_served_cameras_have_no_wide_ray(walk):
     assert all(k[0] < 300 and k[1] == 1.0 for k in kept)
     view = _colmajor(_m44(np.array([[1, 1, 0], [0, 1e-6, 0], [0, 0, 1]]), (lo + hi) / 2))
     assert not walk.served(_p(cells), len(cells), _p(IDENTITY), C.c_float(np.inf), _p(lo), _p(hi), _p(view))
+
+
+@pytest.mark.parametrize("count", [0, 1, 64, 65, 2097152, 2097153, 1 << 31, (1 << 32) - 2097152, (1 << 32) - 1])
+def test_strided_batches_end(walk, count):
+    stride = 2097152  # 64 rays for each wave of a full grid
+    for base in (0, 64, stride - 64):
+        want = 0 if base >= count else -(-(count - base) // stride)
+        assert walk.batches(base, C.c_uint32(count), stride, 10000) == want
