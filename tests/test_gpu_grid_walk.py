@@ -144,11 +144,11 @@ def test_far_rays_take_the_bvh(gpu):
 def test_frames_of_far_cameras(gpu, far):
     """Frames from a camera far outside the scene: the bits of frames that walk
     the BVH (instrumented ones)."""
-    w = ctamd.hd_di(width=160, height=96, grid=32, chunk=16)
+    w = ctamd.hd_di(width=640, height=360, grid=32, chunk=16)
     scenes = [ctamd.Scene(ctamd.scene_desc(w)) for _ in range(2)]
     lo, hi = scenes[0].grid_min.astype(np.float64), scenes[0].grid_max.astype(np.float64)
-    eye = (lo + hi) / 2 + far * np.array([0.6, 0.0, 0.8])
-    w.camera = lambda f: (tuple(eye.tolist()), (-0.6, 0.0, -0.8), (0.0, 1.0, 0.0))
+    eye = (lo + hi) / 2 + far * np.array([0.48, 0.6, 0.64])
+    w.camera = lambda f: (tuple(eye.tolist()), (-0.48, -0.6, -0.64), (0.0, 1.0, 0.0))
     w.fov_radians = 1.2 * float((hi - lo).max()) / far
     images = []
     for k in range(2):
