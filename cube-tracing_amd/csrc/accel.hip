@@ -786,8 +786,9 @@ __global__ void __launch_bounds__(kBlock) k_grid_ids(SegView sv, const uint32_t 
 
 // Builds the scene's cell grid (DGrid) when it can have one: every instance
 // has the same transform, every voxel is a cell of the 2^-5 lattice, no cell
-// holds two voxels, and the bricks of the bounding box are few against the
-// voxels (16 B a brick against about 130 B a voxel for the BVH).  Enqueued
+// holds two voxels, the bricks of the bounding box are few against the
+// voxels (16 B a brick against about 130 B a voxel for the BVH), and there is
+// memory for it.  Enqueued
 // on `st`, which reads `seg` and writes `flags`: once it has drained, the
 // caller drops the grid if `flags` is not zero.
 int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::vector<uint32_t> &seg, uint32_t &flags) {
@@ -838,8 +839,7 @@ int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::
   };
   const size_t o_bricks = place(16 * (size_t)nrec), o_ids = place(8 * (size_t)n), o_slots = place(4 * (size_t)n),
                o_cells = place(4 * (size_t)S.prim_capacity), o_work = place(8 + 4 * seg.size());
-  int rc;
-  if ((rc = S.grid_mem.reserve(total))) return rc;
+  if (!reserve_optional(S.grid_mem, total)) return CT_OK;
   unsigned char *mem = S.grid_mem.as<unsigned char>();
   uint4 *bricks = reinterpret_cast<uint4 *>(mem + o_bricks);
   uint2 *d_ids = reinterpret_cast<uint2 *>(mem + o_ids);

@@ -142,6 +142,14 @@ struct DevBuf {
   template <class T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Memory for what a scene can do without: false when it is refused, with no
+// error left behind in the runtime, where the next launch would find it.
+inline bool reserve_optional(DevBuf &b, size_t n) {
+  if (b.reserve(n) == CT_OK) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Pinned host memory (hipHostMalloc) with RAII: device-to-host copies into
 // it run at the link's rate, where pageable memory is staged by the runtime.
 struct PinnedBuf {

@@ -27,7 +27,13 @@ using std::isnan;
 typedef void *hipStream_t, *hipEvent_t;
 typedef int hipError_t;
 constexpr int hipSuccess = 0, hipHostMallocDefault = 0;
-inline hipError_t hipMalloc(void **, size_t) { return 1; }
+inline hipError_t hip_last_error = hipSuccess;  // hipMalloc refuses every request
+inline hipError_t hipMalloc(void **, size_t) { return hip_last_error = 2; }
+inline hipError_t hipGetLastError() {
+  const hipError_t e = hip_last_error;
+  hip_last_error = hipSuccess;
+  return e;
+}
 inline hipError_t hipFree(void *) { return 0; }
 inline hipError_t hipHostMalloc(void **, size_t, int) { return 1; }
 inline hipError_t hipHostFree(void *) { return 0; }

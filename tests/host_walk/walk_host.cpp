@@ -246,6 +246,13 @@ extern "C" void query_and_bvh(const int32_t *cells, uint32_t n, const float *w2o
   }
 }
 
+// Memory a scene can do without, refused: no buffer and no error left (0).
+extern "C" int refused_memory() {
+  DevBuf b;
+  const bool got = reserve_optional(b, (size_t)1 << 30);
+  return (got ? 1 : 0) | (b.p ? 2 : 0) | (b.bytes ? 4 : 0) | (hipGetLastError() != hipSuccess ? 8 : 0);
+}
+
 // Batches a wave takes, from `base` on (at most `most`, so that a loop without
 // an end shows).
 extern "C" uint32_t batches(uint32_t base, uint32_t count, uint32_t stride, uint32_t most) {

@@ -228,3 +228,10 @@ def test_strided_batches_end(walk, count):
     for base in (0, 64, stride - 64):
         want = 0 if base >= count else -(-(count - base) // stride)
         assert walk.batches(base, C.c_uint32(count), stride, 10000) == want
+
+
+def test_refused_grid_memory_leaves_no_error(walk):
+    """Without memory for its grid a scene is built all the same (and walked
+    through its BVH); the runtime's error state must be clear for the
+    launches that follow."""
+    assert walk.refused_memory() == 0
