@@ -1,4 +1,5 @@
-"""Scenes that keep the BVH (two transforms, so no cell grid): path tracing."""
+"""Scenes that keep the BVH (two transforms, so no cell grid): path tracing
+and the adjoint."""
 import numpy as np
 import pytest
 
@@ -56,3 +57,36 @@ def test_path_trace_matches_oracle(gpu, width, height, spp, depth):
     ref = osc.path_trace(ctamd.AdjointDesc(len(views), spp, depth, 0x77), views, mats)
     assert np.array_equal(bits(img), bits(ref))
     assert np.isfinite(img).all() and (img.any() or width * height == 1)
+
+
+@pytest.mark.parametrize("depth", [0, 3, 5, 6, 7])
+def test_adjoint_matches_oracle(gpu, depth):
+    """Depths on both sides of where the backward pass keeps a path's vertices
+    elsewhere."""
+    import torch
+    w = AD.AdjointWorkload(grid=48, chunk=16, width=40, height=31, views=2, spp=3, max_depth=depth)
+    sc, alb, emi = AD.build_scene(w)
+    acc = _accel(sc)
+    AD._load_geometry(sc, acc)
+    slots = AD.VoxelSlots(sc, acc)
+    _shift_one(acc)
+    extent = w.grid * ctamd.CT_VOXEL_EXTENT
+    views = AD.orbit_views(w.views, w.width, w.height, (0, 0, 0), 1.6 * extent, 0.4 * extent)
+    r = AD.DiffRenderer(acc, views, w.spp, w.max_depth, w.target_seed)
+    a, e = slots.scatter(alb), slots.scatter(emi)
+    dev = torch.device("cuda")
+    a_t, e_t = torch.from_numpy(a).to(dev), torch.from_numpy(e).to(dev)
+    print("bvh adjoint", depth, flush=True)
+    img = r.forward(a_t, e_t).cpu().numpy()
+    osc, _, _ = oracle_scene_from_accel(acc, list(sc.materials), O.light_config_for(0, 0, 0))
+    desc = ctamd.AdjointDesc(len(views), w.spp, w.max_depth, w.target_seed)
+    n = len(acc.read_world()["aabbs"])  # the oracle's voxels are the accel's slots
+    ref = osc.adjoint_render(desc, views, a[:n], e[:n])
+    assert np.array_equal(bits(img), bits(ref))
+    g = np.random.default_rng(3).normal(size=ref.shape).astype(np.float32)
+    ga, ge = (v.cpu().numpy()[:n] for v in r.backward(a_t, e_t, torch.from_numpy(g).to(dev)))
+    oga, oge = osc.adjoint_backward(desc, views, a[:n], e[:n], g)
+    # sums of 32-bit terms in another order than the oracle's, in 64 bits
+    assert np.allclose(ge, oge, rtol=1e-4, atol=1e-6 * np.abs(oge).max())
+    assert np.allclose(ga, oga, rtol=1e-4, atol=1e-6 * max(np.abs(oga).max(), 1e-30))
+    assert np.abs(oge).sum() > 0
