@@ -18,6 +18,7 @@
 
 #include "ct_device.h"
 #include "ct_internal.h"
+#include "grid_plan.h"
 #include "grid_reach.h"
 
 namespace ct {
@@ -667,8 +668,6 @@ int build_segments(Accel &a, hipStream_t st, const std::vector<uint32_t> &off,
 // ------------------------------------------------------------ cell grid
 namespace {
 
-constexpr float kGridMaxCell = 4194304.0f;  // 2^22: cell centres and planes are exact floats
-
 // Cell of a voxel centre; false when the centre is not a cell's.
 __device__ __forceinline__ bool centre_cell(float c, int32_t &cell) {
   const float x = c * 32.0f, f = floorf(x);  // exact: a power of two
@@ -676,19 +675,35 @@ __device__ __forceinline__ bool centre_cell(float c, int32_t &cell) {
   return fabsf(x) < kGridMaxCell && f + 0.5f == x;
 }
 
-__global__ void k_grid_clear(uint4 *bricks, uint32_t n, uint32_t *work) {
+__global__ void k_grid_clear(uint4 *bricks, uint2 *was, uint32_t n, uint32_t *used) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) bricks[i] = make_uint4(0u, 0u, 0u, 0u);
-  if (i < 2u) work[i] = 0u;
+  if (i < n) {
+    bricks[i] = make_uint4(0u, 0u, 0u, 0u);
+    was[i] = make_uint2(0u, 0u);
+  }
+  if (i == 0u) *used = 0u;
 }
 
-// Sets each voxel's bit.  work[0] collects why the scene cannot have a grid:
-// 1 a centre off the lattice or out of range, 2 two voxels in one cell.
-__global__ void __launch_bounds__(kBlock) k_grid_mark(SegView sv, const ct_aabb *aabbs, DGrid g, uint32_t *bricks,
-                                                      uint32_t *cells, uint32_t *work) {
+// Clears the bits of the slots' voxels.
+__global__ void __launch_bounds__(kBlock) k_grid_unmark(SegView sv, uint32_t *bricks, uint32_t *cells) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= sv.n) return;
+  const uint32_t s = find_seg(sv.off, sv.nseg, k), slot = sv.base[s] + (k - sv.off[s]), c = cells[slot];
+  if (c == kInvalid) return;
+  atomicAnd(bricks + 4 * (size_t)(c >> 6) + ((c >> 5) & 1u), ~(1u << (c & 31u)));
+  cells[slot] = kInvalid;
+}
+
+// Sets each voxel's bit.  A voxel off the lattice, out of range or in a cell
+// that another one has keeps none (cells: kInvalid) and makes its instance
+// bad: the scene has no grid until a later update finds the cell free.
+// Segments from `retry` on mark only the voxels without a bit.
+__global__ void __launch_bounds__(kBlock) k_grid_mark(SegView sv, uint32_t retry, const ct_aabb *aabbs, DGrid g,
+                                                      uint32_t *bricks, uint32_t *cells, uint32_t *bad) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= sv.n) return;
   const uint32_t s = find_seg(sv.off, sv.nseg, k), slot = sv.base[s] + (k - sv.off[s]);
+  if (s >= retry && cells[slot] != kInvalid) return;
   const ct_aabb &b = aabbs[slot];
   int32_t c[3];
   bool ok = true;
@@ -699,38 +714,62 @@ __global__ void __launch_bounds__(kBlock) k_grid_mark(SegView sv, const ct_aabb 
     r[a] = (uint32_t)(c[a] - g.org[a]);
     ok = ok && r[a] < 16u * g.nblk[a];
   }
-  if (!ok) {
-    cells[slot] = kInvalid;
-    atomicOr(work, 1u);
-    return;
+  uint32_t cell = kInvalid;
+  if (ok) {
+    const uint32_t blk = ((r[2] >> 4) * g.nblk[1] + (r[1] >> 4)) * g.nblk[0] + (r[0] >> 4);
+    const uint32_t rec = (blk << 6) | ((r[0] >> 2) & 3u) | (r[1] & 12u) | ((r[2] & 12u) << 2);
+    const uint32_t bit = (r[0] & 3u) | ((r[1] & 3u) << 2) | ((r[2] & 3u) << 4);
+    const uint32_t old = atomicOr(bricks + 4 * (size_t)rec + (bit >> 5), 1u << (bit & 31u));
+    if (((old >> (bit & 31u)) & 1u) == 0u) cell = (rec << 6) | bit;
   }
-  const uint32_t blk = ((r[2] >> 4) * g.nblk[1] + (r[1] >> 4)) * g.nblk[0] + (r[0] >> 4);
-  const uint32_t rec = (blk << 6) | ((r[0] >> 2) & 3u) | (r[1] & 12u) | ((r[2] & 12u) << 2);
-  const uint32_t bit = (r[0] & 3u) | ((r[1] & 3u) << 2) | ((r[2] & 3u) << 4);
-  cells[slot] = (rec << 6) | bit;
-  const uint32_t old = atomicOr(bricks + 4 * (size_t)rec + (bit >> 5), 1u << (bit & 31u));
-  if ((old >> (bit & 31u)) & 1u) atomicOr(work, 2u);
+  cells[slot] = cell;
+  if (cell == kInvalid) bad[s] = 1u;
 }
 
-// One wave per block of 64 bricks: each brick's place in `ids` (the order of
-// bricks there is free, so a wave takes its range with one atomic) and its
-// empty cubes.  The occupancy of the bricks within kGridSkip - 1 of the
-// block is staged in LDS as rows of bits along x.
+// The blocks of a grid from lo on, n of them along each axis.
+struct GridRegion {
+  uint32_t lo[3], n[3];
+};
+
+// One wave per block of 64 bricks: each brick's place in `ids` and its empty
+// cubes.  A brick whose mask has changed takes a new place at the end (the
+// order of bricks there is free, so a wave takes its range with one atomic)
+// and brings the entries of the voxels that it keeps; past the end of `ids`
+// `full` is set instead.  The occupancy of the bricks within kGridSkip - 1 of
+// the block is staged in LDS as rows of bits along x.
 constexpr int kSkipHalo = (int)kGridSkip - 1, kSkipRow = 4 + 2 * kSkipHalo;
-__global__ void __launch_bounds__(64) k_grid_link(DGrid g, uint4 *bricks, uint32_t *work) {
+__global__ void __launch_bounds__(64) k_grid_link(DGrid g, GridRegion reg, uint4 *bricks, uint2 *was, uint2 *ids,
+                                                  uint32_t *slots, uint32_t id_cap, uint32_t *used, uint32_t *full) {
   __shared__ uint32_t rows[kSkipRow * kSkipRow];
-  const uint32_t blk = blockIdx.x, l = threadIdx.x;
+  const uint32_t l = threadIdx.x, rx = blockIdx.x % reg.n[0], ry = blockIdx.x / reg.n[0];
+  const uint32_t blk = ((reg.lo[2] + ry / reg.n[1]) * g.nblk[1] + reg.lo[1] + ry % reg.n[1]) * g.nblk[0] + reg.lo[0] + rx;
   const uint32_t rec = (blk << 6) | l;
   const uint4 e = bricks[rec];
-  const uint32_t n = (uint32_t)(__popc(e.x) + __popc(e.y));
-  uint32_t at = n;  // inclusive prefix over the wave
-  for (uint32_t o = 1; o < 64u; o <<= 1) {
-    const uint32_t v = __shfl_up(at, o);
-    if (l >= o) at += v;
+  const uint2 o = was[rec];
+  const bool changed = e.x != o.x || e.y != o.y;
+  const uint32_t n = (uint32_t)(__popc(e.x) + __popc(e.y)), need = changed ? n : 0u;
+  uint32_t at = need;  // inclusive prefix over the wave
+  for (uint32_t k = 1; k < 64u; k <<= 1) {
+    const uint32_t v = __shfl_up(at, k);
+    if (l >= k) at += v;
   }
   uint32_t first = 0;
-  if (l == 63u && at) first = atomicAdd(work + 1, at);
-  first = __shfl(first, 63);
+  if (l == 63u && at) first = atomicAdd(used, at);
+  first = __shfl(first, 63) + at - need;
+  if (need) {
+    if (first > id_cap || id_cap - first < need) {
+      *full = 1u;
+    } else {
+      const unsigned long long m = ((unsigned long long)e.y << 32) | e.x, q = ((unsigned long long)o.y << 32) | o.x;
+      for (unsigned long long keep = m & q; keep; keep &= keep - 1ull) {
+        const unsigned long long below = (keep & (~keep + 1ull)) - 1ull;
+        const uint32_t from = e.z + (uint32_t)__popcll(q & below), to = first + (uint32_t)__popcll(m & below);
+        ids[to] = ids[from];
+        slots[to] = slots[from];
+      }
+    }
+  }
+  if (changed) was[rec] = make_uint2(e.x, e.y);
   const int32_t x0 = (int32_t)(4u * (blk % g.nblk[0])), y0 = (int32_t)(4u * ((blk / g.nblk[0]) % g.nblk[1])),
                 z0 = (int32_t)(4u * (blk / (g.nblk[0] * g.nblk[1])));
   for (uint32_t r = l; r < (uint32_t)(kSkipRow * kSkipRow); r += 64u) {
@@ -766,11 +805,11 @@ __global__ void __launch_bounds__(64) k_grid_link(DGrid g, uint4 *bricks, uint32
       skip |= side << (4u * o);
     }
   }
-  reinterpret_cast<uint2 *>(bricks + rec)[1] = make_uint2(first + at - n, skip);
+  reinterpret_cast<uint2 *>(bricks + rec)[1] = make_uint2(changed ? first : e.z, skip);
 }
 
 __global__ void __launch_bounds__(kBlock) k_grid_ids(SegView sv, const uint32_t *inst, const uint4 *bricks,
-                                                     const uint32_t *cells, uint2 *ids, uint32_t *slots) {
+                                                     const uint32_t *cells, uint2 *ids, uint32_t *slots, uint32_t id_cap) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= sv.n) return;
   const uint32_t s = find_seg(sv.off, sv.nseg, k), p = k - sv.off[s], c = cells[sv.base[s] + p];
@@ -778,57 +817,18 @@ __global__ void __launch_bounds__(kBlock) k_grid_ids(SegView sv, const uint32_t 
   const uint4 e = bricks[c >> 6];
   const unsigned long long m = ((unsigned long long)e.y << 32) | e.x;
   const uint32_t i = e.z + (uint32_t)__popcll(m & ((1ull << (c & 63u)) - 1ull));
-  if (i < sv.n) {
+  if (i < id_cap) {
     ids[i] = make_uint2(inst[s], p);
     slots[i] = sv.base[s] + p;
   }
 }
 
-// Builds the scene's cell grid (DGrid) when it can have one: every instance
-// has the same transform, every voxel is a cell of the 2^-5 lattice, no cell
-// holds two voxels, the bricks of the bounding box are few against the
-// voxels (16 B a brick against about 130 B a voxel for the BVH), and there is
-// memory for it.  Enqueued
-// on `st`, which reads `seg` and writes `flags`: once it has drained, the
-// caller drops the grid if `flags` is not zero.
-int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::vector<uint32_t> &seg, uint32_t &flags) {
-  BvhSet &S = a.set;
-  S.grid = DGrid{};
-  flags = 0;
-  if (ids.empty()) return CT_OK;
-  const float *w = &a.w2o[16 * ids[0]];
-  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-  seg.assign(3 * ids.size() + 1, 0u);  // offsets, first slots, instance ids
-  const size_t nseg = ids.size();
-  for (size_t q = 0; q < nseg; ++q) {
-    const uint32_t id = ids[q];
-    if (std::memcmp(w, &a.w2o[16 * id], 16 * sizeof(float)) != 0 ||
-        std::memcmp(a.instances[ids[0]].transform, a.instances[id].transform, 16 * sizeof(float)) != 0)
-      return CT_OK;
-    for (int c = 0; c < 3; ++c) {
-      lo[c] = std::fmin(lo[c], a.blas_root_box[6 * id + c]);
-      hi[c] = std::fmax(hi[c], a.blas_root_box[6 * id + 3 + c]);
-    }
-    seg[q + 1] = seg[q] + a.instances[id].primitive_count;
-    seg[nseg + 1 + q] = a.instances[id].first_primitive_index;
-    seg[2 * nseg + 1 + q] = id;
-  }
-  const uint32_t n = seg[nseg];
-  DGrid g{};
-  uint64_t nblk = 1;
-  for (int c = 0; c < 3; ++c) {
-    if (!(std::fabs(lo[c]) < kGridMaxCell / 64.0f) || !(std::fabs(hi[c]) < kGridMaxCell / 64.0f)) return CT_OK;
-    // an empty brick at least around the boxes
-    const int32_t l = (int32_t)std::floor(lo[c] * 32.0f) - 5, h = (int32_t)std::floor(hi[c] * 32.0f) + 5;
-    g.org[c] = l & ~15;
-    g.nblk[c] = (uint32_t)((h | 15) + 1 - g.org[c]) / 16u;
-    nblk *= g.nblk[c];
-    if (g.nblk[c] > 1024u || nblk > (1u << 19)) return CT_OK;
-  }
-  const uint32_t nrec = (uint32_t)(64 * nblk);
-  if ((uint64_t)nrec > 4ull * n + (1u << 20)) return CT_OK;
-  for (int c = 0; c < 4; ++c)
-    for (int r = 0; r < 3; ++r) g.w2o[c * 3 + r] = w[c * 4 + r];
+// Takes the grid's memory for a build; false when it is refused.
+bool reserve_grid(Accel &a, const GridPlan &p) {
+  GridState &g = a.set.grid_state;
+  const uint32_t nrec = 64u * p.nblk[0] * p.nblk[1] * p.nblk[2];
+  g.id_cap = p.n + p.n / 8u + 16384u;                                   // room for bricks that later updates move
+  g.work_words = 2u + 6u * (uint32_t)(a.instances.size() + 64u);
   // One allocation: each takes and gives back about 0.4 ms, which a small
   // world's load would feel.
   size_t total = 0;
@@ -837,29 +837,140 @@ int build_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids, std::
     total += (bytes + 255) & ~(size_t)255;
     return at;
   };
-  const size_t o_bricks = place(16 * (size_t)nrec), o_ids = place(8 * (size_t)n), o_slots = place(4 * (size_t)n),
-               o_cells = place(4 * (size_t)S.prim_capacity), o_work = place(8 + 4 * seg.size());
-  if (!reserve_optional(S.grid_mem, total)) return CT_OK;
-  unsigned char *mem = S.grid_mem.as<unsigned char>();
-  uint4 *bricks = reinterpret_cast<uint4 *>(mem + o_bricks);
-  uint2 *d_ids = reinterpret_cast<uint2 *>(mem + o_ids);
-  uint32_t *slots = reinterpret_cast<uint32_t *>(mem + o_slots), *cells = reinterpret_cast<uint32_t *>(mem + o_cells),
-           *work = reinterpret_cast<uint32_t *>(mem + o_work), *d_seg = work + 2;
-  CT_HIP(hipMemcpyAsync(d_seg, seg.data(), 4 * seg.size(), hipMemcpyHostToDevice, st));
-  const SegView sv{d_seg, d_seg + nseg + 1, nullptr, (uint32_t)nseg, n};
-  hipLaunchKernelGGL(k_grid_clear, dim3(blocks(nrec)), dim3(kBlock), 0, st, bricks, nrec, work);
-  hipLaunchKernelGGL(k_grid_mark, dim3(blocks(n)), dim3(kBlock), 0, st, sv, S.aabbs.as<ct_aabb>(), g,
-                     reinterpret_cast<uint32_t *>(bricks), cells, work);
-  hipLaunchKernelGGL(k_grid_link, dim3((uint32_t)nblk), dim3(64), 0, st, g, bricks, work);
-  hipLaunchKernelGGL(k_grid_ids, dim3(blocks(n)), dim3(kBlock), 0, st, sv, d_seg + 2 * nseg + 1, bricks,
-                     cells, d_ids, slots);
+  const size_t o_bricks = place(16 * (size_t)nrec), o_was = place(8 * (size_t)nrec), o_ids = place(8 * (size_t)g.id_cap),
+               o_slots = place(4 * (size_t)g.id_cap), o_cells = place(4 * (size_t)a.set.prim_capacity),
+               o_work = place(4 * (size_t)g.work_words);
+  if (!reserve_optional(g.mem, total)) return false;
+  unsigned char *mem = g.mem.as<unsigned char>();
+  g.lay = DGrid{};
+  g.lay.bricks = reinterpret_cast<const uint4 *>(mem + o_bricks);
+  g.lay.ids = reinterpret_cast<const uint2 *>(mem + o_ids);
+  g.lay.slots = reinterpret_cast<const uint32_t *>(mem + o_slots);
+  g.lay.cells = reinterpret_cast<const uint32_t *>(mem + o_cells);
+  g.was = reinterpret_cast<uint2 *>(mem + o_was);
+  g.work = reinterpret_cast<uint32_t *>(mem + o_work);
+  for (int c = 0; c < 3; ++c) {
+    g.lay.org[c] = p.org[c];
+    g.lay.nblk[c] = p.nblk[c];
+  }
+  return true;
+}
+
+// Enqueues a plan's kernels on `st`, which reads `words` until it has
+// drained.  The update's results follow in work[1 + ...]: whether `ids` ran
+// out, then a word for each marked instance, whether it is bad.
+int enqueue_grid(Accel &a, hipStream_t st, const GridPlan &p, std::vector<uint32_t> &words) {
+  BvhSet &S = a.set;
+  GridState &g = S.grid_state;
+  std::vector<uint32_t> mark(p.mark);
+  mark.insert(mark.end(), p.retry.begin(), p.retry.end());
+  const uint32_t nm = (uint32_t)mark.size(), nu = (uint32_t)p.unmark.size();
+  // results, then offsets, first slots and ids of the marked instances, then
+  // offsets and first slots of the unmarked ones
+  words.assign(1u + nm, 0u);
+  words.push_back(0u);
+  for (uint32_t id : mark) words.push_back(words.back() + a.instances[id].primitive_count);
+  for (uint32_t id : mark) words.push_back(a.instances[id].first_primitive_index);
+  words.insert(words.end(), mark.begin(), mark.end());
+  words.push_back(0u);
+  for (uint32_t id : p.unmark) words.push_back(words.back() + g.inst[id].count);
+  for (uint32_t id : p.unmark) words.push_back(g.inst[id].first);
+  uint32_t *full = g.work + 1, *bad = full + 1, *off = bad + nm, *base = off + nm + 1, *inst = base + nm, *uoff = inst + nm,
+           *ubase = uoff + nu + 1;
+  const SegView sv{off, base, nullptr, nm, words[1 + nm + nm]}, uv{uoff, ubase, nullptr, nu, words[1 + nm + nm + 1 + 2 * nm + nu]};
+  uint4 *bricks = (uint4 *)(const uint4 *)g.lay.bricks;
+  uint2 *ids = (uint2 *)(const uint2 *)g.lay.ids;
+  uint32_t *slots = (uint32_t *)(const uint32_t *)g.lay.slots, *cells = (uint32_t *)(const uint32_t *)g.lay.cells;
+  const uint32_t nrec = 64u * p.nblk[0] * p.nblk[1] * p.nblk[2];
+  CT_HIP(hipMemcpyAsync(full, words.data(), 4 * words.size(), hipMemcpyHostToDevice, st));
+  if (p.kind == GridPlan::kFull)
+    hipLaunchKernelGGL(k_grid_clear, dim3(blocks(nrec)), dim3(kBlock), 0, st, bricks, g.was, nrec, g.work);
+  if (uv.n)
+    hipLaunchKernelGGL(k_grid_unmark, dim3(blocks(uv.n)), dim3(kBlock), 0, st, uv, reinterpret_cast<uint32_t *>(bricks),
+                       cells);
+  if (sv.n)
+    hipLaunchKernelGGL(k_grid_mark, dim3(blocks(sv.n)), dim3(kBlock), 0, st, sv, (uint32_t)p.mark.size(),
+                       S.aabbs.as<ct_aabb>(), g.lay, reinterpret_cast<uint32_t *>(bricks), cells, bad);
+  GridRegion reg;
+  for (int c = 0; c < 3; ++c) {
+    reg.lo[c] = p.lo[c];
+    reg.n[c] = p.hi[c] - p.lo[c];
+  }
+  hipLaunchKernelGGL(k_grid_link, dim3(reg.n[0] * reg.n[1] * reg.n[2]), dim3(64), 0, st, g.lay, reg, bricks, g.was, ids,
+                     slots, g.id_cap, g.work, full);
+  if (sv.n)
+    hipLaunchKernelGGL(k_grid_ids, dim3(blocks(sv.n)), dim3(kBlock), 0, st, sv, inst, bricks, cells, ids, slots, g.id_cap);
   CT_HIP(hipGetLastError());
-  CT_HIP(hipMemcpyAsync(&flags, work, 4, hipMemcpyDeviceToHost, st));
-  g.bricks = bricks;
-  g.ids = d_ids;
-  g.slots = slots;
-  g.cells = cells;
-  S.grid = g;
+  return CT_OK;
+}
+
+// Brings the scene's cell grid in line with the BVH set (GridPlan): begin_grid
+// enqueues, and finish_grid takes the results, after the TLAS, and says what
+// the walks use: the grid, when every instance has the same transform and
+// none is bad.
+struct GridUpdate {
+  GridPlan plan;
+  std::vector<uint32_t> words;
+};
+GridScene grid_scene(const Accel &a, const std::vector<uint32_t> &changed, bool everything) {
+  return GridScene{&a.instances, &a.instance_used, a.w2o.data(), a.blas_root_box.data(), changed, everything};
+}
+int begin_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &changed, bool everything, GridUpdate &u) {
+  GridState &g = a.set.grid_state;
+  u.plan = plan_grid(grid_scene(a, changed, everything), g);
+  if (u.plan.kind == GridPlan::kPart &&
+      2u + 4u * (u.plan.mark.size() + u.plan.retry.size()) + 2u * u.plan.unmark.size() + 2u > g.work_words)
+    u.plan = plan_grid(grid_scene(a, changed, true), g);  // more instances than its tables hold
+  g.given_up = u.plan.give_up || (g.given_up && !everything);
+  if (u.plan.kind == GridPlan::kFull && !reserve_grid(a, u.plan)) {
+    u.plan.kind = GridPlan::kNone;
+    g.given_up = true;
+  }
+  if (u.plan.kind == GridPlan::kNone) g.lay = DGrid{};
+  if (u.plan.kind == GridPlan::kNone || u.plan.kind == GridPlan::kKeep) return CT_OK;
+  const int rc = enqueue_grid(a, st, u.plan, u.words);
+  if (rc) g.lay = DGrid{};
+  return rc;
+}
+int finish_grid(Accel &a, hipStream_t st, GridUpdate &u) {
+  BvhSet &S = a.set;
+  GridState &g = S.grid_state;
+  if (u.plan.kind == GridPlan::kPart || u.plan.kind == GridPlan::kFull) {
+    const uint32_t nm = (uint32_t)(u.plan.mark.size() + u.plan.retry.size());
+    std::vector<uint32_t> res(1u + nm);
+    const DGrid lay = g.lay;
+    g.lay = DGrid{};  // none, if a call below fails
+    CT_HIP(hipMemcpyAsync(res.data(), g.work + 1, 4 * res.size(), hipMemcpyDeviceToHost, st));
+    CT_HIP(hipStreamSynchronize(st));
+    if (res[0]) {  // no room left for moved bricks: build it anew
+      GridUpdate again;
+      const std::vector<uint32_t> none;
+      const int rc = begin_grid(a, st, none, true, again);
+      return rc ? rc : finish_grid(a, st, again);
+    }
+    g.lay = lay;
+    if (u.plan.kind == GridPlan::kFull) g.inst.assign(a.instances.size(), GridInst{});
+    g.inst.resize(std::max(g.inst.size(), a.instances.size()));
+    for (uint32_t id : u.plan.unmark) g.inst[id] = GridInst{};
+    for (uint32_t q = 0; q < nm; ++q) {
+      const uint32_t id = q < u.plan.mark.size() ? u.plan.mark[q] : u.plan.retry[q - u.plan.mark.size()];
+      GridInst &i = g.inst[id];
+      i.first = a.instances[id].first_primitive_index;
+      i.count = a.instances[id].primitive_count;
+      std::memcpy(i.box, &a.blas_root_box[6 * (size_t)id], sizeof(i.box));
+      i.bad = res[1 + q] != 0u;
+    }
+  }
+  if (!g.lay.bricks || !u.plan.one_transform) return CT_OK;
+  for (const GridInst &i : g.inst)
+    if (i.bad) return CT_OK;
+  uint32_t id = 0;
+  while (!a.instance_used[id]) ++id;
+  DGrid out = g.lay;
+  for (int c = 0; c < 4; ++c)
+    for (int r = 0; r < 3; ++r) out.w2o[c * 3 + r] = a.w2o[16 * (size_t)id + c * 4 + r];
+  out.max_o = world_reach(a.instances[id].transform, &a.w2o[16 * (size_t)id], S.world_lo, S.world_hi);
+  if (out.max_o > 0.0f) S.grid = out;
   return CT_OK;
 }
 
@@ -1139,7 +1250,10 @@ int commit(Accel &a, const Dirty &d) {
   a.blas_depth.resize(a.instances.size(), 0);
   const uint32_t cap = std::max<uint32_t>(a.prim_high_water, 1);
   const bool full = d.full || S.prim_capacity != cap || !S.nodes.p;
-  S.grid = DGrid{};  // until this commit's own is built
+  // None until this commit's own is in place, also when it fails half way.
+  const DGrid had_grid = S.grid_state.lay;
+  S.grid_state.lay = DGrid{};
+  S.grid = DGrid{};
   if (full) {
     S.prim_capacity = cap;
     if ((rc = S.aabbs.reserve(sizeof(ct_aabb) * (size_t)cap)) || (rc = S.prims.reserve(sizeof(ct_primitive) * (size_t)cap)) ||
@@ -1219,18 +1333,18 @@ int commit(Accel &a, const Dirty &d) {
     if ((rc = refit_blas_set(a, st, d.refit))) return rc;
   }
   if ((rc = upload_tables(a, st))) return rc;
-  uint32_t grid_flags = 0;
-  std::vector<uint32_t> grid_seg;
-  rc = build_grid(a, st, used_ids(a), grid_seg, grid_flags);
+  std::vector<uint32_t> changed(d.rebuild);
+  changed.insert(changed.end(), d.refit.begin(), d.refit.end());
+  GridUpdate grid;
+  S.grid_state.lay = had_grid;
+  rc = begin_grid(a, st, changed, full, grid);
   if (!rc) rc = build_tlas(a, st);
-  const hipError_t e = hipStreamSynchronize(st);  // grid_seg was read, grid_flags has arrived
-  if (rc || e != hipSuccess || grid_flags) S.grid = DGrid{};
-  if (S.grid.bricks) {
-    const uint32_t id = used_ids(a)[0];
-    S.grid.max_o = world_reach(a.instances[id].transform, &a.w2o[16 * id], S.world_lo, S.world_hi);
-    if (!(S.grid.max_o > 0.0f)) S.grid = DGrid{};
+  if (!rc) rc = finish_grid(a, st, grid);
+  if (rc) {
+    (void)hipStreamSynchronize(st);  // `grid` is read until then
+    S.grid_state.lay = DGrid{};
+    S.grid = DGrid{};
   }
-  if (!rc && e != hipSuccess) return fail(CT_E_HIP, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
   return rc;
 }
 

@@ -187,6 +187,22 @@ struct BuildScratch {
 };
 
 // ---------------------------------------------------------- accel
+// The cell grid between updates, also while the walk may not use it.
+struct GridInst {
+  uint32_t first = 0, count = 0;  // the slots last marked
+  float box[6] = {0, 0, 0, 0, 0, 0};
+  bool bad = false;               // a voxel off the lattice, or in another's cell
+};
+struct GridState {
+  DevBuf mem;                     // its arrays
+  DGrid lay{};                    // bricks null: none
+  uint2 *was = nullptr;           // per brick: its mask when last linked
+  uint32_t *work = nullptr;       // entries of `ids` in use, then an update's tables (work_words)
+  uint32_t work_words = 0, id_cap = 0;
+  std::vector<GridInst> inst;     // by instance id
+  bool given_up = false;          // no grid until the slots are all new
+};
+
 struct BvhSet {
   DevBuf nodes, leaves, instances_d, prims, aabbs, cube_lights, inst_aos;
   DevBuf tlas_nodes, tlas_inst, tlas_keys, tlas_parent;
@@ -203,8 +219,8 @@ struct BvhSet {
   uint32_t prim_capacity = 0;
   uint32_t cube_light_count = 0;
   uint32_t cube_light_hw = 0;   // entries held: deleted lights leave stale records past the count
-  DevBuf grid_mem;              // the cell grid's arrays
-  DGrid grid{};                 // bricks null: no grid
+  GridState grid_state;
+  DGrid grid{};                 // what the walks use; bricks null: the BVH
   float world_lo[3] = {0, 0, 0}, world_hi[3] = {0, 0, 0};  // the instances' padded world boxes (build_tlas)
 };
 

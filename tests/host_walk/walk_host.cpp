@@ -10,6 +10,7 @@
 namespace ct {
 int fail(int code, const std::string &) { return code; }
 }  // namespace ct
+#include "../../cube-tracing_amd/csrc/grid_plan.h"
 using namespace ct;
 using namespace ct::dev;
 
@@ -259,6 +260,54 @@ extern "C" uint32_t batches(uint32_t base, uint32_t count, uint32_t stride, uint
   uint32_t n = 0;
   for (; base < count && n < most; base = next_batch(base, count, stride)) ++n;
   return n;
+}
+
+// Updates of a scene's grid, planned (csrc/grid_plan.h): `count` instances of
+// 8^3 cells side by side along x, all marked.  Then, by instance: first slots,
+// counts, boxes' shifts in cells along x, bits (1 used, 2 changed, 4 bad, 8 turned).
+// Returns the kind; lists and region as the plan has them.
+extern "C" int plan_update(uint32_t count, const uint32_t *first, const uint32_t *prims, const float *shift,
+                           const uint8_t *bits, int everything, int given_up, uint32_t *lists, uint32_t *region) {
+  GridState g;
+  std::vector<ct_instance> inst(count);
+  std::vector<uint8_t> used(count);
+  std::vector<float> w2o(16 * count, 0.0f), boxes(6 * count);
+  const uint4 some{};
+  g.lay.bricks = &some;
+  g.given_up = given_up != 0;
+  for (int a = 0; a < 3; ++a) {
+    g.lay.org[a] = -16;
+    g.lay.nblk[a] = a == 0 ? (8 * count + 15) / 16 + 2 : 3;
+  }
+  GridScene s{&inst, &used, w2o.data(), boxes.data(), {}, everything != 0};
+  g.inst.resize(count);
+  for (uint32_t i = 0; i < count; ++i) {
+    inst[i] = ct_instance{};
+    for (int k = 0; k < 16; k += 5) inst[i].transform[k] = w2o[16 * i + k] = 1.0f;
+    inst[i].first_primitive_index = first[i];
+    inst[i].primitive_count = prims[i];
+    used[i] = bits[i] & 1u;
+    if (bits[i] & 2u) s.changed.push_back(i);
+    if (bits[i] & 8u) inst[i].transform[12] = w2o[16 * i + 12] = 0.5f;
+    for (int a = 0; a < 3; ++a) {
+      const float lo = a == 0 ? 8.0f * (float)i : 0.0f;
+      g.inst[i].box[a] = lo / 32.0f;
+      g.inst[i].box[3 + a] = (lo + 8.0f) / 32.0f;
+      boxes[6 * i + a] = (lo + (a == 0 ? shift[i] : 0.0f)) / 32.0f;
+      boxes[6 * i + 3 + a] = (lo + 8.0f + (a == 0 ? shift[i] : 0.0f)) / 32.0f;
+    }
+    g.inst[i].first = 64 * i;
+    g.inst[i].count = 64;
+    g.inst[i].bad = (bits[i] & 4u) != 0u;
+  }
+  const GridPlan p = plan_grid(s, g);
+  for (uint32_t i = 0; i < count; ++i) lists[i] = 0;
+  for (uint32_t i : p.unmark) lists[i] |= 1u;
+  for (uint32_t i : p.mark) lists[i] |= 2u;
+  for (uint32_t i : p.retry) lists[i] |= 4u;
+  region[0] = p.lo[0];
+  region[1] = p.hi[0];
+  return (int)p.kind | (p.one_transform ? 16 : 0) | (p.give_up ? 32 : 0);
 }
 
 extern "C" float reach_of(const float *m, const float *w, const float *lo, const float *hi) { return world_reach(m, w, lo, hi); }

@@ -1,6 +1,8 @@
 """Scenes with a cell grid are walked through it, except by counted launches
 (`stats`), which walk the BVH: both must give the same hits to the bit, and a
 scene that an update takes off the lattice must leave the grid."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -164,3 +166,110 @@ def test_frames_of_far_cameras(gpu, far):
         images.append((ctx.read(ctamd.CT_BUF_IMAGE, w.width, w.height), bytes(ctx.read(ctamd.CT_BUF_DI, w.width, w.height))))
     assert np.array_equal(images[0][0].view(np.uint32), images[1][0].view(np.uint32))
     assert images[0][1] == images[1][1]
+
+
+def _add_instance(acc, boxes, prims):
+    """A BUILD task of one instance."""
+    st = acc.staging()
+    st.instances[0].first_primitive_index = 0
+    st.instances[0].primitive_count = len(boxes)
+    b, p = np.ascontiguousarray(boxes, np.float32), np.ascontiguousarray(prims, np.uint32)
+    C.memmove(st.aabbs, b.ctypes.data, b.nbytes)
+    C.memmove(st.primitives, p.ctypes.data, p.nbytes)
+    t = ctamd.Task()
+    t.type = ctamd.CT_TASK_BUILD_BLAS_FROM_CPU
+    t.u.blas_build_from_cpu.instance_count = 1
+    t.u.blas_build_from_cpu.primitive_count = len(boxes)
+    for k in range(16):
+        t.u.blas_build_from_cpu.transform[k] = 1.0 if k % 5 == 0 else 0.0
+    acc.task_queue_add(t)
+
+
+# instances that share bricks (chunks of 5 and 6 cells), a brick's multiple, one
+# instance; the sequences take the grid away and bring it back
+@pytest.mark.parametrize("grid,chunk,fill", [(17, 5, 0.3), (24, 6, 0.6), (48, 16, 0.1), (90, 30, 0.01), (12, 12, 0.5)])
+def test_grid_follows_edit_sequences(gpu, grid, chunk, fill):
+    sc, acc = _load(grid, chunk, fill, seed=grid)
+    rng = np.random.default_rng(grid)
+    step = np.eye(4, dtype=np.float32)
+    back, at = [], 0
+    cell = np.float32(1 / 32)
+
+    def update():
+        nonlocal at
+        acc.update_scene()
+        at += 1
+        print("edit", grid, at, flush=True)
+        _same(acc, sc, 100 + at, n=12000)
+
+    for _ in range(24):
+        while back:
+            back.pop()()
+            update()
+        insts = acc.read_instances()
+        used = [i for i, r in enumerate(insts) if r.primitive_count > 4]
+        inst = int(rng.choice(used))
+        r, box = insts[inst], acc.read_world()["aabbs"]
+        first, n = r.first_primitive_index, r.primitive_count
+        op = rng.choice(["delete", "two", "brush", "move", "off", "double", "shift", "drop", "still", "grow"])
+        if op == "delete":
+            acc.delete_primitive(inst, int(rng.integers(0, n)))
+            if rng.random() < 0.5:
+                back.append(acc.undo)
+        elif op == "two":  # two instances in one update
+            other = int(rng.choice(used))
+            acc.delete_primitive(inst, 0)
+            acc.delete_primitive(other, 1)
+        elif op == "brush":
+            acc.brush_mark([(inst, int(p)) for p in rng.choice(n, 2, replace=False)])
+            acc.process_voxel_modifications()
+        elif op in ("move", "off", "double", "grow"):
+            p = int(rng.integers(0, n))
+            old = box[first + p].copy()
+            other = insts[int(rng.choice(used))].first_primitive_index
+            new = {"move": old + cell * np.tile(rng.integers(-3, 4, 3), 2), "off": old + np.float32(0.007),
+                   "double": box[other].copy(), "grow": old + np.float32(0.5 * (1 + at % 3))}[op]
+            acc.update_blas(inst, edits=[(p, new.astype(np.float32))])
+            back.append(lambda i=inst, p=p, b=old: acc.update_blas(i, edits=[(p, b)]))
+        elif op == "shift":
+            m = step.copy()
+            m[3, 0] = 0.25
+            acc.update_blas(inst, transform=m.reshape(16))
+            m = m.copy()
+            m[3, 0] = -0.25
+            back.append(lambda i=inst, m=m: acc.update_blas(i, transform=m.reshape(16)))
+        elif op == "drop" and len(used) > 1:
+            boxes, prims = box[first:first + n].copy(), acc.read_world()["prims"][first:first + n].copy()
+            acc.delete_blas(inst)
+            back.append(lambda b=boxes, p=prims: _add_instance(acc, b, p))
+        else:
+            acc.update_blas(inst, transform=step.reshape(16))
+        update()
+
+
+def test_grid_finds_room_again_through_other_instances(gpu):
+    """A voxel put into another instance's cell takes the grid away; the other
+    instance's voxel leaving brings it back, right, with the first untouched."""
+    sc, acc = _load(20, 10, 0.4)
+    insts, box = acc.read_instances(), acc.read_world()["aabbs"]
+    assert len(insts) >= 3
+    a, b = insts[0].first_primitive_index, insts[1].first_primitive_index
+    old_a, old_b = box[a].copy(), box[b].copy()
+    acc.update_blas(0, edits=[(0, old_b)])
+    acc.update_scene()
+    _same(acc, sc, 1, n=30000)
+    acc.update_blas(2, edits=[(0, box[insts[2].first_primitive_index] + np.float32(1 / 32))])
+    acc.update_scene()
+    _same(acc, sc, 2, n=30000)
+    acc.delete_primitive(1, 0)
+    acc.update_scene()
+    _same(acc, sc, 3, n=30000)
+    acc.undo()
+    acc.update_scene()
+    _same(acc, sc, 4, n=30000)
+    acc.update_blas(1, edits=[(0, old_a)])
+    acc.update_scene()
+    _same(acc, sc, 5, n=30000)
+    acc.delete_blas(1)
+    acc.update_scene()
+    _same(acc, sc, 6, n=30000)

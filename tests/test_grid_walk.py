@@ -235,3 +235,41 @@ def test_refused_grid_memory_leaves_no_error(walk):
     through its BVH); the runtime's error state must be clear for the
     launches that follow."""
     assert walk.refused_memory() == 0
+
+
+def test_updates_touch_the_grid_where_the_scene_changed(walk):
+    """40 instances of 64 voxels in a row: what each update does to the grid."""
+    n = 40
+    NONE_, KEEP, PART, FULL, ONE, GIVE_UP = 0, 1, 2, 3, 16, 32
+
+    def plan(first=(), prims=(), shift=(), bits=(), everything=0, given_up=0):
+        f, p = np.arange(n, dtype=np.uint32) * 64, np.full(n, 64, np.uint32)
+        s, b = np.zeros(n, np.float32), np.ones(n, np.uint8)
+        for a, edits in ((f, first), (p, prims), (s, shift), (b, bits)):
+            for i, v in edits:
+                a[i] = v
+        lists, region = np.zeros(n, np.uint32), np.zeros(2, np.uint32)
+        kind = walk.plan_update(n, _p(f), _p(p), _p(s), _p(b), everything, given_up, _p(lists), _p(region))
+        return kind, {int(i): int(lists[i]) for i in np.flatnonzero(lists)}, tuple(int(v) for v in region)
+
+    assert plan()[:2] == (KEEP | ONE, {})                                # nothing moved
+    k, lists, region = plan(bits=[(20, 3)])                              # one instance: its voxels, its blocks
+    assert (k, lists) == (PART | ONE, {20: 3})
+    assert region[1] - region[0] <= 5 and 16 * region[0] - 16 <= 8 * 20 - 17 and 16 * region[1] - 16 >= 8 * 21 + 17
+    assert plan(prims=[(7, 63)])[:2] == (PART | ONE, {7: 3})             # a voxel fewer
+    assert plan(first=[(7, 9000)])[:2] == (PART | ONE, {7: 3})           # other slots
+    assert plan(bits=[(7, 0)])[:2] == (PART | ONE, {7: 1})               # an instance gone
+    assert plan(bits=[(7, 3), (9, 5)])[:2] == (PART | ONE, {7: 3, 9: 4})  # a bad one is tried again
+    assert plan(bits=[(9, 5)])[:2] == (KEEP | ONE, {})                   # but not when nothing made room
+    assert plan(bits=[(i, 5) for i in range(6)] + [(20, 3)])[0] == NONE_ | ONE | GIVE_UP
+    assert plan(bits=[(20, 3)], given_up=1)[0] == NONE_ | ONE | GIVE_UP
+    assert plan(given_up=1, everything=1)[0] == FULL | ONE
+    assert plan(shift=[(39, 200.0)], bits=[(39, 3)])[0] == FULL | ONE    # out of the grid
+    assert plan(bits=[(i, 3) for i in range(21)])[0] == FULL | ONE       # more than half of it
+    assert plan(bits=[(i, 3) for i in range(20)])[0] == PART | ONE
+    assert plan(everything=1)[0] == FULL | ONE
+    assert plan(bits=[(5, 9)])[:2] == (KEEP, {})                         # moved by its transform: the arrays stay right
+    assert plan(bits=[(5, 9), (6, 3)])[0] == NONE_
+    assert plan(shift=[(3, 1e9)], bits=[(3, 3)])[0] == NONE_ | ONE       # out of range
+    assert plan(shift=[(3, np.nan)], bits=[(3, 3)])[0] in (NONE_ | ONE, FULL | ONE)
+    assert plan(bits=[(i, 0) for i in range(n)])[0] == NONE_             # an empty scene
