@@ -551,6 +551,11 @@ __global__ void k_refit_prep(SegView sv, const uint32_t *blas_ids, const float4 
 }
 
 // dst[w.x] = w.y for each (index, value) pair; indices are checked on the host.
+__global__ void k_leaf_ids(const float4 *leaves, uint32_t n, uint32_t *ids) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) ids[i] = __float_as_uint(leaves[i].w);
+}
+
 __global__ void k_scatter_u32(const uint2 *w, uint32_t n, uint32_t *dst) {
   uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[w[i].x] = w[i].y;
@@ -576,6 +581,11 @@ void host_xform_point(const float *m, const float p[3], float out[3]) {
 struct BuildOut {
   std::vector<float> root_box;   // [nseg][6]
   std::vector<uint32_t> depth;   // [nseg]
+  bool want_box = true;
+  // Copied to the host with the build's own results, under their one wait.
+  void *with_dst = nullptr;
+  const void *with_src = nullptr;
+  size_t with_bytes = 0;
 };
 
 // Generic LBVH build over nseg segments of items.  centers/lo/hi are
@@ -656,8 +666,10 @@ int build_segments(Accel &a, hipStream_t st, const std::vector<uint32_t> &off,
   CT_HIP(hipMemcpyAsync(&herr, d_err, 4, hipMemcpyDeviceToHost, st));
   out.root_box.resize(6 * (size_t)nseg);
   out.depth.resize(nseg);
-  CT_HIP(hipMemcpyAsync(out.root_box.data(), S.root_box.p, 24 * (size_t)nseg, hipMemcpyDeviceToHost, st));
+  if (out.want_box)
+    CT_HIP(hipMemcpyAsync(out.root_box.data(), S.root_box.p, 24 * (size_t)nseg, hipMemcpyDeviceToHost, st));
   CT_HIP(hipMemcpyAsync(out.depth.data(), S.depth.p, 4 * (size_t)nseg, hipMemcpyDeviceToHost, st));
+  if (out.with_bytes) CT_HIP(hipMemcpyAsync(out.with_dst, out.with_src, out.with_bytes, hipMemcpyDeviceToHost, st));
   CT_HIP(hipStreamSynchronize(st));
   if (herr) return fail(CT_E_HIP, "LBVH validation failed (code " + std::to_string(herr) + ")");
   return CT_OK;
@@ -910,7 +922,7 @@ int enqueue_grid(Accel &a, hipStream_t st, const GridPlan &p, std::vector<uint32
 // none is bad.
 struct GridUpdate {
   GridPlan plan;
-  std::vector<uint32_t> words;
+  std::vector<uint32_t> words, results;  // the latter: work[1 ...] as the kernels left it
 };
 GridScene grid_scene(const Accel &a, const std::vector<uint32_t> &changed, bool everything) {
   return GridScene{&a.instances, &a.instance_used, a.w2o.data(), a.blas_root_box.data(), changed, everything};
@@ -928,6 +940,7 @@ int begin_grid(Accel &a, hipStream_t st, const std::vector<uint32_t> &changed, b
   }
   if (u.plan.kind == GridPlan::kNone) g.lay = DGrid{};
   if (u.plan.kind == GridPlan::kNone || u.plan.kind == GridPlan::kKeep) return CT_OK;
+  u.results.assign(1u + u.plan.mark.size() + u.plan.retry.size(), 0u);
   const int rc = enqueue_grid(a, st, u.plan, u.words);
   if (rc) g.lay = DGrid{};
   return rc;
@@ -937,18 +950,16 @@ int finish_grid(Accel &a, hipStream_t st, GridUpdate &u) {
   GridState &g = S.grid_state;
   if (u.plan.kind == GridPlan::kPart || u.plan.kind == GridPlan::kFull) {
     const uint32_t nm = (uint32_t)(u.plan.mark.size() + u.plan.retry.size());
-    std::vector<uint32_t> res(1u + nm);
-    const DGrid lay = g.lay;
-    g.lay = DGrid{};  // none, if a call below fails
-    CT_HIP(hipMemcpyAsync(res.data(), g.work + 1, 4 * res.size(), hipMemcpyDeviceToHost, st));
-    CT_HIP(hipStreamSynchronize(st));
-    if (res[0]) {  // no room left for moved bricks: build it anew
+    if (u.results[0]) {  // no room left for moved bricks: build it anew
       GridUpdate again;
       const std::vector<uint32_t> none;
       const int rc = begin_grid(a, st, none, true, again);
-      return rc ? rc : finish_grid(a, st, again);
+      if (rc) return rc;
+      if (again.results.empty()) return CT_OK;
+      CT_HIP(hipMemcpyAsync(again.results.data(), g.work + 1, 4 * again.results.size(), hipMemcpyDeviceToHost, st));
+      CT_HIP(hipStreamSynchronize(st));
+      return finish_grid(a, st, again);  // a build has room
     }
-    g.lay = lay;
     if (u.plan.kind == GridPlan::kFull) g.inst.assign(a.instances.size(), GridInst{});
     g.inst.resize(std::max(g.inst.size(), a.instances.size()));
     for (uint32_t id : u.plan.unmark) g.inst[id] = GridInst{};
@@ -958,7 +969,7 @@ int finish_grid(Accel &a, hipStream_t st, GridUpdate &u) {
       i.first = a.instances[id].first_primitive_index;
       i.count = a.instances[id].primitive_count;
       std::memcpy(i.box, &a.blas_root_box[6 * (size_t)id], sizeof(i.box));
-      i.bad = res[1 + q] != 0u;
+      i.bad = u.results[1 + q] != 0u;
     }
   }
   if (!g.lay.bricks || !u.plan.one_transform) return CT_OK;
@@ -1160,8 +1171,8 @@ int refit_blas_set(Accel &a, hipStream_t st, const std::vector<uint32_t> &ids) {
 }
 
 // TLAS over the instances' padded world boxes, in slot order (build_tlas,
-// accel_struct_mngr.cpp:1854-1973).
-int build_tlas(Accel &a, hipStream_t st) {
+// accel_struct_mngr.cpp:1854-1973).  Brings the grid update's results along.
+int build_tlas(Accel &a, hipStream_t st, GridUpdate &grid) {
   BvhSet &S = a.set;
   int rc;
   const std::vector<uint32_t> ids = used_ids(a);
@@ -1220,14 +1231,18 @@ int build_tlas(Accel &a, hipStream_t st) {
   uint32_t *tk = S.tlas_keys.as<uint32_t>();
   uint32_t *tpar = S.tlas_parent.as<uint32_t>();
   BuildOut to;
+  to.want_box = false;
+  if (!grid.results.empty()) {
+    to.with_dst = grid.results.data();
+    to.with_src = S.grid_state.work + 1;
+    to.with_bytes = 4 * grid.results.size();
+  }
   rc = build_segments(a, st, toff, tbase, tsrc, false, nullptr, dc, dl, dh, dpay, 0.0f, ni, S.tlas_nodes.as<DNode>(),
                       tleaves.as<float4>(), tk, tk + ni, tpar, tpar + ni, to);
   if (rc) return rc;
-  std::vector<float4> hl(ni);
-  CT_HIP(hipMemcpy(hl.data(), tleaves.p, 16 * (size_t)ni, hipMemcpyDeviceToHost));
-  std::vector<uint32_t> tinst(ni);
-  for (uint32_t q = 0; q < ni; ++q) std::memcpy(&tinst[q], &hl[q].w, 4);
-  CT_HIP(hipMemcpy(S.tlas_inst.p, tinst.data(), 4 * (size_t)ni, hipMemcpyHostToDevice));
+  hipLaunchKernelGGL(k_leaf_ids, dim3(blocks(ni)), dim3(kBlock), 0, st, tleaves.as<float4>(), ni, S.tlas_inst.as<uint32_t>());
+  CT_HIP(hipGetLastError());
+  CT_HIP(hipStreamSynchronize(st));  // the leaves are released on return
   S.tlas_root = ni == 1 ? kLeaf : 0u;
   S.tlas_depth = to.depth[0];
   S.generation = ++a.generation;
@@ -1338,7 +1353,7 @@ int commit(Accel &a, const Dirty &d) {
   GridUpdate grid;
   S.grid_state.lay = had_grid;
   rc = begin_grid(a, st, changed, full, grid);
-  if (!rc) rc = build_tlas(a, st);
+  if (!rc) rc = build_tlas(a, st, grid);
   if (!rc) rc = finish_grid(a, st, grid);
   if (rc) {
     (void)hipStreamSynchronize(st);  // `grid` is read until then
