@@ -33,7 +33,10 @@ CT_D float dot(F3 a, F3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 CT_D float length(F3 a) { return sqrtf(dot(a, a)); }
 CT_D F3 normalize(F3 a) { return divs(a, length(a)); }
 // normalize of what is mostly an axis vector already: its length is 1, and
-// the square root and the divisions by 1 (45 instructions) are left out.
+// the square root and the divisions by 1 (45 instructions) are left out.  For
+// scattered directions only (a fit's step 14.40 -> 14.19 ms): the branch keeps
+// more alive around it, and with it in the material terms k_pt_end (finish,
+// hybrid shift) held 232 VGPRs instead of 149.
 CT_D F3 normalize_axis(F3 a) {
   const float d = dot(a, a);
   return d == 1.0f ? a : divs(a, sqrtf(d));
@@ -50,33 +53,40 @@ CT_D F3 mix3(F3 x, F3 y, float a) { return f3(mixf(x.x, y.x, a), mixf(x.y, y.y, 
 CT_D float gsign(float x) { return x > 0.0f ? 1.0f : (x < 0.0f ? -1.0f : 0.0f); }
 CT_D F3 xyz(float4 v) { return f3(v.x, v.y, v.z); }
 
-// Saturating conversions (NaN -> 0), which the hardware's are (a C++ cast
-// leaves values out of range undefined, and guarding it takes 8 instructions;
-// compute_ray_origin converts three values, and each pass calls it 2 to 6
-// times a pixel).
-#if defined(__HIP_DEVICE_COMPILE__)
-CT_D uint32_t f2u_sat(float x) {
-  uint32_t r;
-  asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x));
-  return r;
-}
-CT_D int32_t f2i_sat(float x) {
-  int32_t r;
-  asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x));
-  return r;
-}
-#else
-CT_D uint32_t f2u_sat(float x) {
+// Saturating conversions (NaN -> 0).
+CT_D uint32_t f2u_clamped(float x) {
   if (!(x > 0.0f)) return 0u;
   if (x >= 4294967296.0f) return 0xFFFFFFFFu;
   return (uint32_t)x;
 }
-CT_D int32_t f2i_sat(float x) {
-  if (isnan(x)) return 0;
+CT_D int32_t f2i_clamped(float x) {
+  if (!(x == x)) return 0;
   if (x >= 2147483648.0f) return 0x7FFFFFFF;
   if (x <= -2147483648.0f) return (int32_t)0x80000000;
   return (int32_t)x;
 }
+// The same as the hardware's own instruction (a C++ cast leaves values out of
+// range undefined, and guarding it takes 8 instructions; compute_ray_origin
+// converts three values, and each pass calls it 2 to 6 times a pixel).  The
+// compiler neither leaves out an asm statement whose result nothing uses nor
+// moves it into the branch that does: code whose results may go unused takes
+// the guarded ones.  (Path reuse, which loads vertices for tests that may not
+// need them: k_pt_end held 219 VGPRs in its finish pass and 185 in the request
+// pass, instead of 121 and 20.)
+#if defined(__HIP_DEVICE_COMPILE__)
+CT_D uint32_t f2u_sat(float x) {
+  uint32_t r;
+  [[clang::noconvergent]] { asm("v_cvt_u32_f32 %0, %1" : "=v"(r) : "v"(x)); }
+  return r;
+}
+CT_D int32_t f2i_sat(float x) {
+  int32_t r;
+  [[clang::noconvergent]] { asm("v_cvt_i32_f32 %0, %1" : "=v"(r) : "v"(x)); }
+  return r;
+}
+#else
+CT_D uint32_t f2u_sat(float x) { return f2u_clamped(x); }
+CT_D int32_t f2i_sat(float x) { return f2i_clamped(x); }
 #endif
 
 // Memory that no kernel of the launch writes, as constant memory: uniform
@@ -128,9 +138,12 @@ CT_D uint32_t urnd_interval(uint32_t &prev, uint32_t mn, uint32_t mx) {
 CT_D float safe_inverse(float x) { return (x == 0.0f) ? 1e12f : (1.0f / x); }
 
 // primitives.glsl:233-257
+// kMaybeUnused: the result may go unused (f2i_sat).
+template <bool kMaybeUnused = false>
 CT_D F3 compute_ray_origin(F3 pos, F3 n) {
   const float origin = 1.f / 32.f, f_scale = 1.f / 65536.f, i_scale = 256.f;
-  int32_t ix = f2i_sat(n.x * i_scale), iy = f2i_sat(n.y * i_scale), iz = f2i_sat(n.z * i_scale);
+  auto cvt = [](float x) { return kMaybeUnused ? f2i_clamped(x) : f2i_sat(x); };
+  int32_t ix = cvt(n.x * i_scale), iy = cvt(n.y * i_scale), iz = cvt(n.z * i_scale);
   float px = __uint_as_float(__float_as_uint(pos.x) + (uint32_t)(pos.x < 0.0f ? -ix : ix));
   float py = __uint_as_float(__float_as_uint(pos.y) + (uint32_t)(pos.y < 0.0f ? -iy : iy));
   float pz = __uint_as_float(__float_as_uint(pos.z) + (uint32_t)(pos.z < 0.0f ? -iz : iz));

@@ -305,7 +305,7 @@ CT_D bool occluded(const DFrame &F, Vis &v, F3 o, F3 d, float dist, uint32_t ti,
 }
 
 // mat.glsl:24-27, 58-88; light.glsl:200-229 (Lambertian)
-CT_D float local_z(F3 n, F3 v) { return dot(v, normalize_axis(n)); }
+CT_D float local_z(F3 n, F3 v) { return dot(v, normalize(n)); }
 CT_D float material_pdf(F3 n, F3 wo, F3 wi) {
   float a = local_z(n, wo), b = local_z(n, wi);
   if (gmin(a, b) < kMinCosTheta) return 0.0f;
@@ -328,8 +328,8 @@ struct Shade {
 };
 CT_D Shade shade_of(F3 ray_d, const Hit &hit) {
   Shade s;
-  s.sn = normalize_axis(hit.n);
-  s.nsn = normalize_axis(s.sn);
+  s.sn = normalize(hit.n);
+  s.nsn = normalize(s.sn);
   s.wo = neg(normalize(ray_d));
   s.a_eval = dot(s.wo, s.nsn);
   s.a_pdf = dot(neg(ray_d), s.sn);

@@ -337,8 +337,8 @@ CT_D Isect load_vertex(const DFrame &F, const ObjHit &h, F3 world_pos) {
   float t;
   F3 pos, nor;
   if (!hit_from_ray(F, h.inst, h.prim, world_pos, rd, t, pos, nor)) return isect_empty();
-  pos = compute_ray_origin(pos, nor);
-  pos = compute_ray_origin(pos, nor);
+  pos = compute_ray_origin<true>(pos, nor);
+  pos = compute_ray_origin<true>(pos, nor);
   Isect i;
   i.is_hit = true;
   i.distance = length(sub(world_pos, pos));
@@ -355,7 +355,7 @@ CT_D Isect load_vertex(const DFrame &F, const ObjHit &h, F3 world_pos) {
 // compute_new_ray_origin, primitives.glsl:259-264
 CT_D F3 new_ray_origin(F3 pos, F3 n, bool view_side) {
   F3 nn = view_side ? n : neg(n);
-  return compute_ray_origin(compute_ray_origin(pos, nn), nn);
+  return compute_ray_origin<true>(compute_ray_origin<true>(pos, nn), nn);
 }
 
 // ---------------------------------------------------------------- sampling
