@@ -1,12 +1,13 @@
-"""Scenes that keep the BVH (two transforms, so no cell grid): path tracing
-and the adjoint."""
+"""Scenes that keep the BVH (two transforms, so no cell grid): path tracing,
+the adjoint, frames with the RIS BRDF strategy and the hybrid shift, and
+batches that mix such a scene with one walked through its grid."""
 import numpy as np
 import pytest
 
 import ctamd
 import oracle as O
 from ctamd import adjoint as AD
-from helpers import bits, oracle_scene_from_accel
+from helpers import all_buffers_equal, bits, oracle_scene_from_accel
 
 pytestmark = pytest.mark.gpu
 
@@ -90,3 +91,67 @@ def test_adjoint_matches_oracle(gpu, depth):
     assert np.allclose(ge, oge, rtol=1e-4, atol=1e-6 * np.abs(oge).max())
     assert np.allclose(ga, oga, rtol=1e-4, atol=1e-6 * max(np.abs(oga).max(), 1e-30))
     assert np.abs(oge).sum() > 0
+
+
+def _loaded(w, shift):
+    sc = ctamd.Scene(ctamd.scene_desc(w))
+    acc, first = _accel(sc), ctamd.Ctx(8, 8)
+    ctamd.load_scene(sc, acc, first)  # the accel holds the scene; contexts bind to it
+    if shift:
+        _shift_one(acc)
+    return sc, acc
+
+
+def _ctx(sc, w):
+    ctx = ctamd.Ctx(w.width, w.height)
+    ctamd.bind_scene(sc, ctx)
+    return ctx
+
+
+@pytest.mark.parametrize("kind", ["plain", "ris_brdf", "hybrid", "hybrid_ris_brdf"])
+def test_frames_match_oracle(gpu, kind):
+    w = ctamd.hd_di(width=57, height=35, grid=48, chunk=16, frames=3, max_depth=3)
+    if "hybrid" in kind:
+        w.restir.pt_shift_mapping = ctamd.CT_SHIFT_HYBRID
+    if "brdf" in kind:
+        w.features |= ctamd.CT_RIS_BRDF_BIT
+        w.emissive *= 10
+    sc, acc = _loaded(w, True)
+    ctx = _ctx(sc, w)
+    osc, _, _ = oracle_scene_from_accel(acc, list(sc.materials), ctx.light_config())
+    ofr = O.OFrame(osc, w.width, w.height)
+    for f in range(3):
+        print("bvh frame", kind, f, flush=True)
+        p = ctamd.frame_params(w, f)
+        ctx.render(acc, p)
+        ofr.render(p)
+        hit = all_buffers_equal(ctx, ofr, w, f)
+        assert hit.any() and not hit.all()
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_batch_of_bvh_and_grid_scenes(gpu, use_graph):
+    """Views of a scene with a cell grid beside views of one without, in one
+    batch (which walks BVHs then), with the hybrid shift and the RIS BRDF
+    strategy in some of them: each view's bits equal its own render."""
+    scenes, views = ctamd.batched_views(n_views=6, seed=0xC3, grids=(48, 64), max_depth=2, size_scale=0.08)
+    built = [_loaded(s, k == 0) for k, s in enumerate(scenes)]
+    for n, (k, w) in enumerate(views):
+        w.restir = ctamd.RestirParams.from_buffer_copy(bytes(w.restir))
+        if n % 3 == 0:
+            w.restir.pt_shift_mapping = ctamd.CT_SHIFT_HYBRID
+        if n % 2 == 0:
+            w.features |= ctamd.CT_RIS_BRDF_BIT
+    assert {k for k, _ in views} >= {0, 1}
+    plain = [_ctx(built[k][0], w) for k, w in views]
+    batch_ctx = [_ctx(built[k][0], w) for k, w in views]
+    b = ctamd.Batch(batch_ctx, [built[k][1] for k, _ in views])
+    for f in range(3):
+        print("mixed batch", use_graph, f, flush=True)
+        ps = [ctamd.frame_params(w, f) for _, w in views]
+        b.render(ps, use_graph=use_graph)
+        for (k, w), ctx, p in zip(views, plain, ps):
+            ctx.render(built[k][1], p)
+        for n, ((k, w), pc, bc) in enumerate(zip(views, plain, batch_ctx)):
+            for which in (ctamd.CT_BUF_IMAGE, ctamd.CT_BUF_DI, ctamd.CT_BUF_TEMPORAL_PATH_RESERVOIR):
+                assert bytes(pc.read(which, w.width, w.height)) == bytes(bc.read(which, w.width, w.height)), (f, n, which)
