@@ -383,7 +383,6 @@ struct Ctx {
   Reach reach;                  // the scenes this context has rendered since its reset
   const void *lights_accel = nullptr;  // accel and build whose cube lights were uploaded
   uint32_t lights_generation = 0;
-  bool cube_plain = false;             // every uploaded cube light is of type CUBE and emits
   // A frame can run as kSplitParts interleaved parts of the image on as
   // many streams (the render stream and part_stream[1..]). Each part has
   // its own frame record, block table, ray and segment queues, counters and

@@ -59,7 +59,6 @@ struct DFrame {
   uint32_t W, H, npix, frame, active, afternoon;
   float time;
   uint32_t n_cube, n_point, n_env, n_mats;
-  uint32_t cube_plain;  // every cube light is of type CUBE and emits
   float inv_view[16], inv_proj[16];
   ct_restir_params rp;
   ct_light_config cfg;
@@ -2058,12 +2057,6 @@ int prepare_frame(Ctx *c, Accel *a, const ct_frame_params *p, hipStream_t st, DF
     CT_HIP(hipStreamSynchronize(st));  // earlier frames may still read the old table
     std::vector<float4> pk;
     pack_lights(a->cube_lights_host.data(), ncube, pk);
-    c->cube_plain = true;
-    for (uint32_t i = 0; i < ncube; ++i) {
-      const ct_light &l = a->cube_lights_host[i];
-      c->cube_plain = c->cube_plain && l.type == CT_LIGHT_CUBE &&
-                      !(l.emissive[0] <= 0.0f && l.emissive[1] <= 0.0f && l.emissive[2] <= 0.0f);
-    }
     if ((rc = cube.reserve(16 * pk.size()))) return rc;
     CT_HIP(hipMemcpy(cube.p, pk.data(), 16 * pk.size(), hipMemcpyHostToDevice));
     c->lights_accel = a;
@@ -2076,7 +2069,6 @@ int prepare_frame(Ctx *c, Accel *a, const ct_frame_params *p, hipStream_t st, DF
   F.frame = p->frame_number; F.active = p->is_active; F.afternoon = p->is_afternoon; F.time = p->time;
   F.n_cube = ncube; F.n_point = (uint32_t)c->point_host.size(); F.n_env = (uint32_t)c->env_host.size();
   F.n_mats = (uint32_t)c->mats_host.size();
-  F.cube_plain = c->cube_plain ? 1u : 0u;
   std::memcpy(F.inv_view, p->inv_view, sizeof(F.inv_view));
   std::memcpy(F.inv_proj, p->inv_proj, sizeof(F.inv_proj));
   F.rp = p->restir;
