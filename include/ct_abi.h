@@ -672,8 +672,9 @@ int ct_batch_get_stats(ct_batch *batch, ct_frame_stats *out);
  * is the number of view groups (1 to 4: contiguous ranges of views of
  * about equal pixel count, each with its own queues, run on concurrent
  * streams so one group's traversal tail overlaps another's passes), the
- * grid of the persistent traversal kernels (3, 4 or 5 blocks per CU; a
- * grid never exceeds the blocks that can be resident at once) and the ray
+ * grid of the persistent traversal kernels (3, 4 or 5 blocks per CU where
+ * BVHs are walked; it never exceeds the blocks that can be resident at
+ * once, which a batch of scenes with cell grids always takes) and the ray
  * queue's order (shadow rays at least far_ray long are queued and traced
  * first: 1, 2, 4 world units or none): 48 shapes.  No shape changes a
  * result.  A new batch starts with 2 groups, 5 blocks per CU and 2 units.
