@@ -467,6 +467,34 @@ SPATIAL_NEIGHBOUR_BYTES = 128 + 2 * 48
 RAY_BYTES = 36
 
 
+WALKS = ("k_trace_any", "k_trace_segments", "k_primary")
+KERNELS = {"k_trace_any": "k_trace_any_frames (shadow-ray any-hit traversal)",
+           "k_trace_segments": "k_trace_segments (path-segment closest-hit traversal)",
+           "k_primary": "k_primary (camera-ray closest-hit traversal)",
+           "k_ris": "k_ris (hit shading, motion vector, RIS candidates, visibility-ray emission)",
+           "k_spatial": "k_spatial (spatial reuse emit + finish, shading)"}
+
+
+def roofline(k, ms_per_frame, launches, algo_bytes, traffic):
+    """One kernel against the HBM peak: ms and launches of a frame, the
+    algorithm's and the measured HBM bytes of a launch (None: not measured).
+    The traversal kernels walk the scene's cell grid, whose bricks nothing
+    counts: their fraction is the measured traffic's or none, and the bytes
+    of an instrumented frame, which walks the BVH, are given as such."""
+    s = ms_per_frame / 1e3
+    rate = lambda b: round(b * launches / s / 1e9, 1) if b is not None and s > 0 else None
+    frac = lambda g: None if g is None else round(g / HBM_PEAK_GBS, 4)
+    r = {"bound": "hbm", "peak": HBM_PEAK_GBS, "unit": "GB/s", "traffic": traffic, "kernel": KERNELS[k],
+         "ms_per_frame": round(ms_per_frame, 3), "launches_per_frame": launches}
+    if k in WALKS:
+        r.update(bound="latency", achieved=rate(traffic), frac=frac(rate(traffic)), bvh_bytes_per_launch=round(algo_bytes))
+        return r
+    r.update(achieved=rate(algo_bytes), frac=frac(rate(algo_bytes)), algorithmic_bytes_per_launch=round(algo_bytes))
+    if traffic is not None:
+        r.update(hbm_gbs_physical=rate(traffic), frac_physical=frac(rate(traffic)))
+    return r
+
+
 def frame_bench(w, acc, ctx, K, Wm, traffic):
     """K timed frames of workload w (two halves on two streams, as the
     library renders a large frame) after Wm warm-up frames and one
@@ -486,7 +514,8 @@ def frame_bench(w, acc, ctx, K, Wm, traffic):
     ist = ctx.stats()
     hits = int((np.frombuffer(bytes(ctx.read(ctamd.CT_BUF_DI, w.width, w.height)), np.float32)
                 .reshape(-1, 15)[:, 3] > 0).sum())
-    # Algorithmic bytes per query: a shadow ray reads its 36 B record, a
+    # Bytes per query of the BVH walk (the instrumented frame's; the timed
+    # frames walk the cell grid): a shadow ray reads its 36 B record, a
     # path segment reads 32 B and writes a 16 B hit; every BVH2 node
     # fetched is 64 B, every leaf 28 B (centre + id + instance record
     # share), every instance entry 64 B.
@@ -552,24 +581,8 @@ def frame_bench(w, acc, ctx, K, Wm, traffic):
     # (with paths), spatial visibility
     launches = {"k_trace_any": 3 if depth else 2,
                 "k_trace_segments": max(depth, 1), "k_primary": 1, "k_ris": 1, "k_spatial": 2}
-    desc = {"k_trace_any": "k_trace_any_frames (shadow-ray any-hit traversal)",
-            "k_trace_segments": "k_trace_segments (path-segment closest-hit traversal)",
-            "k_primary": "k_primary (camera-ray closest-hit traversal)",
-            "k_ris": "k_ris (hit shading, motion vector, RIS candidates, visibility-ray emission)",
-            "k_spatial": "k_spatial (spatial reuse emit + finish, shading)"}
-
     def roof(k):
-        per_frame_ms = ms[k] / K
-        achieved = algo[k] / (per_frame_ms / 1e3) / 1e9 if per_frame_ms > 0 else 0.0
-        t = traffic.get(k)
-        r = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": t,
-             "algorithmic_bytes_per_launch": round(algo[k] / launches[k]),
-             "kernel": desc[k], "ms_per_frame": round(per_frame_ms, 3), "launches_per_frame": launches[k]}
-        if t:
-            r["hbm_gbs_physical"] = round(t * launches[k] / (per_frame_ms / 1e3) / 1e9, 1)
-            r["frac_physical"] = round(r["hbm_gbs_physical"] / HBM_PEAK_GBS, 4)
-        return r
+        return roofline(k, ms[k] / K, launches[k], algo[k] / launches[k], traffic.get(k))
 
     order = sorted(("k_trace_any", "k_trace_segments"), key=lambda k: -ms[k])
     med = lambda v: sorted(v)[len(v) // 2]
