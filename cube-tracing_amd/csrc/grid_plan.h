@@ -49,7 +49,7 @@ inline bool grid_cells(const float *box, int32_t *l, int32_t *h) {
 // A grid needs one transform for every instance, voxels on the 2^-5 lattice,
 // one to a cell (both found while marking), and bricks that are few against
 // the voxels.  The cost of an update is that of the instances it changed:
-// rebuilding the whole grid added 0.35 ms to an update of 256^3 voxels
+// building the whole grid anew took 0.35 ms of an update of 256^3 voxels
 // whatever it changed (0.48 -> 0.83 ms for one that moves no voxel).  A
 // change of half of the voxels is built anew, which also closes the gaps
 // that parts leave in `ids`.  Where bad instances that the update leaves alone
