@@ -332,13 +332,14 @@ CT_D bool vertex_visible(const DFrame &F, F3 o, F3 d, float dist, uint32_t ti, u
 }
 
 // load_intersection_data_vertex_position, primitives.glsl:567-611
+template <bool kMaybeUnused>
 CT_D Isect load_vertex(const DFrame &F, const ObjHit &h, F3 world_pos) {
   F3 rd = sub(h.hit, world_pos);
   float t;
   F3 pos, nor;
   if (!hit_from_ray(F, h.inst, h.prim, world_pos, rd, t, pos, nor)) return isect_empty();
-  pos = compute_ray_origin<true>(pos, nor);
-  pos = compute_ray_origin<true>(pos, nor);
+  pos = compute_ray_origin<kMaybeUnused>(pos, nor);
+  pos = compute_ray_origin<kMaybeUnused>(pos, nor);
   Isect i;
   i.is_hit = true;
   i.distance = length(sub(world_pos, pos));
@@ -353,9 +354,10 @@ CT_D Isect load_vertex(const DFrame &F, const ObjHit &h, F3 world_pos) {
   return i;
 }
 // compute_new_ray_origin, primitives.glsl:259-264
+template <bool kMaybeUnused>
 CT_D F3 new_ray_origin(F3 pos, F3 n, bool view_side) {
   F3 nn = view_side ? n : neg(n);
-  return compute_ray_origin<true>(compute_ray_origin<true>(pos, nn), nn);
+  return compute_ray_origin<kMaybeUnused>(compute_ray_origin<kMaybeUnused>(pos, nn), nn);
 }
 
 // ---------------------------------------------------------------- sampling
@@ -835,7 +837,9 @@ CT_D void ld_pstate(const float4 *S, uint32_t np, uint32_t p, PState &s, bool re
 // connection is rejected; with use_cached the source side's geometry term
 // and pdfs come from the reservoir's cached Jacobian, and a successful
 // shift leaves the destination's there.
-template <int kWalk, int kVis = kVisInline>
+// (The hybrid emit pass uses the vertex on nearly every path: there the
+// guarded conversions only cost, 118 -> 132 us a palette frame.)
+template <int kWalk, int kVis = kVisInline, bool kHybrid = false>
 CT_D F3 shift_reconnection(const DFrame &F, float &dst_jac, Isect dst, Isect src, PRes &s, bool eval_vis,
                            PtTrace &tr, bool use_hybrid = false, bool use_cached = false) {
   dst_jac = 0.0f;
@@ -846,8 +850,9 @@ CT_D F3 shift_reconnection(const DFrame &F, float &dst_jac, Isect dst, Isect src
   const uint32_t plen = pf_path_length(s.flags);
   const bool nee = pf_last_nee(s.flags);
   const bool trans = pf_transmission(s.flags, true);
-  src.P = new_ray_origin(src.P, src.n, !trans);
-  dst.P = new_ray_origin(dst.P, dst.n, !trans);
+  constexpr bool kMaybeUnused = !(kHybrid && kVis == kVisEmit);
+  src.P = new_ray_origin<kMaybeUnused>(src.P, src.n, !trans);
+  dst.P = new_ray_origin<kMaybeUnused>(dst.P, dst.n, !trans);
   if (!exists) {
     F3 integrand = f3(0, 0, 0);
     if (pf_light_type(s.flags) == kGeomLightEnv && plen + 1u == rc_len && !nee) {
@@ -870,7 +875,7 @@ CT_D F3 shift_reconnection(const DFrame &F, float &dst_jac, Isect dst, Isect src
   const bool escaped = plen + 1u == rc_len && !nee;
   const bool rc_nee = is_final && nee;
   if (pf_delta(s.flags, true) || pf_delta(s.flags, false)) return f3(0, 0, 0);
-  const Isect rc = load_vertex(F, s.rc, dst.P);
+  const Isect rc = load_vertex<kMaybeUnused>(F, s.rc, dst.P);
   const F3 dst_cv = neg(rc.wo);
   const F3 src_cv = normalize(sub(rc.P, src.P));
   const F3 sdisp = sub(rc.P, dst.P);
@@ -1067,7 +1072,7 @@ CT_D F3 shifted_integrand(const DFrame &F, float &dst_jac, const Isect &dst, con
     if (!(tp.x > 0.0f || tp.y > 0.0f || tp.z > 0.0f)) return f3(0, 0, 0);
   }
   float rj = 0.0f;
-  const F3 r = shift_reconnection<kWalk, kVis>(F, rj, retraced ? rc.prev : dst, src, s, eval_vis, tr, hyb, retraced);
+  const F3 r = shift_reconnection<kWalk, kVis, true>(F, rj, retraced ? rc.prev : dst, src, s, eval_vis, tr, hyb, retraced);
   dst_jac = rj;  // the hybrid shift's 1.0f * rj
   return hyb ? mulv(tp, r) : r;
 }
