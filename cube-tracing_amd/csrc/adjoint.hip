@@ -147,9 +147,9 @@ CT_D bool segment(const AArgs &A, const Path &P, uint32_t *stk, uint32_t &g, F3 
 
 // Traces every path of the wave's A.per_lane * 64 pixels.  A lane that has
 // ended its path starts the next sample of its pixel, or takes the next pixel
-// of the wave, at once: paths of a wave have 1 to max_depth + 1 segments of 1
-// to 20 steps, and a wave that waits for its longest runs at 31% of its lanes
-// (with this 44%).  The samples of a pixel stay in order on one lane, so the
+// of the wave, at once: paths of a wave have 1 to max_depth + 1 segments, each
+// of a few steps or many, and a wave that waits for its longest runs at 31% of
+// its lanes (with this 44%).  The samples of a pixel stay in order on one lane, so the
 // image is the same whatever the schedule.  hit(path, g, pos, nrm) shades a
 // vertex and returns whether the path goes on from path.o along path.d;
 // end(path) takes a finished sample (path.s, from 1 up to spp).

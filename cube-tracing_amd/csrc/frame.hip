@@ -284,8 +284,8 @@ struct Vis {
 };
 // Where the ray of pixel px and slot k is kept: slot by slot, so that a wave
 // writes whole lines (16 slots beside each other per pixel were 64 lines a
-// store, and as many a load: 8 frames at 1080p 21020 -> 20920 us, 4 palette
-// frames 14970 -> 14560).
+// store, and as many a load, which the L2 mostly absorbed: 4 palette frames
+// 14970 -> 14560 us, 8 frames at 1080p 21020 -> 20920, which is within noise).
 CT_D size_t ray_at(const DFrame &F, uint32_t px, uint32_t k) { return (size_t)k * F.npix + px; }
 CT_D bool occluded(const DFrame &F, Vis &v, F3 o, F3 d, float dist, uint32_t ti, uint32_t tp) {
   ++v.queries;
