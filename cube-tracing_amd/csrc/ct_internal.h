@@ -380,7 +380,7 @@ struct Ctx {
   DevBuf frame_dev, blk_dev;    // the frame record and its block tables on the device
   uint32_t blk_key[4] = {0, 0, 0, 0};
   uint32_t blk_counts[3] = {0, 0, 0};
-  Reach reach;                  // the scenes this context has rendered since its reset
+  Reach reach;                  // scenes rendered since the reset (a pixel that misses keeps its old record)
   const void *lights_accel = nullptr;  // accel and build whose cube lights were uploaded
   uint32_t lights_generation = 0;
   // A frame can run as kSplitParts interleaved parts of the image on as
