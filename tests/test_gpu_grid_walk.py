@@ -273,3 +273,64 @@ def test_grid_finds_room_again_through_other_instances(gpu):
     acc.delete_blas(1)
     acc.update_scene()
     _same(acc, sc, 6, n=30000)
+
+
+def test_grid_is_rebuilt_when_its_ids_run_out(gpu):
+    """Instances that leave and come back take new ranges of ids each time,
+    more in all than an update's reserve holds."""
+    sc, acc = _load(40, 20, 0.5)
+    assert len(acc.read_instances()) == 8
+    for k in range(14):
+        inst = k % 8
+        r = acc.read_instances()[inst]
+        W = acc.read_world()
+        f, n = r.first_primitive_index, r.primitive_count
+        boxes, prims = W["aabbs"][f:f + n].copy(), W["prims"][f:f + n].copy()
+        acc.delete_blas(inst)
+        acc.update_scene()
+        _add_instance(acc, boxes, prims)
+        acc.update_scene()
+        print("in and out", k, flush=True)
+        _same(acc, sc, 200 + k, n=12000)
+
+
+def test_update_with_more_instances_than_the_grid_was_built_for(gpu):
+    """One instance of 7000 slots gives way to 100 small ones in one update,
+    in the same slots: nothing else of the scene is new."""
+    d = ctamd.SceneDesc()
+    d.grid[:] = [24, 24, 48]
+    d.chunk[:] = [24] * 3
+    d.occupied_count = 14000
+    d.le_min = d.le_max = 1.0
+    d.albedo_min, d.albedo_max = 0.2, 0.8
+    d.seed = 9
+    d.voxel_extent = ctamd.CT_VOXEL_EXTENT
+    sc = ctamd.Scene(d)
+    acc = ctamd.Accel(max_instances=200, max_primitives=sc.info.primitive_count + 20000, max_cube_lights=8)
+    adj._load_geometry(sc, acc)
+    _same(acc, sc, 1, n=20000)
+    r = acc.read_instances()[0]
+    W = acc.read_world()
+    f = r.first_primitive_index
+    assert r.primitive_count > 32 * 100
+    boxes, prims = W["aabbs"][f:f + 3200].copy(), W["prims"][f:f + 3200].copy()
+    acc.delete_blas(0)
+    st = acc.staging()
+    C.memmove(st.aabbs, boxes.ctypes.data, boxes.nbytes)
+    C.memmove(st.primitives, prims.ctypes.data, prims.nbytes)
+    t = ctamd.Task()
+    t.type = ctamd.CT_TASK_BUILD_BLAS_FROM_CPU
+    t.u.blas_build_from_cpu.instance_count = 100
+    t.u.blas_build_from_cpu.primitive_count = 3200
+    for k in range(16):
+        t.u.blas_build_from_cpu.transform[k] = 1.0 if k % 5 == 0 else 0.0
+    for k in range(100):
+        st.instances[k].first_primitive_index = 32 * k
+        st.instances[k].primitive_count = 32
+    acc.task_queue_add(t)
+    acc.update_scene()
+    assert sum(i.primitive_count > 0 for i in acc.read_instances()) == 101
+    _same(acc, sc, 2, n=20000)
+    acc.delete_primitive(50, 3)
+    acc.update_scene()
+    _same(acc, sc, 3, n=20000)
