@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import ctamd
+import oracle as O
 from ctamd import adjoint as adj
 
 pytestmark = pytest.mark.gpu
@@ -142,16 +143,27 @@ def test_far_rays_take_the_bvh(gpu):
         assert np.array_equal(occ, bocc)
 
 
-@pytest.mark.parametrize("far", [12.0, 2e4])
+@pytest.mark.parametrize("far", [12.0, 2e4, 1e5])
 def test_frames_of_far_cameras(gpu, far):
     """Frames from a camera far outside the scene: the bits of frames that walk
     the BVH (instrumented ones)."""
     w = ctamd.hd_di(width=640, height=360, grid=32, chunk=16)
     scenes = [ctamd.Scene(ctamd.scene_desc(w)) for _ in range(2)]
     lo, hi = scenes[0].grid_min.astype(np.float64), scenes[0].grid_max.astype(np.float64)
-    eye = (lo + hi) / 2 + far * np.array([0.48, 0.6, 0.64])
-    w.camera = lambda f: (tuple(eye.tolist()), (-0.48, -0.6, -0.64), (0.0, 1.0, 0.0))
+    back = np.array([0.48, 0.6, 0.64])
+    eye = (lo + hi) / 2 + far * back
+    # the library's camera loses the direction in the position's rounding
+    right = np.cross([0.0, 1.0, 0.0], back)
+    right /= np.linalg.norm(right)
+    view = np.zeros((4, 4))
+    view[:3, 0], view[:3, 1], view[:3, 2], view[:3, 3], view[3, 3] = right, np.cross(back, right), back, eye, 1.0
     w.fov_radians = 1.2 * float((hi - lo).max()) / far
+
+    def params(f):
+        p = ctamd.frame_params(w, f)
+        p.inv_view[:] = np.float32(view.T.reshape(16)).tolist()
+        return p
+
     images = []
     for k in range(2):
         sc = scenes[k]
@@ -162,8 +174,10 @@ def test_frames_of_far_cameras(gpu, far):
         ctamd.load_scene(sc, acc, ctx)
         ctx.set_instrumentation(2 if k else 0)
         for f in range(2):
-            ctx.render(acc, ctamd.frame_params(w, f))
+            ctx.render(acc, params(f))
         images.append((ctx.read(ctamd.CT_BUF_IMAGE, w.width, w.height), bytes(ctx.read(ctamd.CT_BUF_DI, w.width, w.height))))
+    hits = (np.frombuffer(images[1][1], np.float32).reshape(-1, 15)[:, 3] > 0).mean()
+    assert 0.1 < hits < 1.0, hits
     assert np.array_equal(images[0][0].view(np.uint32), images[1][0].view(np.uint32))
     assert images[0][1] == images[1][1]
 
@@ -334,3 +348,29 @@ def test_update_with_more_instances_than_the_grid_was_built_for(gpu):
     acc.delete_primitive(50, 3)
     acc.update_scene()
     _same(acc, sc, 3, n=20000)
+
+
+def test_path_tracing_from_far_away_matches_oracle(gpu):
+    """A far view beside a near one: path tracing asks about every view."""
+    w = ctamd.hd_di(width=16, height=16, grid=32, chunk=16)
+    sc = ctamd.Scene(ctamd.scene_desc(w))
+    acc = ctamd.Accel(max_instances=sc.info.instance_count + 8,
+                      max_primitives=sc.info.primitive_count + 32 * sc.info.instance_count + 1024,
+                      max_cube_lights=sc.info.cube_light_count + 8)
+    ctx = ctamd.Ctx(16, 16)
+    ctamd.load_scene(sc, acc, ctx)
+    back = np.array([0.48, 0.6, 0.64])
+    right = np.cross([0.0, 1.0, 0.0], back)
+    right /= np.linalg.norm(right)
+    far = 2e4
+    views = adj.orbit_views(2, 160, 120, (0, 0, 0), 1.6, 0.4, fov_radians=1.2 / far)
+    near = adj.orbit_views(1, 160, 120, (0, 0, 0), 1.6, 0.4)[0]
+    views[0] = near
+    m = np.zeros((4, 4))
+    m[:3, 0], m[:3, 1], m[:3, 2], m[:3, 3], m[3, 3] = right, np.cross(back, right), back, far * back, 1.0
+    views[1].inv_view[:] = np.float32(m.T.reshape(16)).tolist()
+    img = adj.path_trace(acc, views, list(sc.materials), spp=2, max_depth=2, seed=5).cpu().numpy()
+    osc = O.OScene.from_scene(sc)
+    ref = osc.path_trace(ctamd.AdjointDesc(2, 2, 2, 5), views, list(sc.materials))
+    assert np.array_equal(img.view(np.uint32), ref.view(np.uint32))
+    assert (img[:19200] != 0).any() and (img[19200:] != 0).any()
